@@ -265,7 +265,7 @@ int launch_gemv_argmax(kh_ctx *ctx, int precision, const GemvJob &job, float *ar
 constexpr int MULTI_TOKENS = 8;  // token slots of one VALU multi-token launch
 // Whether m token rows against a rows x cols weight take the multi-token
 // GEMV (else the GEMM): kh_matmul, and the session's single projections.
-bool matmul_takes_multi(size_t m, size_t rows, size_t cols);
+bool matmul_takes_multi(int precision, size_t m, size_t rows, size_t cols);
 int launch_gemv_multi(kh_ctx *ctx, const kh_weight *w, const QAct &x, size_t m, const float *bias, float *y);
 // The same for up to MULTI_JOBS weights of one precision and width over the
 // same rows of codes, in one launch: y[i] (+)= x W_i^T (+ bias[i]), adding
@@ -285,12 +285,15 @@ inline unsigned multi_firsts(int njobs, int g1, int g2) {
 // Whether the multi-token GEMV should stage m f32 rows of `cols` itself
 // (quantising them in every workgroup) rather than read codes quantised once
 // by a launch of their own: only while the stage is small.
-bool multi_stages_f32(int precision, size_t m, size_t cols);
-// Token rows from which the multi-token GEMV runs on the matrix cores
-// (launch_gemv_mma) when it is given codes.
-size_t mma_min_tokens();
+bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols);
+// Whether the multi-token GEMV over `rows` weight rows in all runs on the
+// matrix cores (launch_gemv_mma) when it is given codes.
+bool mma_takes(size_t m, size_t rows, size_t cols);
+// Whether the matrix-core multi-token GEMV addresses a weight (32-bit buffer
+// offsets for its rows, its scales and 32 tokens' outputs).
+bool mma_addresses(int prec, size_t rows, size_t cols);
 // The multi-token GEMV on the matrix cores (gemv_mma.hip): the same
-// contract as launch_gemv_multi_jobs over codes, 16 token rows a launch.
+// contract as launch_gemv_multi_jobs over codes, any number of token rows.
 int launch_gemv_mma(kh_ctx *ctx, int njobs, const kh_weight *const *w, const float *const *bias, float *const *y,
                     const int *accumulate, const QAct &x, size_t m);
 int launch_gemv_multi_jobs(kh_ctx *ctx, int njobs, const kh_weight *const *w, const float *const *bias,
@@ -345,6 +348,12 @@ int launch_gemm_q(kh_ctx *ctx, int precision, const GemmArgs &a, int max_tiles, 
 // Allocates the split-K workspace now (a GEMM captured into a graph splits
 // only when it was allocated before the capture).
 int gemm_split_reserve(kh_ctx *ctx);
+// The split-K workspace for `bytes` of partials, or null where it does not
+// hold them (or was not allocated before a capture).
+float *split_partials(kh_ctx *ctx, size_t bytes);
+// y[M][N] (+)= the ks planes of part added in order (+ bias).
+int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, const float *bias, int accumulate,
+                        float *y);
 // Sets a's split-K fields for an ungrouped launch of tile_m-token tiles when
 // splitting its k-stages pays (ksplit 0: no split).
 int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n = 128);

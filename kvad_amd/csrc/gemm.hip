@@ -816,6 +816,23 @@ int gemm_split_reserve(kh_ctx *ctx) {
     return KH_OK;
 }
 
+float *split_partials(kh_ctx *ctx, size_t bytes) {
+    if (bytes > SPLIT_BYTES) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) return nullptr;
+    if (cap == hipStreamCaptureStatusNone && gemm_split_reserve(ctx) != KH_OK) return nullptr;  // no allocation under capture
+    return static_cast<float *>(ctx->gemm.ptr);
+}
+
+int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, const float *bias, int accumulate,
+                        float *y) {
+    const size_t quads = ((size_t)M * N + 3) / 4;
+    hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, ctx->stream, part, ks,
+                       M, N, bias, accumulate, y);
+    KH_HIP(hipGetLastError());
+    return KH_OK;
+}
+
 int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
     a.ksplit = 0;
     if (a.tiles) return KH_OK;  // grouped launches are not split
@@ -878,8 +895,8 @@ int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, co
     }
     // up to eight rows: the multi-token GEMV quantises them as it stages them
     // (QActBatch::new's codes, one launch fewer) while they are few values
-    const bool multi = matmul_takes_multi(m, rows, cols) && !matmul_force_gemm();
-    if (multi && multi_stages_f32(w->precision, m, cols))
+    const bool multi = matmul_takes_multi(w->precision, m, rows, cols) && !matmul_force_gemm();
+    if (multi && multi_stages_f32(w->precision, m, rows, cols))
         return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, &accumulate, QAct{}, m, xs);
     // QActBatch::new (quant.rs:693-714): the activation rows quantised per block
     const size_t qb = (m * cols + 255) / 256 * 256, sb = (4 * m * cols / BLOCK + 255) / 256 * 256;
@@ -899,7 +916,7 @@ int launch_matmul_q(kh_ctx *ctx, const kh_weight *w, const QAct &q, size_t m, co
         rows > 0x7fffffff || m > 0x7fffffff)
         return fail(KH_DECLINED, "matmul: operands of 4 GiB or more are not addressed here");
     // a few tokens: stream the weights once through the multi-token GEMV
-    if (matmul_takes_multi(m, rows, cols) && !matmul_force_gemm())
+    if (matmul_takes_multi(w->precision, m, rows, cols) && !matmul_force_gemm())
         return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, &accumulate, q, m);
     GemmArgs a{};
     a.w = w->qs;

@@ -1225,11 +1225,13 @@ int launch_gemv_argmax(kh_ctx *ctx, int precision, const GemvJob &job, float *ar
 int launch_gemv_multi_jobs(kh_ctx *ctx, int njobs, const kh_weight *const *w, const float *const *bias,
                            float *const *y, const int *accumulate, const QAct &x, size_t m, const float *xf) {
     if (m == 0) return KH_OK;
-    // the matrix cores from mma_min_tokens() rows, and from two over a tall
-    // matrix (a vocabulary head, 151936x896 at 2 rows: 32.3 against 35.9 us)
     size_t rows_total = 0;
-    for (int i = 0; i < njobs && i < MULTI_JOBS; i++) rows_total += w[i]->rows;
-    if (!xf && w[0]->precision != KH_F32 && (m >= mma_min_tokens() || (m >= 2 && rows_total >= 65536)))
+    bool fits = true;
+    for (int i = 0; i < njobs && i < MULTI_JOBS; i++) {
+        rows_total += w[i]->rows;
+        fits = fits && mma_addresses(w[i]->precision, w[i]->rows, w[i]->cols);
+    }
+    if (!xf && fits && w[0]->precision != KH_F32 && mma_takes(m, rows_total, w[0]->cols))
         return launch_gemv_mma(ctx, njobs, w, bias, y, accumulate, x, m);
     if (njobs < 1 || njobs > MULTI_JOBS) return fail(KH_EINVAL, "matmul: one to three weights per launch");
     MultiArgs a{};
@@ -1264,30 +1266,50 @@ int launch_gemv_multi(kh_ctx *ctx, const kh_weight *w, const QAct &x, size_t m, 
     return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, nullptr, x, m);
 }
 
-bool multi_stages_f32(int precision, size_t m, size_t cols) {
+bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols) {
     // Every workgroup quantises its token slots' rows (2, 4 or 8 slots); past
     // about 12K values that costs more than a quantising launch of its own
     // plus a stage of codes (measured over q8 and Q4_K weights of 896 to
-    // 14336 columns at m = 2..8).
-    // From mma_min_tokens() rows the matrix-core kernel takes the rows' codes.
-    if (m >= mma_min_tokens()) return false;
+    // 14336 columns at m = 2..8).  The matrix-core kernel takes the rows' codes.
+    if (mma_takes(m, rows, cols) && mma_addresses(precision, rows, cols)) return false;
     const size_t slots = m <= 2 ? 2 : m <= 4 ? 4 : 8;
     const int lim = env_int("KVAD_MULTI_STAGE_F32", 12288);  // tuning knob
-    (void)precision;
     return slots * cols <= (size_t)lim;
 }
 
-size_t mma_min_tokens() { return (size_t)env_int("KVAD_MMA_MIN", 5); }  // tuning knob
+bool mma_takes(size_t m, size_t rows, size_t cols) {
+    if (m >= 2 && rows >= 65536) return true;
+    const int forced = env_int("KVAD_MMA_MIN", 0);  // tuning knob: from this many rows
+    if (forced > 0) return m >= (size_t)forced;
+    // The VALU kernel's time grows with its token slots (2, 4, 8), the
+    // matrix-core kernel's hardly at all.  Measured with the rows'
+    // quantisation (us, VALU / matrix cores): at two rows the VALU everywhere
+    // but a vocabulary head (Q4_K 4096x4096 7.2 / 7.8; q8 151936x896 42.0 /
+    // 32.6); at three and four, large matrices change over (Q4_K 14336x4096
+    // 14.9 / 13.4, 4096x14336 17.5 / 14.8, 4096x4096 8.6 / 7.7, q4 11008x4096
+    // 13.2 / 10.9, q8 8960x1536 9.2 / 8.4) and small or flat ones do not (q8
+    // 4864x896 5.5 / 5.7, 896x4864 8.3 / 9.5, 1536x8960 10.6 / 12.5).
+    return m >= 5 || (m >= 3 && rows >= 4096 && rows * cols >= (size_t)12 << 20);
+}
 
-bool matmul_takes_multi(size_t m, size_t rows, size_t cols) {
+bool matmul_takes_multi(int precision, size_t m, size_t rows, size_t cols) {
     const int forced = env_int("KVAD_MULTI_TOKENS", 0);  // tuning knob: the multi-token GEMV up to this many rows
     if (forced > 0) return m <= (size_t)forced;
-    // Past eight rows the matrix-core kernel (16 rows a launch) beats the
-    // GEMM only over narrow rows of a not-too-tall matrix; the GEMM's time is
-    // nearly flat in m.  Measured (us): 4864x896 at 16 rows 10.1 against
-    // 12.4; 896x896 7.9 / 12.1; 896x4864 18.1 / 12.0; 151936x896 (a
-    // vocabulary head) 95.9 / 72.7, at 8 rows 49.7 / 72.0.
-    return m <= (size_t)MULTI_TOKENS || (m <= 16 && cols <= 2048 && rows <= 16384);
+    if (!mma_addresses(precision, rows, cols)) return m <= (size_t)MULTI_TOKENS;
+    // Up to 16 rows the matrix-core kernel is ahead of the GEMM everywhere
+    // (with the rows' quantisation, us, GEMM / it: Q4_K 14336x4096 24.8 /
+    // 14.1, 4096x14336 25.0 / 16.3, 4096x4096 14.1 / 8.1; q8 896x4864 10.7 /
+    // 9.8, 1536x8960 14.2 / 13.0, 151936x896 37.4 / 35.7).  Past that it
+    // streams the weights once per 32 rows while a wave's registers hold its
+    // slice of 32 rows' codes, and splits wider rows over the grid: ahead to
+    // 64 rows up to 4096 columns (Q4_K 14336x4096 43.5 / 30.8, 1024x4096 13.0
+    // / 10.1; q8 14336x4096 34.8 / 31.9, 4864x896 13.5 / 8.7, 8960x1536 18.8 /
+    // 14.7; at 96 rows 4096x4096 25.0 / 24.1, at 128 26.3 / 30.9) and of Q4_K
+    // at any width (4096x14336 38.1 / 37.3), behind over wider q8 and q4 rows
+    // (1536x8960 at 32 rows 15.2 / 15.3, at 64 16.5 / 21.1) and over a
+    // vocabulary head, which the GEMM's tiles fill (38.7 / 40.4 at 32).
+    if (m <= 16) return true;
+    return m <= 64 && rows < 65536 && (precision == KH_Q4K || cols <= 4096);
 }
 
 bool gemv_pairs_fit(int precision, size_t cols) {

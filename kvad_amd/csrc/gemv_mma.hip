@@ -1,37 +1,55 @@
-// Multi-token GEMV on the matrix cores: y[t][r] (+)= sum_b ws[r,b] xs[t,b]
-// D_b[r,t] for up to 16 token rows at once (Weight::matmul_bt at a few
-// tokens, crates/llm/src/quant.rs:751-907, as forward_each calls it,
+// Few-row matmul on the matrix cores: y[t][r] (+)= sum_b ws[r,b] xs[t,b]
+// D_b[r,t] for a few to a few dozen token rows (Weight::matmul_bt,
+// crates/llm/src/quant.rs:751-907, as forward_each calls it,
 // llama.rs:418-434), q8 / q4 / Q4_K weights against the rows' int8 codes.
 //
 // D_b, the exact i32 dot of weight row r's 32-block b with token t's codes,
-// comes from the matrix core, 16 weight rows a wave:
-//   - up to 8 tokens: one v_mfma_i32_16x16x64_i8 per pair of blocks.  The
-//     64-wide k of the instruction spans blocks 2p and 2p+1; output columns
-//     0-7 are the tokens against block 2p (their codes zero in block 2p+1's
-//     k-range) and columns 8-15 the tokens against block 2p+1, so every
-//     output lane holds a block dot some token needs;
-//   - 9 to 16 tokens: one v_mfma_i32_16x16x32_i8 per block, a column per
-//     token.
-// The block's scaling follows in registers (convert, scale product, fused
-// multiply-add per output).  Q4_K's minimum terms sum_j dmin m_j[r] xs[t,j]
-// sum_j[t] are a true product over the sub-block index and go through
-// v_mfma_f32_16x16x4_f32, four sub-blocks an instruction.
+// is one v_mfma_i32_16x16x32_i8 for 16 weight rows x 16 tokens.  The block's
+// scale products ws[r] xs[t] are an outer product, four blocks per
+// v_mfma_f32_16x16x1_4b_f32 (block k from lanes 16k..16k+15 of both
+// operands, its products in elements 4k..4k+3), so two VALU operations per
+// output and block remain: convert the dot, fused multiply-add.  Q4_K's
+// minimum terms sum_j dmin m_j[r] xs[t,j] sum_j[t] are a true product over
+// the sub-block index: v_mfma_f32_16x16x4_f32, four sub-blocks an
+// instruction, straight into the accumulators.
 //
-// Work.  A workgroup owns 16 weight rows of one job; its NW waves split the
-// row's k-range into contiguous unit ranges (a unit: four 32-blocks of q8 /
-// q4, one 256-wide Q4_K super-block).  Lanes load the weights and codes they
-// feed the matrix core straight from memory (the codes are a few hundred KB
-// at most and stay in the caches); a wave issues the loads of R units before
-// it computes any, and every load is unconditional (a lane with nothing to
-// read addresses past its buffer's end, which reads zeros), so each wait
-// covers only the loads it needs.  Scales and block parameters, loaded one
-// per lane, reach the accumulator layout (rows 4 (lane >> 4) .. + 4 of the
-// lane's column) through a wave-private LDS exchange.  The waves' partial
-// tiles are summed in wave order in LDS, so results do not depend on timing;
-// bias and the residual add are applied once.
+// What bounds it: the weights' stream, and at its ends the latency of the
+// first loads.  A wave owns a fixed slice of the k-range, holds its slice of
+// the codes and block scales of all 16 T tokens in registers in the matrix
+// core's operand layout (the codes are read once per workgroup, not once per
+// 16 weight rows), and walks the 16-row groups of its workgroup with D units
+// of weights in flight in registers (a unit: 128 k-values of q8 / q4, a
+// 256-wide Q4_K super-block).  KW waves share a group's k-range.
+//
+// Weights and codes come in with consecutive lanes on consecutive 16-byte
+// pieces of a row and turn into the operand layout (a row per lane & 15)
+// through a wave-private LDS stage.  Loads in the operand layout itself put
+// every lane on a line of its own, which took the address units 43 cycles an
+// instruction (s_memtime stamps), against 16.
+//
+// The waves' partial tiles meet in LDS in wave order (results do not depend on
+// timing), double buffered, one barrier that waits on LDS only per group; the
+// adds and the store fall to another wave each group.  Every load is
+// unconditional (a lane with nothing to read addresses past its buffer's end,
+// which reads zeros), so each wait covers only the loads it needs; bias and
+// residual values are loaded ahead by the wave that will store the group.
+//
+// Measured (us per matmul under graph replay, the rows' quantisation launch of
+// about 3 us included; against a kernel that loaded in the operand layout up
+// to 8 tokens and the int8 GEMM above): Q4_K 14336x4096 at 5 / 12 / 32 / 64
+// tokens 19.7 / 24.2 / 26.9 / 43.5 -> 13.8 / 14.0 / 19.5 / 30.8, 4096x14336
+// 18.6 / 24.5 / 25.9 / 38.0 -> 15.2 / 15.2 / 22.4 / 37.3, 4096x4096 9.2 / 13.7
+// / 16.2 / 19.5 -> 7.7 / 7.9 / 10.4 / 17.3; q8 4864x896 at 5 / 16 / 64 6.4 /
+// 8.7 / 13.5 -> 5.8 / 5.9 / 8.7; q4 4096x4096 at 8 / 16 9.4 / 13.6 -> 7.7 /
+// 7.8.  Eight waves of up to 256 registers a workgroup and one workgroup a CU
+// beat sixteen of 128 (Q4_K 4096x4096 at 12 tokens 8.2 / 12.0, the registers
+// spilling) and two workgroups a CU where a slice is more than a unit
+// (14336x4096 13.9 / 16.8).
 //
 // Sums run in another order than the single-token GEMV's, so a token's row
 // agrees with its matvec to rounding (1e-5 relative), not to the bit.
+#include <algorithm>
+
 #include "gemv_core.hpp"
 
 namespace kh {
@@ -39,9 +57,11 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned long long u64;
 
-constexpr unsigned XOOB = 0x80000000u;  // a base past every codes / scales buffer (< 2 GiB)
-constexpr int MMA_TOKENS = 16, PAIR_TOKENS = 8;
+constexpr unsigned OOB = 0xfff00000u;  // past every buffer here, immediate offsets included
+constexpr int GROUP = 16;              // weight rows of a group, tokens of a tile
 
 struct MmaJob {
     const void *w;
@@ -49,357 +69,458 @@ struct MmaJob {
     const float *bias;   // [rows] or null
     float *y;            // [m][rows]
     int rows, accumulate;
-    int g0;              // the job's first workgroup (16 rows each)
+    int wg0, nwg;        // the job's workgroups
 };
 
 struct MmaArgs {
-    const int8_t *xq;     // [m][cols] codes
-    const float *xs;      // [m][nb] block scales
-    const int32_t *xsum;  // [m][nb] block code sums (Q4_K's minimum term)
-    int cols, m, njobs;
-    int units;            // per row: four-block quads (q8, q4) or super-blocks (Q4_K)
     MmaJob j[MULTI_JOBS];
+    // split z of the units (grid z, `per` units each) stores its sums to
+    // part[z][all][rows] for a reduce launch, one job only; null: no split
+    float *part;
+    int per, all;
 };
 
-// Orders this wave's LDS writes before its next reads (LDS serves a wave's
-// requests in order; the clobber keeps the compiler from moving them).
-__device__ __forceinline__ void wave_lds_sync() { __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// What a launch runs on.
+struct MmaRows {
+    QAct x;  // the rows' codes, block scales and code sums (Q4_K's minimum term)
+    int cols, m, njobs;
+    int units;  // per row
+};
 
-__device__ __forceinline__ unsigned long long bld8(const rsrc_t &r, unsigned off) {
-    return __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+// Keeps the compiler from moving this wave's LDS accesses across (LDS serves
+// a wave's requests in order).
+__device__ __forceinline__ void wave_order() { __asm__ volatile("" ::: "memory"); }
+
+__device__ __forceinline__ u64 bld8(const rsrc_t &r, unsigned off) {
+    return __builtin_bit_cast(u64, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+
+// A buffer descriptor over fewer than 2^32 bytes.
+__device__ __forceinline__ rsrc_t rsrc32(const void *p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, RSRC_WORD3);
 }
 
 // Four nibble codes per byte lane -> signed (code - 8) bytes, no borrows.
 __device__ __forceinline__ unsigned nib_minus8(unsigned x) {
     return ((x | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
 }
+__device__ __forceinline__ u64 pack64(unsigned lo, unsigned hi) { return (u64)lo | ((u64)hi << 32); }
 
-__device__ __forceinline__ v4i mma32(unsigned long long a, unsigned long long b) {
+__device__ __forceinline__ v4i mma32(u64 a, u64 b) {
     const v4i z = {0, 0, 0, 0};
     return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)a, (long)b, z, 0, 0, 0);
 }
-__device__ __forceinline__ v4i mma64(const int4 &a, const int4 &b) {
-    const v4i z = {0, 0, 0, 0};
-    const v4i va = {a.x, a.y, a.z, a.w}, vb = {b.x, b.y, b.z, b.w};
-    return __builtin_amdgcn_mfma_i32_16x16x64_i8(va, vb, z, 0, 0, 0);
-}
 
-// acc[i] += D[i] * (w[i] * x)
-__device__ __forceinline__ void scale_add(v4f &acc, const v4i &D, const float4 &w, float x) {
-    acc[0] = fmaf((float)D[0], w.x * x, acc[0]);
-    acc[1] = fmaf((float)D[1], w.y * x, acc[1]);
-    acc[2] = fmaf((float)D[2], w.z * x, acc[2]);
-    acc[3] = fmaf((float)D[3], w.w * x, acc[3]);
-}
-
-// A lane's fixed addressing: lr = lane & 15, lg = lane >> 4.  Rows past the
-// job's end and tokens past m address past their buffers' ends.
-struct Lane {
-    int lr, lg;
-    unsigned wrow;   // weight row lr's first byte
-    unsigned wsrow;  // its block scales (q8 / q4), bytes
-    unsigned xrow;   // 16-token mode: token lr's codes; paired mode: the codes this lane feeds
-    unsigned xsrow;  // token scales / sums of the lane's token, bytes
-    unsigned xsrow2; // paired q8 / q4: token lr & 7's scales, bytes
+template <int PREC>
+struct Shape {
+    static constexpr int UK = PREC == KH_Q4K ? QK_K : 4 * BLOCK;  // k-values of a unit
+    static constexpr int NB = UK / BLOCK, NQ = NB / 4;            // blocks, quads of blocks
 };
 
-// ---- one unit's registers, per lane --------------------------------------
-template <int PREC, bool PAIR>
-struct Unit;
-template <>
-struct Unit<KH_Q8, false> {
-    unsigned long long a[4], b[4];
-    float ws, xs;
-};
-template <>
-struct Unit<KH_Q4, false> {
-    unsigned a[4];
-    unsigned long long b[4];
-    float ws, xs;
-};
-template <>
-struct Unit<KH_Q8, true> {  // the quad's two block pairs
-    int4 a[2], b[2];
-    float ws, xs;
-};
-template <>
-struct Unit<KH_Q4, true> {
-    int4 a[2], b[2];
-    float ws, xs;
-};
-template <bool PAIR>
-struct Unit<KH_Q4K, PAIR> {
-    int4 h;
-    typename std::conditional<PAIR, int4, unsigned long long>::type a[4];
-    typename std::conditional<PAIR, int4, unsigned long long>::type b[PAIR ? 4 : 8];
-    float xs[2];
-    int sum[2];
+// A stage row is a unit's codes of a weight row and 16 bytes of its scales:
+// Q4_K's block as it lies (header, then codes), q8 / q4 codes, then four block
+// scales.  Rows 36 (q4 20) banks apart serve the operand reads without
+// conflicts.
+template <int PREC>
+struct RowStage {
+    static constexpr int CB = PREC == KH_Q4 ? 64 : 128;  // bytes of codes
+    static constexpr int STR = CB + 16;
+    static constexpr int CODES = PREC == KH_Q4K ? 16 : 0, SCALES = PREC == KH_Q4K ? 0 : CB;
+    static constexpr int RUN = PREC == KH_Q4K ? 9 : CB / 16;               // 16-byte pieces of a row in one run
+    static constexpr int NL = (GROUP * RUN + WAVE - 1) / WAVE;             // loads a wave
 };
 
-template <int PREC, bool PAIR>
-__device__ __forceinline__ void load_unit(Unit<PREC, PAIR> &u, int q, unsigned um, const Lane &L, const rsrc_t &W,
-                                          const rsrc_t &WS, const rsrc_t &X, const rsrc_t &XS, const rsrc_t &XM,
-                                          int nb) {
-    // um: 0, or all ones for a unit past the wave's share (every load reads zeros)
-    if constexpr (PREC == KH_Q4K) {
-        const unsigned base = L.wrow + (unsigned)q * Q4K_BYTES;
-        u.h = bld16(W, base | um);
-        if constexpr (PAIR) {
-            // pair c: qs bytes 32c + 16 (lg & 1) .. + 16 (sub-block 2c low, 2c+1 high nibbles)
-#pragma unroll
-            for (int c = 0; c < 4; c++) u.a[c] = bld16(W, (base + 16 + 32 * c + 16 * (L.lg & 1)) | um);
-#pragma unroll
-            for (int c = 0; c < 4; c++) u.b[c] = bld16(X, (L.xrow + (unsigned)q * QK_K + 64 * c) | um);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 4; c++) u.a[c] = bld8(W, (base + 16 + 32 * c + 8 * L.lg) | um);
-#pragma unroll
-            for (int j = 0; j < 8; j++) u.b[j] = bld8(X, (L.xrow + (unsigned)q * QK_K + 32 * j + 8 * L.lg) | um);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const unsigned o = (L.xsrow + (8 * q + 4 * h + L.lg) * 4) | um;
-            u.xs[h] = bldf(XS, o);
-            u.sum[h] = bldi(XM, o);
-        }
-    } else {
-        const int b0 = 4 * q;
-        if constexpr (PAIR) {
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const unsigned pb = (unsigned)(2 * q + p);
-                u.a[p] = bld16(W, (PREC == KH_Q8 ? L.wrow + 64 * pb + 16 * L.lg
-                                                 : L.wrow + 32 * pb + 16 * (L.lg >> 1)) | um);
-                u.b[p] = bld16(X, (L.xrow + 64 * pb) | um);
-            }
-            u.xs = bldf(XS, (L.xsrow2 + (b0 + L.lg) * 4) | um);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if constexpr (PREC == KH_Q8) {
-                    u.a[k] = bld8(W, (L.wrow + 32 * (b0 + k) + 8 * L.lg) | um);
-                    u.b[k] = bld8(X, (L.xrow + 32 * (b0 + k) + 8 * L.lg) | um);
-                } else {
-                    u.a[k] = (unsigned)bldi(W, (L.wrow + 16 * (b0 + k) + 4 * L.lg) | um);
-                    const unsigned tb = L.xrow + 32 * (b0 + k) + 4 * L.lg;
-                    const unsigned lo = (unsigned)bldi(X, tb | um), hi = (unsigned)bldi(X, (tb + 16) | um);
-                    u.b[k] = (unsigned long long)lo | ((unsigned long long)hi << 32);
-                }
-            }
-            u.xs = bldf(XS, (L.xsrow + (b0 + L.lg) * 4) | um);
-        }
-        // past the row's last block the loads read the next row's bytes: the
-        // scale is zeroed there, so those products add nothing
-        const float w = bldf(WS, (L.wsrow + (b0 + L.lg) * 4) | um);
-        u.ws = b0 + L.lg < nb ? w : 0.0f;
-    }
-}
+// One unit of 16 weight rows in flight: piece i * 64 + lane of their runs,
+// and for q8 / q4 row lane's four block scales (lanes 0-15).
+template <int PREC>
+struct Wts {
+    int4 a[RowStage<PREC>::NL];
+    int4 ws;
+};
 
-// ex: this wave's 256-float exchange area.  acc: the lane's column, rows
-// 4 lg .. + 4; accm: Q4_K's minimum terms (token lr's column).
-template <int PREC, bool PAIR>
-__device__ __forceinline__ void compute_unit(const Unit<PREC, PAIR> &u, v4f &acc, v4f &accm, float *ex,
-                                             const Lane &L) {
-    const int lr = L.lr, lg = L.lg;
-    if constexpr (PREC == KH_Q4K) {
-        // sub-blocks lg and lg + 4 of row lr: d * sc and dmin * m (mpp.rs:276-282, 304-315)
-        const float d = half_bits_to_float((unsigned)u.h.x), dmin = half_bits_to_float((unsigned)u.h.x >> 16);
-        float dl[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            unsigned sc, mn;
-            q4k_scale_min_bfe(u.h, q4k_lane(lg + 4 * h), sc, mn);
-            dl[h] = d * (float)sc;
-            const float ml = dmin * (float)mn;
-            // minimum terms of sub-blocks 4h .. 4h + 3: A[row][k] = ml of
-            // sub-block 4h + k, B[k][tok] = xs * sum of the token's sub-block
-            const float s = u.xs[h] * (float)u.sum[h];
-            accm = __builtin_amdgcn_mfma_f32_16x16x4f32(ml, s, accm, 0, 0, 0);
-        }
-        ex[lg * 16 + lr] = dl[0];
-        ex[(lg + 4) * 16 + lr] = dl[1];
-        if constexpr (PAIR) {
-            // [token][parity][pair]: sub-block j = 2c + p at 4p + c
-            if (lr < PAIR_TOKENS) {
-                ex[128 + lr * 8 + 4 * (lg & 1) + (lg >> 1)] = u.xs[0];
-                ex[128 + lr * 8 + 4 * (lg & 1) + 2 + (lg >> 1)] = u.xs[1];
-            }
-            wave_lds_sync();
-            const int t = lr & 7, p = lr >> 3;
-            const float4 x4 = *reinterpret_cast<const float4 *>(ex + 128 + t * 8 + 4 * p);
-            const float xk[4] = {x4.x, x4.y, x4.z, x4.w};
-            const int sh = 4 * (lg >> 1);  // lanes lg < 2 feed the low nibbles (sub-block 2c), others the high
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int4 q4 = u.a[c];
-                const int4 w = {(int)(((unsigned)q4.x >> sh) & 0x0f0f0f0fu), (int)(((unsigned)q4.y >> sh) & 0x0f0f0f0fu),
-                                (int)(((unsigned)q4.z >> sh) & 0x0f0f0f0fu), (int)(((unsigned)q4.w >> sh) & 0x0f0f0f0fu)};
-                const v4i D = mma64(w, u.b[c]);
-                const float4 dl4 = *reinterpret_cast<const float4 *>(ex + (2 * c + p) * 16 + 4 * lg);
-                scale_add(acc, D, dl4, xk[c]);
-            }
-        } else {
-            ex[128 + lr * 8 + lg] = u.xs[0];
-            ex[128 + lr * 8 + lg + 4] = u.xs[1];
-            wave_lds_sync();
-            const float4 x0 = *reinterpret_cast<const float4 *>(ex + 128 + lr * 8);
-            const float4 x1 = *reinterpret_cast<const float4 *>(ex + 128 + lr * 8 + 4);
-            const float xs8[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const unsigned long long q = u.a[j >> 1];
-                const unsigned lo = (unsigned)q, hi = (unsigned)(q >> 32);
-                const unsigned w0 = (j & 1) ? (lo >> 4) & 0x0f0f0f0fu : lo & 0x0f0f0f0fu;
-                const unsigned w1 = (j & 1) ? (hi >> 4) & 0x0f0f0f0fu : hi & 0x0f0f0f0fu;
-                const v4i D = mma32((unsigned long long)w0 | ((unsigned long long)w1 << 32), u.b[j]);
-                const float4 dl4 = *reinterpret_cast<const float4 *>(ex + j * 16 + 4 * lg);
-                scale_add(acc, D, dl4, xs8[j]);
-            }
-        }
-        wave_lds_sync();
-    } else {
-        ex[lg * 16 + lr] = u.ws;  // [block][row]
-        if constexpr (PAIR) {
-            // [token][parity][pair]: block 2 pp + p of the quad at 2p + pp
-            ex[64 + (lr & 7) * 4 + 2 * (lg & 1) + (lg >> 1)] = u.xs;
-            wave_lds_sync();
-            const int t = lr & 7, p = lr >> 3;
-            const float2 x2 = *reinterpret_cast<const float2 *>(ex + 64 + t * 4 + 2 * p);
-            const float xk[2] = {x2.x, x2.y};
-#pragma unroll
-            for (int pp = 0; pp < 2; pp++) {
-                int4 A = u.a[pp];
-                if constexpr (PREC == KH_Q4) {
-                    // block 2 pb + (lg >> 1), weights 16 (lg & 1) .. + 16: low nibbles of its
-                    // 16 bytes for the first half, high for the second (quant.rs:258-274)
-                    const int sh = 4 * (lg & 1);
-                    A = {(int)nib_minus8(((unsigned)A.x >> sh) & 0x0f0f0f0fu),
-                         (int)nib_minus8(((unsigned)A.y >> sh) & 0x0f0f0f0fu),
-                         (int)nib_minus8(((unsigned)A.z >> sh) & 0x0f0f0f0fu),
-                         (int)nib_minus8(((unsigned)A.w >> sh) & 0x0f0f0f0fu)};
-                }
-                const v4i D = mma64(A, u.b[pp]);
-                const float4 w4 = *reinterpret_cast<const float4 *>(ex + (2 * pp + p) * 16 + 4 * lg);
-                scale_add(acc, D, w4, xk[pp]);
-            }
-        } else {
-            ex[64 + lr * 4 + lg] = u.xs;  // [token][block]
-            wave_lds_sync();
-            const float4 x4 = *reinterpret_cast<const float4 *>(ex + 64 + lr * 4);
-            const float xk[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                unsigned long long A;
-                if constexpr (PREC == KH_Q8) {
-                    A = u.a[k];
-                } else {
-                    // byte i: weight i (low nibble), 16 + i (high)
-                    const unsigned lo = nib_minus8(u.a[k] & 0x0f0f0f0fu),
-                                   hi = nib_minus8((u.a[k] >> 4) & 0x0f0f0f0fu);
-                    A = (unsigned long long)lo | ((unsigned long long)hi << 32);
-                }
-                const v4i D = mma32(A, u.b[k]);
-                const float4 w4 = *reinterpret_cast<const float4 *>(ex + k * 16 + 4 * lg);
-                scale_add(acc, D, w4, xk[k]);
-            }
-        }
-        wave_lds_sync();
-    }
-}
+// A wave's slice of the tokens' codes and block scales, S units of T tiles of
+// 16 tokens (token lane & 15, k-slot lane >> 4; scales of block lane >> 4).
+template <int PREC, int S, int T>
+struct Acts {
+    u64 b[S][T][Shape<PREC>::NB];
+    float xs[S][T][Shape<PREC>::NQ];
+    float xm[PREC == KH_Q4K ? S : 1][T][Shape<PREC>::NQ];  // xs * code sum
+};
 
-template <int PREC, bool PAIR, int NW, int R>
-__global__ __launch_bounds__(WAVE * NW) void gemv_mma_kernel(unsigned g12, MmaArgs a) {
+// The first job's pointers and sizes lead the arguments (preloaded into
+// scalar registers); gm: its workgroups << 16 | tokens.
+template <int PREC, int KW, int S, int T, int D, int WPE, bool WIDE, bool SPLIT>
+__global__ __launch_bounds__(WAVE *KW, WPE) void rows_mma_kernel(unsigned g12, unsigned gm, const void *w0,
+                                                                 const float *ws0, const int8_t *xq, const float *xs,
+                                                                 int rows0, int cols, const int32_t *xsum, MmaArgs a) {
     static_assert(MULTI_JOBS == 3, "g12 holds jobs 1 and 2");
-    __shared__ __align__(16) float s_ex[NW][256];
-    __shared__ __align__(16) float s_red[NW][WAVE * 4];
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    constexpr int UK = Shape<PREC>::UK, NB = Shape<PREC>::NB, NQ = Shape<PREC>::NQ;
+    using RS = RowStage<PREC>;
+    constexpr int XSTR = UK + 16;  // a token's stage row
+    constexpr int STAGE = GROUP * (XSTR > 16 * S * NQ ? XSTR : 16 * S * NQ);
+    static_assert(XSTR >= RS::STR, "the stage holds a unit of weights too");
+    __shared__ __align__(16) v4f s_red[2][KW][T][WAVE];
+    __shared__ __align__(16) char s_stage[KW][STAGE];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), lr = lane & 15, lg = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ji = ((int)blockIdx.x >= (int)(g12 & 0xffffu) ? 1 : 0) + ((int)blockIdx.x >= (int)(g12 >> 16) ? 1 : 0);
     const MmaJob &job = a.j[ji];
-    // the fields the first loads need, in one batch of scalar loads
-    __asm__ volatile("" ::"s"(job.w), "s"(job.ws), "s"(job.rows), "s"(job.g0), "s"(a.cols), "s"(a.m), "s"(a.units),
-                     "s"(a.xq), "s"(a.xs), "s"(a.xsum));
-    const int rg = (int)blockIdx.x - job.g0, rows = job.rows, nb = a.cols / BLOCK;
+    const void *wp = w0;
+    const float *wsp = ws0;
+    int rows = rows0;
+    unsigned wg = blockIdx.x, step = gm >> 16;
+    if (ji) {
+        wp = job.w, wsp = job.ws, rows = job.rows;
+        wg -= (unsigned)job.wg0, step = (unsigned)job.nwg;
+    }
+    const unsigned nb = (unsigned)cols / BLOCK, groups = ((unsigned)rows + GROUP - 1) / GROUP;
+    unsigned units = ((unsigned)cols + UK - 1) / UK, first = 0;
+    if constexpr (SPLIT) {
+        first = blockIdx.z * (unsigned)a.per;
+        units = min(units - first, (unsigned)a.per);
+    }
+    const int t0 = (int)blockIdx.y * GROUP * T, m = (int)(gm & 0xffffu) - t0;
+    const unsigned mt = (unsigned)min(m, GROUP * T);  // this workgroup's tokens
+    const unsigned row_bytes = PREC == KH_Q8 ? (unsigned)cols
+                               : PREC == KH_Q4 ? (unsigned)cols / 2
+                                               : (unsigned)cols / QK_K * Q4K_BYTES;
+    constexpr unsigned UB = PREC == KH_Q4K ? Q4K_BYTES : RS::CB;  // a unit's bytes of a row
+    // (sizes fit 32 bits: mma_addresses)
+    const rsrc_t X = rsrc32(xq + (size_t)t0 * cols, mt * (unsigned)cols);
+    const rsrc_t XS = rsrc32(xs + (size_t)t0 * nb, mt * nb * 4);
+    const rsrc_t XM = rsrc32(xsum + (size_t)t0 * nb, mt * nb * 4);
+    const rsrc_t W = rsrc32(wp, (unsigned)rows * row_bytes);
+    const rsrc_t WS = rsrc32(wsp, PREC == KH_Q4K ? 0 : (unsigned)rows * nb * 4);
+    char *const st = s_stage[wv];
 
-    Lane L;
-    L.lr = lane & 15;
-    L.lg = lane >> 4;
-    const unsigned row_bytes = PREC == KH_Q8 ? (unsigned)a.cols
-                               : PREC == KH_Q4 ? (unsigned)a.cols / 2
-                                               : (unsigned)(a.cols / QK_K) * Q4K_BYTES;
-    const unsigned row = (unsigned)(rg * 16 + L.lr);
-    L.wrow = row * row_bytes;
-    L.wsrow = row * (unsigned)nb * 4;
-    if constexpr (PAIR) {
-        // column lr: token lr & 7 against the pair's block lr >> 3; lane
-        // group lg feeds k 16 lg .. + 16, i.e. block lg >> 1 of the pair
-        L.xrow = (L.lg >> 1) == (L.lr >> 3) ? (unsigned)(L.lr & 7) * (unsigned)a.cols + 16 * L.lg : XOOB;
-        L.xsrow2 = (unsigned)(L.lr & 7) * (unsigned)nb * 4;
-    } else {
-        L.xrow = (unsigned)L.lr * (unsigned)a.cols;
-        L.xsrow2 = 0;
-    }
-    L.xsrow = (unsigned)L.lr * (unsigned)nb * 4;
-    const rsrc_t W = rsrc(job.w, (size_t)rows * row_bytes);
-    const rsrc_t WS = rsrc(job.ws, PREC == KH_Q4K ? 0 : (size_t)rows * nb * 4);
-    const rsrc_t X = rsrc(a.xq, (size_t)a.m * a.cols);
-    const rsrc_t XS = rsrc(a.xs, (size_t)a.m * nb * 4), XM = rsrc(a.xsum, (size_t)a.m * nb * 4);
+    // k-ranges of KW * S units in turn (WIDE), or one
+    for (unsigned c0 = 0; c0 < (WIDE ? units : 1u); c0 += KW * S) {
+        const unsigned U = WIDE ? min(units - c0, (unsigned)(KW * S)) : units;
+        const unsigned u0 = first + c0 + U * wv / KW, cnt = first + c0 + U * (wv + 1) / KW - u0;  // this wave's units
 
-    // this wave's units: a contiguous share of the row's k-range
-    const int u0 = (int)((long long)a.units * wv / NW), u1 = (int)((long long)a.units * (wv + 1) / NW);
-    v4f acc = {0.f, 0.f, 0.f, 0.f}, accm = {0.f, 0.f, 0.f, 0.f};
-    float *ex = s_ex[wv];
-    for (int q0 = u0; q0 < u1; q0 += R) {
-        Unit<PREC, PAIR> u[R];
+        // The tokens' codes in 16-byte pieces, then their scales and code
+        // sums, 16 bytes (four blocks) a piece.  Units past the wave's share
+        // are never used and tokens past m lie past the buffers' ends.
+        constexpr int XL = UK / 64;                              // code loads of a unit of 16 tokens
+        constexpr int SP = S * NQ, SL = (GROUP * SP + WAVE - 1) / WAVE;  // scale pieces a token, loads
+        int4 rx[S][T][XL], rs[SL][T], rm[PREC == KH_Q4K ? SL : 1][T];
 #pragma unroll
-        for (int i = 0; i < R; i++) load_unit<PREC, PAIR>(u[i], q0 + i, q0 + i < u1 ? 0u : ~0u, L, W, WS, X, XS, XM, nb);
+        for (int u = 0; u < S; u++)
 #pragma unroll
-        for (int i = 0; i < R; i++)
-            if (q0 + i < u1) compute_unit<PREC, PAIR>(u[i], acc, accm, ex, L);
-    }
-    if constexpr (PREC == KH_Q4K) acc -= accm;  // paired: accm is zero in columns 8-15
-    *reinterpret_cast<v4f *>(&s_red[wv][lane * 4]) = acc;
-    __syncthreads();
-    if (wv != 0) return;
-    v4f s = *reinterpret_cast<const v4f *>(&s_red[0][lane * 4]);
-    for (int w = 1; w < NW; w++) s += *reinterpret_cast<const v4f *>(&s_red[w][lane * 4]);
-    if constexpr (PAIR) {
-        // column lr + 8 holds the same token against the pairs' odd blocks.
-        // Added through LDS: a DPP row rotate of the vector's elements was
-        // miscompiled (only element 0 rotated, the others read its result).
-        if (L.lr < PAIR_TOKENS)
-            for (int w = 0; w < NW; w++) s += *reinterpret_cast<const v4f *>(&s_red[w][(lane + 8) * 4]);
-    }
-    const int tok = L.lr;
-    if (tok >= a.m || (PAIR && tok >= PAIR_TOKENS)) return;
+            for (int tt = 0; tt < T; tt++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = rg * 16 + 4 * L.lg + i;
-        if (r < rows) {
-            float *dst = job.y + (size_t)tok * rows + r;
-            const float o = job.bias ? s[i] + job.bias[r] : s[i];
-            *dst = job.accumulate ? *dst + o : o;  // x += proj (llama.rs:273-276)
+                for (int i = 0; i < XL; i++) {
+                    const unsigned p = i * WAVE + lane, tok = tt * GROUP + p / (UK / 16), k = (u0 + u) * UK + 16 * (p % (UK / 16));
+                    const unsigned o = tok * (unsigned)cols + k;
+                    rx[u][tt][i] = bld16(X, PREC == KH_Q4K || k < (unsigned)cols ? o : OOB);  // a k tail is zero codes
+                }
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+#pragma unroll
+            for (int i = 0; i < SL; i++) {
+                const unsigned p = i * WAVE + lane, tok = tt * GROUP + p / SP;
+                const unsigned o = SL * WAVE == GROUP * SP || p < GROUP * SP ? (tok * nb + u0 * NB + 4 * (p % SP)) * 4 : OOB;
+                rs[i][tt] = bld16(XS, o);
+                if constexpr (PREC == KH_Q4K) rm[i][tt] = bld16(XM, o);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+
+        // this lane's pieces of a group's rows, from the group's first row
+        unsigned lw[RS::NL];
+#pragma unroll
+        for (int i = 0; i < RS::NL; i++) {
+            const unsigned p = i * WAVE + lane;
+            lw[i] = p / RS::RUN * row_bytes + u0 * UB + 16 * (p % RS::RUN);
+            if (RS::NL * WAVE != GROUP * RS::RUN && p >= GROUP * RS::RUN) lw[i] = OOB;
         }
+        const unsigned lws = lane < GROUP ? ((unsigned)lane * nb + u0 * NB) * 4 : OOB;
+        auto load = [&](Wts<PREC> &w, unsigned group, int u) {
+            // a unit past the wave's share, or a lane without a piece, reads
+            // past the end; a group past the last does by itself
+            const unsigned base = (unsigned)u < cnt ? group * GROUP * row_bytes + u * UB : OOB;
+#pragma unroll
+            for (int i = 0; i < RS::NL; i++) w.a[i] = bld16(W, max(base, lw[i]) >= OOB ? OOB : base + lw[i]);
+            if constexpr (PREC != KH_Q4K) {
+                const unsigned bs = (unsigned)u < cnt ? group * GROUP * nb * 4 + u * NB * 4 : OOB;
+                w.ws = bld16(WS, max(bs, lws) >= OOB ? OOB : bs + lws);
+            }
+        };
+        Wts<PREC> w[D];
+#pragma unroll
+        for (int i = 0; i < D; i++) load(w[i], wg + (i / S) * step, i % S);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // the scales, then the codes, through the wave's stage into the
+        // operand layout
+        Acts<PREC, S, T> x;
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+#pragma unroll
+            for (int u = 0; u < S; u++) {
+#pragma unroll
+                for (int i = 0; i < XL; i++) {
+                    const int p = i * WAVE + lane;
+                    *reinterpret_cast<int4 *>(st + (p / (UK / 16)) * XSTR + 16 * (p % (UK / 16))) = rx[u][tt][i];
+                }
+                wave_order();
+#pragma unroll
+                for (int k = 0; k < NB; k++) {
+                    if constexpr (PREC == KH_Q4) {
+                        // byte i of a weight block: weight i (low nibble), 16 + i (high)
+                        const char *p = st + lr * XSTR + 32 * k + 4 * lg;
+                        x.b[u][tt][k] = pack64(*reinterpret_cast<const unsigned *>(p),
+                                               *reinterpret_cast<const unsigned *>(p + 16));
+                    } else {
+                        x.b[u][tt][k] = *reinterpret_cast<const u64 *>(st + lr * XSTR + 32 * k + 8 * lg);
+                    }
+                }
+                wave_order();
+            }
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+#pragma unroll
+            for (int pass = 0; pass < (PREC == KH_Q4K ? 2 : 1); pass++) {
+#pragma unroll
+                for (int i = 0; i < SL; i++)
+                    if (SL * WAVE == GROUP * SP || i * WAVE + lane < GROUP * SP)
+                        *reinterpret_cast<int4 *>(st + (i * WAVE + lane) * 16) = pass ? rm[i][tt] : rs[i][tt];
+                wave_order();
+#pragma unroll
+                for (int u = 0; u < S; u++)
+#pragma unroll
+                    for (int q = 0; q < NQ; q++) {
+                        const char *p = st + (lr * SP + u * NQ + q) * 16 + 4 * lg;
+                        if (pass == 0) {
+                            const float v = *reinterpret_cast<const float *>(p);
+                            x.xs[u][tt][q] = PREC == KH_Q4K || (u0 + u) * NB + 4 * q + lg < nb ? v : 0.0f;
+                        } else if constexpr (PREC == KH_Q4K) {
+                            x.xm[u][tt][q] = x.xs[u][tt][q] * (float)*reinterpret_cast<const int *>(p);
+                        }
+                    }
+                wave_order();
+            }
+
+        v4f acc[T];
+#pragma unroll
+        for (int tt = 0; tt < T; tt++) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+        auto stage = [&](const Wts<PREC> &w) {
+#pragma unroll
+            for (int i = 0; i < RS::NL; i++) {
+                const int p = i * WAVE + lane;
+                if (RS::NL * WAVE == GROUP * RS::RUN || p < GROUP * RS::RUN)
+                    *reinterpret_cast<int4 *>(st + (p / RS::RUN) * RS::STR + 16 * (p % RS::RUN)) = w.a[i];
+            }
+            if constexpr (PREC != KH_Q4K)
+                if (lane < GROUP) *reinterpret_cast<int4 *>(st + lane * RS::STR + RS::SCALES) = w.ws;
+            wave_order();
+        };
+        auto compute = [&](int u) {
+            const char *const sr = st + lr * RS::STR;
+            int4 h;
+            float d, dmin;
+            if constexpr (PREC == KH_Q4K) {
+                h = *reinterpret_cast<const int4 *>(sr);
+                d = half_bits_to_float((unsigned)h.x), dmin = half_bits_to_float((unsigned)h.x >> 16);
+            }
+            // four blocks at a time: their operands, scale products and dots
+            // are the only ones live
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                float sc, mn;
+                u64 A[4];
+                if constexpr (PREC == KH_Q4K) {
+                    // sub-block lg + 4q of row lr: d * sc and dmin * m (mpp.rs:276-282, 304-315)
+                    unsigned s6, m6;
+                    q4k_scale_min_bfe(h, q4k_lane(lg + 4 * q), s6, m6);
+                    sc = d * (float)s6;
+                    mn = -(dmin * (float)m6);
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        const u64 v = *reinterpret_cast<const u64 *>(sr + RS::CODES + 64 * q + 32 * c + 8 * lg);
+                        const unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
+                        A[2 * c] = pack64(lo & 0x0f0f0f0fu, hi & 0x0f0f0f0fu);
+                        A[2 * c + 1] = pack64((lo >> 4) & 0x0f0f0f0fu, (hi >> 4) & 0x0f0f0f0fu);
+                    }
+                } else {
+                    // past the row's last block the stage holds the next row's
+                    // scale: kept out (its codes meet zero codes)
+                    const float v = *reinterpret_cast<const float *>(sr + RS::SCALES + 4 * lg);
+                    sc = (u0 + u) * NB + lg < nb ? v : 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        if constexpr (PREC == KH_Q8) {
+                            A[k] = *reinterpret_cast<const u64 *>(sr + 32 * k + 8 * lg);
+                        } else {
+                            const unsigned c = *reinterpret_cast<const unsigned *>(sr + 16 * k + 4 * lg);
+                            A[k] = pack64(nib_minus8(c & 0x0f0f0f0fu), nib_minus8((c >> 4) & 0x0f0f0f0fu));
+                        }
+                    }
+                }
+#pragma unroll
+                for (int tt = 0; tt < T; tt++) {
+                    const v16f z16 = {};
+                    const v16f P = __builtin_amdgcn_mfma_f32_16x16x1f32(sc, x.xs[u][tt][q], z16, 0, 0, 0);
+                    v4i Dv[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) Dv[k] = mma32(A[k], x.b[u][tt][4 * q + k]);
+                    if constexpr (PREC == KH_Q4K)
+                        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(mn, x.xm[u][tt][q], acc[tt], 0, 0, 0);
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[tt][i] = fmaf(P[4 * k + i], (float)Dv[k][i], acc[tt][i]);
+                    if constexpr (NQ * T > 1) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+
+        const bool plain = !SPLIT || !a.part;
+        float *yp = job.y + (size_t)t0 * rows;
+        if (!plain) yp = a.part + ((size_t)blockIdx.z * a.all + t0) * rows;
+        const bool add_old = (plain && job.accumulate) || (WIDE && c0 > 0), add_bias = plain && job.bias && !(WIDE && c0 > 0);
+        const rsrc_t BI = rsrc32(job.bias, add_bias && !add_old ? (unsigned)rows * 4 : 0);
+        const rsrc_t Y = rsrc32(yp, mt * (unsigned)rows * 4);
+        // steps run through the groups' units; buffer i takes steps i, i + D,
+        // ...: an unrolled body of TB groups brings the buffers round
+        constexpr int TB = D % S == 0 ? D / S : S % D == 0 ? 1 : D;
+        static_assert((TB * S) % D == 0, "whole rounds of buffers a body");
+        int it = 0;  // groups done: which wave adds and stores, which buffer
+        for (unsigned g = wg; g < groups; g += TB * step) {
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++) {
+                const unsigned group = g + tb * step;
+                if (group >= groups) break;
+                v4f ex[T];  // what the group's stores add: the old values, else the bias
+#pragma unroll
+                for (int tt = 0; tt < T; tt++) {
+                    const bool mine = (it * T + tt) % KW == wv;
+                    const unsigned ro = (group * GROUP + 4 * lg) * 4;
+                    const unsigned tok = (unsigned)(tt * GROUP + lr);
+                    const unsigned o = add_old ? tok * (unsigned)rows * 4 + ro : ro;
+                    ex[tt] = __builtin_bit_cast(v4f, bld16f(add_old ? Y : BI, mine ? o : OOB));
+                }
+#pragma unroll
+                for (int u = 0; u < S; u++) {
+                    const int i = tb * S + u;
+                    if ((unsigned)u < cnt) stage(w[i % D]);
+                    load(w[i % D], group + ((u + D) / S) * step, (u + D) % S);
+                    if ((unsigned)u < cnt) compute(u);
+                    wave_order();
+                }
+                // the group's partial tiles: summed and stored by one wave a tile
+#pragma unroll
+                for (int tt = 0; tt < T; tt++) {
+                    s_red[it & 1][wv][tt][lane] = acc[tt];
+                    acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+                }
+                __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+                for (int tt = 0; tt < T; tt++) {
+                    if ((it * T + tt) % KW != wv) continue;
+                    v4f s = s_red[it & 1][0][tt][lane];
+#pragma unroll
+                    for (int k = 1; k < KW; k++) s += s_red[it & 1][k][tt][lane];
+                    if (add_bias && add_old) {  // (no caller passes both: loaded here)
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            if ((int)group * GROUP + 4 * lg + i < rows) s[i] += job.bias[group * GROUP + 4 * lg + i];
+                    }
+                    // finish, quant.rs:849-858; x += proj (llama.rs:273-276)
+                    if (add_bias || add_old) s = ex[tt] + s;
+                    const int tok = tt * GROUP + lr, r = (int)group * GROUP + 4 * lg;
+                    const unsigned off = ((unsigned)tok * (unsigned)rows + (unsigned)r) * 4;
+                    if (tok < m) {
+                        if (r + 3 < rows) {
+                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, s), Y, off, 0, 0);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 3; i++) {
+                                const float v = s[i];  // (a bit cast of the element itself takes element 0)
+                                if (r + i < rows)
+                                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), Y, off + 4 * i, 0,
+                                                                          0);
+                            }
+                        }
+                    }
+                }
+                it++;
+            }
+        }
+        if constexpr (WIDE) __syncthreads();  // the next k-range adds into what this one stored
     }
 }
 
-template <int PREC, bool PAIR, int R>
-int launch_nw(kh_ctx *ctx, const MmaArgs &a, int nwg, int nw) {
+// (waves along k, units a wave, tiles of 16 tokens, units in flight, waves a SIMD)
+template <int PREC, int KW, int S, int T, int D, int WPE, bool WIDE = false, bool SPLIT = false>
+int launch_rows(kh_ctx *ctx, const MmaRows &r, MmaArgs a, unsigned gz = 1) {
+    const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    // as many workgroups as the CUs hold at WPE waves a SIMD, each job its
+    // share by rows, at least one
+    long long total = 0;
+    for (int i = 0; i < r.njobs; i++) total += (a.j[i].rows + GROUP - 1) / GROUP;
+    // one workgroup per CU, two where a one-unit slice leaves the registers
+    // for it and there are groups enough to keep both busy (q8 151936x896 at
+    // 8 rows 36.0 -> 34.1 us; 4864x896, 304 groups, 5.8 -> 6.1)
+    const int slots = cu * (4 * WPE / KW) * (S == 1 && total >= 8LL * cu ? 2 : 1) / (int)gz;
+    int nwg = 0;
+    for (int i = 0; i < r.njobs; i++) {
+        const int groups = (a.j[i].rows + GROUP - 1) / GROUP;
+        int n = total <= slots ? groups : (int)((long long)slots * groups / total);
+        n = n < 1 ? 1 : n > groups ? groups : n;
+        a.j[i].wg0 = nwg;
+        a.j[i].nwg = n;
+        nwg += n;
+    }
     if (nwg >= 0xffff) return fail(KH_DECLINED, "matmul: 65535 workgroups or more in one launch");
-    const unsigned g12 = multi_firsts(a.njobs, a.j[1].g0, a.j[2].g0);
-    if (nw == 16)
-        hipLaunchKernelGGL((gemv_mma_kernel<PREC, PAIR, 16, R>), dim3(nwg), dim3(WAVE * 16), 0, ctx->stream, g12, a);
-    else if (nw == 8)
-        hipLaunchKernelGGL((gemv_mma_kernel<PREC, PAIR, 8, R>), dim3(nwg), dim3(WAVE * 8), 0, ctx->stream, g12, a);
-    else
-        hipLaunchKernelGGL((gemv_mma_kernel<PREC, PAIR, 4, R>), dim3(nwg), dim3(WAVE * 4), 0, ctx->stream, g12, a);
+    const unsigned gy = (unsigned)((r.m + GROUP * T - 1) / (GROUP * T));
+    const unsigned gm = (unsigned)a.j[0].nwg << 16 | (unsigned)r.m;
+    hipLaunchKernelGGL((rows_mma_kernel<PREC, KW, S, T, D, WPE, WIDE, SPLIT>), dim3((unsigned)nwg, gy, gz), dim3(WAVE * KW), 0,
+                       ctx->stream, multi_firsts(r.njobs, a.j[1].wg0, a.j[2].wg0), gm, a.j[0].w, a.j[0].ws, r.x.qs,
+                       r.x.scales, a.j[0].rows, r.cols, r.x.sums, a);
     KH_HIP(hipGetLastError());
     return KH_OK;
 }
 
-template <int PREC, int R>
-int launch_mode(kh_ctx *ctx, const MmaArgs &a, int nwg, int nw) {
-    return a.m <= PAIR_TOKENS ? launch_nw<PREC, true, R>(ctx, a, nwg, nw) : launch_nw<PREC, false, R>(ctx, a, nwg, nw);
+// Units split over grid z, 8 * S a split: wide rows at more than 16 tokens,
+// whose codes a wave's registers cannot hold for the whole width.
+template <int PREC, int S>
+int launch_split(kh_ctx *ctx, const MmaRows &r, MmaArgs a) {
+    const unsigned gz = (unsigned)((r.units + 8 * S - 1) / (8 * S));
+    a.per = (int)((r.units + gz - 1) / gz);
+    a.all = r.m;
+    const MmaJob j = a.j[0];
+    int rc = launch_rows<PREC, 8, S, 2, 4, 2, false, true>(ctx, r, a, gz);
+    if (rc) return rc;
+    return launch_split_reduce(ctx, a.part, (int)gz, r.m, j.rows, j.bias, j.accumulate, j.y);
+}
+
+template <int PREC, int T>
+int launch_units(kh_ctx *ctx, const MmaRows &r, MmaArgs a) {
+    const int U = r.units;
+    if constexpr (T == 2) {
+        constexpr int S = PREC == KH_Q4K ? 2 : 4;
+        if (U > 8 * S && r.njobs == 1) {
+            const size_t gz = (size_t)(U + 8 * S - 1) / (8 * S);
+            a.part = split_partials(ctx, gz * r.m * a.j[0].rows * 4);
+            if (a.part) return launch_split<PREC, S>(ctx, r, a);
+        }
+    }
+    if (U <= 4) return launch_rows<PREC, 4, 1, T, 3, 2>(ctx, r, a);
+    if (U <= 8) return launch_rows<PREC, 8, 1, T, 3, 2>(ctx, r, a);
+    if (U <= 16) return launch_rows<PREC, 8, 2, T, 4, 2>(ctx, r, a);
+    if constexpr (PREC == KH_Q4K) {
+        if (U <= 32) return launch_rows<PREC, 8, 4, 1, 4, 2>(ctx, r, a);
+        return launch_rows<PREC, 8, 7, 1, 2, 2, true>(ctx, r, a);
+    } else {
+        if (U <= 32) return launch_rows<PREC, 8, 4, T, 4, 2>(ctx, r, a);
+        if (U <= 64) return launch_rows<PREC, 8, 8, 1, 4, 2>(ctx, r, a);
+        return launch_rows<PREC, 8, 14, 1, 2, 2, true>(ctx, r, a);
+    }
+}
+
+template <int PREC>
+int launch_prec(kh_ctx *ctx, const MmaRows &r, const MmaArgs &a) {
+    return r.m <= GROUP ? launch_units<PREC, 1>(ctx, r, a) : launch_units<PREC, 2>(ctx, r, a);
 }
 
 }  // namespace
@@ -413,50 +534,39 @@ int launch_gemv_mma(kh_ctx *ctx, int njobs, const kh_weight *const *w, const flo
     if (prec != KH_Q8 && prec != KH_Q4 && prec != KH_Q4K)
         return fail(KH_EINVAL, "matmul: the matrix-core GEMV takes quantised weights");
     if (cols % (prec == KH_Q4K ? QK_K : BLOCK)) return fail(KH_EINVAL, "matmul: width not a whole number of blocks");
-    if (MMA_TOKENS * cols >= XOOB) return fail(KH_DECLINED, "matmul: rows of codes of 128 MB or more");
     MmaArgs a{};
-    a.cols = (int)cols;
-    a.njobs = njobs;
     const int nb = (int)(cols / BLOCK);
-    a.units = prec == KH_Q4K ? (int)(cols / QK_K) : (nb + 3) / 4;
-    int nwg = 0;
+    MmaRows r{QAct{}, (int)cols, 0, njobs, prec == KH_Q4K ? (int)(cols / QK_K) : (nb + 3) / 4};
     for (int i = 0; i < njobs; i++) {
         if (w[i]->precision != prec || w[i]->cols != cols)
             return fail(KH_EINVAL, "matmul: weights of one launch share precision and width");
-        const size_t rb = prec == KH_Q8 ? cols : prec == KH_Q4 ? cols / 2 : cols / QK_K * Q4K_BYTES;
-        // rows past the end (up to 15) still address below 4 GiB
-        if ((w[i]->rows + 16) * rb >= 0xfff00000ull || (w[i]->rows + 16) * (cols / BLOCK) * 4 >= 0xfff00000ull)
+        if (!mma_addresses(prec, w[i]->rows, cols))
             return fail(KH_DECLINED, "matmul: operands of 4 GiB or more are not addressed here");
         a.j[i] = MmaJob{w[i]->qs, w[i]->scales, bias ? bias[i] : nullptr, y[i], (int)w[i]->rows,
-                        accumulate ? accumulate[i] : 0, nwg};
-        nwg += (int)((w[i]->rows + 15) / 16);
+                        accumulate ? accumulate[i] : 0, 0, 0};
     }
-    // Four waves per workgroup, each taking several rounds of R units when
-    // the rows are long: measured at or ahead of 8 and 16 waves at every
-    // shape (m = 8, us for 4 / 8 / 16 waves: Q4_K 14336x4096 23.1 / 22.8 /
-    // 33.3, 4096x14336 20.7 / 21.2 / 21.9; q8 896x4864 10.8 / 11.3 / 11.9,
-    // 151936x896 49.4 / 78.1 / 91.9)
-    int nw = 4;
-    const int forced = env_int("KVAD_MMA_WAVES", 0);  // tuning knob
-    if (forced == 4 || forced == 8 || forced == 16) nw = forced;
-    for (size_t t0 = 0; t0 < m; t0 += MMA_TOKENS) {
+    // tokens a launch: a 16-bit count
+    const size_t step = 32768;
+    for (size_t t0 = 0; t0 < m; t0 += step) {
         MmaArgs b = a;
-        b.m = (int)(m - t0 < (size_t)MMA_TOKENS ? m - t0 : MMA_TOKENS);
-        b.xq = x.qs + t0 * cols;
-        b.xs = x.scales + t0 * nb;
-        b.xsum = x.sums + t0 * nb;
+        r.m = (int)std::min(m - t0, step);
+        r.x = QAct{x.qs + t0 * cols, x.scales + t0 * nb, x.sums + t0 * nb};
         for (int i = 0; i < njobs; i++) b.j[i].y = a.j[i].y + t0 * a.j[i].rows;
         int rc;
-        // two units a round (measured against 1, 4 and 8 at m = 8: q8
-        // 151936x896 37.2 against 49.5 us at 4; Q4_K level with 1, 4 slower)
         switch (prec) {
-            case KH_Q8: rc = launch_mode<KH_Q8, 2>(ctx, b, nwg, nw); break;
-            case KH_Q4: rc = launch_mode<KH_Q4, 2>(ctx, b, nwg, nw); break;
-            default: rc = launch_mode<KH_Q4K, 2>(ctx, b, nwg, nw); break;
+            case KH_Q8: rc = launch_prec<KH_Q8>(ctx, r, b); break;
+            case KH_Q4: rc = launch_prec<KH_Q4>(ctx, r, b); break;
+            default: rc = launch_prec<KH_Q4K>(ctx, r, b); break;
         }
         if (rc) return rc;
     }
     return KH_OK;
+}
+
+bool mma_addresses(int prec, size_t rows, size_t cols) {
+    const size_t rb = prec == KH_Q8 ? cols : prec == KH_Q4 ? cols / 2 : cols / QK_K * Q4K_BYTES;
+    // the last group's overhang (up to 15 rows) included; 32 tokens' outputs
+    return (rows + 16) * rb < OOB && (rows + 16) * (cols / BLOCK) * 4 < OOB && 32 * rows * 4 < OOB && 32 * cols < ((size_t)1 << 31);
 }
 
 }  // namespace kh

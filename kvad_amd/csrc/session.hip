@@ -487,14 +487,14 @@ int ensure_pass(kh_llm *m, size_t n, size_t max_len) {
 // 128-row tiles leave most CUs idle).  A single projection (o, down, the
 // head) follows kh_matmul's rule.
 size_t rows_multi_max() {
-    static const size_t v = (size_t)env_int("KVAD_ROWS_MULTI", 32);  // tuning knob
+    static const size_t v = (size_t)env_int("KVAD_ROWS_MULTI", 64);  // tuning knob
     return v;
 }
 
 int project(kh_ctx *ctx, const kh_weight *w, const float *xs, const QAct &qa, size_t n, const float *bias, float *y,
             int accumulate = 0) {
     if (w->precision == KH_F32) return launch_matmul(ctx, w, xs, n, bias, y, accumulate);
-    if (n <= rows_multi_max() && matmul_takes_multi(n, w->rows, w->cols))
+    if (n <= rows_multi_max() && matmul_takes_multi(w->precision, n, w->rows, w->cols))
         return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, &accumulate, qa, n);
     return launch_matmul_q(ctx, w, qa, n, bias, y, accumulate);
 }
@@ -585,7 +585,7 @@ int step_rows(kh_ctx *ctx, kh_llm *m, size_t n, const RowsBuf &b, size_t max_len
                    (rc = trace_copy(ctx, tr->att ? tr->att + l * n * qd : nullptr, b.att, n * qd))))
             return rc;
         if (L.o->precision != KH_F32 && n <= (size_t)MULTI_TOKENS && n <= rows_multi_max() &&
-            multi_stages_f32(L.o->precision, n, qd)) {
+            multi_stages_f32(L.o->precision, n, L.o->rows, qd)) {
             // x += o(attn): the multi-token GEMV quantises the attention rows
             // itself, in its one launch, while they are narrow (past eight
             // rows it takes several, each quantising its rows in every

@@ -3,8 +3,8 @@ quant.rs:751-907, as forward_each calls it, llama.rs:418-434), which the
 library runs as a multi-token GEMV that streams the weights once for every
 token: on the VALU (dot4 per row and token; two token rows, or any with
 KVAD_MMA_MIN above m) or on the matrix cores (one v_mfma_i32_16x16x32_i8
-per block pair for 16 rows x 8 tokens, per block for 16 tokens; from five
-token rows).
+per block of 16 rows x 16 tokens; from five token rows, from three over
+large matrices).
 
 Bar: f32 outputs within 1e-5 x max|ref| of the oracle's matmul.  On the VALU
 path each token's row equals, to the bit, a single-token matvec of that
@@ -76,8 +76,8 @@ MMA_SHAPES = {
 @pytest.mark.parametrize("m", [3, 8, 9, 16, 17, 40])
 def test_matrix_core_tokens_match_the_oracle(ctx, monkeypatch, prec, m):
     # up to 40 rows through the matrix-core path (KVAD_MULTI_TOKENS,
-    # KVAD_MMA_MIN): block pairs up to 8 rows, a block per instruction from 9;
-    # 17 and 40 take a launch per 16 rows, each writing its own rows of y
+    # KVAD_MMA_MIN): tiles of 16 tokens, one or two a workgroup; 17 and 40 take
+    # several, each writing its own rows of y
     monkeypatch.setenv("KVAD_MULTI_TOKENS", "64")
     monkeypatch.setenv("KVAD_MMA_MIN", "2")
     for rows, cols in MMA_SHAPES[prec]:
@@ -87,6 +87,62 @@ def test_matrix_core_tokens_match_the_oracle(ctx, monkeypatch, prec, m):
         bias = O.normal(rows + 7, rows)
         for b in (None, bias):
             close(w.matmul_bt(xs, m, b), oracle_matmul(prec, parts, rows, cols, xs, m, b))
+
+
+# k-ranges at the edges of the matrix-core kernel's slices: a wave holds 1, 2,
+# 4, 7 (Q4_K, 256 wide) or 1, 2, 4, 8, 14 (q8 / q4, 128 wide) units of the
+# row, eight waves a workgroup; past the widest slice the row takes a second
+# range, past 16 tokens a split over the grid.  Tails of one block included.
+EDGE_COLS = {
+    "q8": [128, 512, 544, 1056, 2048, 2080, 4096, 4128, 8224, 14368],
+    "q4": [512, 1024, 1056, 2080, 4128, 8192, 14336, 14368],
+    "q4k": [256, 1024, 1280, 2048, 2304, 4096, 4352, 8192, 8448, 14336, 14592],
+}
+
+
+@pytest.mark.parametrize("prec", list(EDGE_COLS))
+@pytest.mark.parametrize("m", [5, 16, 17, 33])
+def test_matrix_core_k_ranges_match_the_oracle(ctx, monkeypatch, prec, m):
+    monkeypatch.setenv("KVAD_MULTI_TOKENS", "64")
+    rows = 35  # three 16-row groups, the last part-filled
+    for cols in EDGE_COLS[prec]:
+        say("matrix-core k-range", prec, m, rows, cols)
+        w, parts = make(ctx, prec, rows, cols, seed=cols + m)
+        xs = O.normal(cols + 11 * m, m * cols)
+        bias = O.normal(rows + 5, rows)
+        close(w.matmul_bt(xs, m, bias), oracle_matmul(prec, parts, rows, cols, xs, m, bias))
+
+
+@pytest.mark.parametrize("prec", ["q8", "q4", "q4k"])
+@pytest.mark.parametrize("rows,cols", [(4113, 256), (8210, 512), (33001, 256), (4500, 2304)])
+def test_matrix_core_groups_in_turn_match_the_oracle(ctx, monkeypatch, prec, rows, cols):
+    # more 16-row groups than workgroups: one, two or a few groups a
+    # workgroup, and two workgroups a CU from eight groups a CU
+    monkeypatch.setenv("KVAD_MULTI_TOKENS", "64")
+    for m in (5, 19):
+        say("matrix-core groups", prec, m, rows, cols)
+        w, parts = make(ctx, prec, rows, cols, seed=rows + m)
+        xs = O.normal(rows + 3 * m, m * cols)
+        close(w.matmul_bt(xs, m), oracle_matmul(prec, parts, rows, cols, xs, m))
+
+
+def test_matrix_core_keeps_odd_values_to_their_rows(ctx, monkeypatch):
+    # an infinite or NaN scale in one weight row or token stays in that row:
+    # the k tail's lanes read the next row's scale
+    monkeypatch.setenv("KVAD_MULTI_TOKENS", "64")
+    rows, cols, m = 40, 160, 6
+    s, q = O.quantize_q8(O.normal(3, rows * cols, 0.02), rows, cols)
+    s = s.reshape(rows, cols // 32).copy()
+    s[7, 0], s[21, 1] = np.inf, np.nan
+    xs = O.normal(4, m * cols)
+    w = K.Weight.from_q8(ctx, rows, cols, s.ravel(), q)
+    got = w.matmul_bt(xs, m).reshape(m, rows)
+    bad = np.zeros(rows, bool)
+    bad[[7, 21]] = True
+    assert not np.isfinite(got[:, bad]).any()
+    s[7, 0] = s[21, 1] = 0.0
+    want = O.matmul_q8(s.ravel(), q, rows, cols, xs, m).reshape(m, rows)
+    close(got[:, ~bad].ravel(), np.ascontiguousarray(want[:, ~bad]).ravel())
 
 
 def test_many_token_slots_stream_in_launches(ctx, monkeypatch):
