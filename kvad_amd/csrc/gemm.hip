@@ -639,12 +639,19 @@ __global__ __launch_bounds__(THREADS) void gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[rt][tt][v] = 0.0f;
 
-    load_stage(0);
-    for (int k0 = 0; k0 < K; k0 += FK) {
+    // split z's stages (all of them without a split)
+    int k_begin = 0, k_end = K;
+    if (a.ksplit > 1) {
+        const int S = (K + FK - 1) / FK, per = (S + a.ksplit - 1) / a.ksplit;
+        k_begin = min(S, (int)blockIdx.z * per) * FK;
+        k_end = min(K, k_begin + per * FK);
+    }
+    if (k_begin < k_end) load_stage(k_begin);
+    for (int k0 = k_begin; k0 < k_end; k0 += FK) {
         __syncthreads();
         store_stage();
         __syncthreads();
-        if (k0 + FK < K) load_stage(k0 + FK);
+        if (k0 + FK < k_end) load_stage(k0 + FK);
         // lane half h takes k = 16h + 4q + e of the stage; A and B agree on it
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -668,7 +675,8 @@ __global__ __launch_bounds__(THREADS) void gemm_f32_kernel(GemmArgs a) {
                 }
         }
     }
-    store_tiles<RT, TT>(a, acc, n0 + wr0, m0 + wm0, a.M, lane);
+    if (a.ksplit > 1) store_partials<RT, TT>(a, acc, n0 + wr0, m0 + wm0, a.M, lane);
+    else store_tiles<RT, TT>(a, acc, n0 + wr0, m0 + wm0, a.M, lane);
 }
 
 // Tile shape for a problem: the largest tile that still gives every CU a
@@ -742,6 +750,8 @@ int launch_i8(kh_ctx *ctx, const GemmArgs &a, int max_tiles, int tile_m, int til
     return KH_OK;
 }
 
+int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m);
+
 // The f32 GEMM runs best on shorter token tiles than the int8 one (swept at
 // both prefill shapes): 64 tokens while that still gives two workgroups per
 // CU, else 32.
@@ -752,24 +762,27 @@ Shape pick_shape_f32(int M, int N, int cu) {
     return nt * ((M + 63) / 64) >= 2LL * cu ? T128x64 : T128x32;
 }
 
-int launch_f32gemm(kh_ctx *ctx, const GemmArgs &a) {
+int launch_f32gemm(kh_ctx *ctx, GemmArgs a) {
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const unsigned gx = (unsigned)((a.N + 127) / 128);
-    switch (pick_shape_f32(a.M, a.N, cu)) {
+    const Shape sh = pick_shape_f32(a.M, a.N, cu);
+    const int tile_m = sh == T128x128 ? 128 : sh == T128x64 ? 64 : 32;
+    const int rc = plan_split_f32(ctx, a, tile_m);
+    if (rc) return rc;
+    const dim3 grid((unsigned)((a.N + 127) / 128), (unsigned)((a.M + tile_m - 1) / tile_m),
+                    a.ksplit > 1 ? (unsigned)a.ksplit : 1u);
+    switch (sh) {
         case T128x128:
-            hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 2, 2>), dim3(gx, (a.M + 127) / 128), dim3(THREADS), 0,
-                               ctx->stream, a);
+            hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 2, 2>), grid, dim3(THREADS), 0, ctx->stream, a);
             break;
         case T128x64:
-            hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 2, 1>), dim3(gx, (a.M + 63) / 64), dim3(THREADS), 0,
-                               ctx->stream, a);
+            hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 2, 1>), grid, dim3(THREADS), 0, ctx->stream, a);
             break;
         default:
-            hipLaunchKernelGGL((gemm_f32_kernel<4, 1, 1, 1>), dim3(gx, (a.M + 31) / 32), dim3(THREADS), 0,
-                               ctx->stream, a);
+            hipLaunchKernelGGL((gemm_f32_kernel<4, 1, 1, 1>), grid, dim3(THREADS), 0, ctx->stream, a);
             break;
     }
     KH_HIP(hipGetLastError());
+    if (a.ksplit > 1) return launch_split_reduce(ctx, a.part, a.ksplit, a.M, a.N, a.bias, a.accumulate, a.y);
     return KH_OK;
 }
 
@@ -833,28 +846,25 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
     return KH_OK;
 }
 
-int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
+namespace {
+
+// Sets a's split-K fields: the k-stages (`stages` of them, at least `min_st`
+// a split) are split so that the grid comes to about SPLIT_PER_CU workgroups
+// per CU (a CU holds several: one's loads wait while another's MFMAs run), at
+// most SPLIT_MAX splits, and partials (4 M N bytes a split, written and read
+// again) of at most the weights' wbytes or 4 MiB, whichever is more (a small
+// weight such as a router's 64 rows would otherwise never split: 512 tokens x
+// 64 x 2048, 16 workgroups, 22.6 us unsplit).
+int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st, size_t wbytes) {
     a.ksplit = 0;
-    if (a.tiles) return KH_OK;  // grouped launches are not split
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    // Split the k-stages so that the grid comes to about SPLIT_PER_CU
-    // workgroups per CU (a CU holds several: one's loads wait while
-    // another's MFMAs run), with at least SPLIT_MIN_STAGES stages a split,
-    // at most SPLIT_MAX splits, and partials (4 M N bytes a split, written
-    // and read again) of at most the weights' N K bytes or 4 MiB, whichever
-    // is more (a small weight such as a router's 64 rows would otherwise
-    // never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit).
-    // a paired launch (a.y2) holds both weights' tiles and partial planes
-    const int pair = a.y2 ? 2 : 1;
-    const long long tiles = (long long)((a.N + tile_n - 1) / tile_n) * ((a.M + tile_m - 1) / tile_m) * pair;
-    const int S = (a.K + BK - 1) / BK;
-    const size_t plane = (size_t)a.M * a.N * 4 * pair;
+    const size_t plane = (size_t)a.M * a.N * 4 * (a.y2 ? 2 : 1);
     long long ks = ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
-    ks = std::min<long long>(ks, S / SPLIT_MIN_STAGES);
+    ks = std::min<long long>(ks, stages / min_st);
     ks = std::min<long long>(ks, SPLIT_MAX);
-    ks = std::min<long long>(ks, (long long)(std::max((size_t)a.N * a.K * pair, (size_t)4 << 20) / plane));
+    ks = std::min<long long>(ks, (long long)(std::max(wbytes, (size_t)4 << 20) / plane));
     const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
-    if (forced > 0) ks = std::min(forced, S);
+    if (forced > 0) ks = std::min(forced, stages);
     ks = std::min<long long>(ks, (long long)(SPLIT_BYTES / plane));
     if (ks < 2) return KH_OK;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -867,6 +877,28 @@ int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
     a.ksplit = (int)ks;
     a.part = static_cast<float *>(ctx->gemm.ptr);
     return KH_OK;
+}
+
+// The f32 GEMM's split, at least two stages of 32 k-values each.  A few
+// 128-row tiles over long rows had left most CUs idle and every workgroup
+// waiting out its stages in turn: (90 tokens, 3000 rows, 2052 columns), 72
+// workgroups of 65 stages, 56 -> 22 us; 4096x4096 at 2 / 32 / 128 tokens 114 ->
+// 20 / 21 / 50; a 64x2048 router at 4 / 512 54 -> 6.3 / 10.8; 896x4864 at 16
+// 126 -> 11.5; 512x512 at 16 15.7 -> 6.9 (at least four stages 8.5, eight 11.7).
+int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
+    const long long tiles = (long long)((a.N + 127) / 128) * ((a.M + tile_m - 1) / tile_m);
+    return set_split(ctx, a, tiles, (a.K + FK - 1) / FK, 2, (size_t)a.N * a.K * 4);
+}
+
+}  // namespace
+
+int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
+    a.ksplit = 0;
+    if (a.tiles) return KH_OK;  // grouped launches are not split
+    // a paired launch (a.y2) holds both weights' tiles and partial planes
+    const int pair = a.y2 ? 2 : 1;
+    const long long tiles = (long long)((a.N + tile_n - 1) / tile_n) * ((a.M + tile_m - 1) / tile_m) * pair;
+    return set_split(ctx, a, tiles, (a.K + BK - 1) / BK, SPLIT_MIN_STAGES, (size_t)a.N * a.K * pair);
 }
 
 int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y,

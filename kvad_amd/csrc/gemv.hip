@@ -1295,7 +1295,9 @@ bool mma_takes(size_t m, size_t rows, size_t cols) {
 bool matmul_takes_multi(int precision, size_t m, size_t rows, size_t cols) {
     const int forced = env_int("KVAD_MULTI_TOKENS", 0);  // tuning knob: the multi-token GEMV up to this many rows
     if (forced > 0) return m <= (size_t)forced;
-    if (!mma_addresses(precision, rows, cols)) return m <= (size_t)MULTI_TOKENS;
+    // (the GEMM's own tuning knobs ask for the GEMM)
+    if (!mma_addresses(precision, rows, cols) || env_int("KVAD_GEMM_TILE_M", 0) > 0 || env_int("KVAD_GEMM_KSPLIT", 0) > 0)
+        return m <= (size_t)MULTI_TOKENS;
     // Up to 16 rows the matrix-core kernel is ahead of the GEMM everywhere
     // (with the rows' quantisation, us, GEMM / it: Q4_K 14336x4096 24.8 /
     // 14.1, 4096x14336 25.0 / 16.3, 4096x4096 14.1 / 8.1; q8 896x4864 10.7 /

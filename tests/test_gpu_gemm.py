@@ -100,6 +100,24 @@ def test_split_k_matches_the_oracle(ctx, prec, monkeypatch):
             np.testing.assert_array_equal(w.matmul_bt(xs, m, bias), got)  # the same order every call
 
 
+@pytest.mark.parametrize("tile", ["32", "64", "128"])
+def test_f32_split_k_matches_the_oracle(ctx, monkeypatch, tile):
+    # the f32 GEMM's 32-wide k-stages split over the grid: fewer stages than
+    # splits, a part-filled last stage, rows that take the scalar tail
+    monkeypatch.setenv("KVAD_GEMM_TILE_M", tile)
+    for m, rows, cols in [(2, 130, 4), (33, 129, 68), (90, 300, 2052), (17, 64, 2048), (130, 257, 516)]:
+        w, parts = make(ctx, "f32", rows, cols, seed=m + rows)
+        xs = O.normal(m + 1, m * cols)
+        bias = O.normal(rows + 2, rows)
+        want = oracle_matmul("f32", parts, rows, cols, xs, m, bias)
+        for ks in ("", "1", "3", "16"):  # automatic, none, forced
+            say("f32 split-k", tile, m, rows, cols, ks or "auto")
+            monkeypatch.setenv("KVAD_GEMM_KSPLIT", ks)
+            got = w.matmul_bt(xs, m, bias)
+            close(got, want)
+            np.testing.assert_array_equal(w.matmul_bt(xs, m, bias), got)  # the same order every call
+
+
 def test_split_k_partials_of_exact_integers_are_exact(ctx, monkeypatch):
     # scale-1 q8 blocks (the block maximum sits where the other operand is 0)
     # and small activation codes: every partial and every sum of partials is
