@@ -602,19 +602,24 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const int32_t *len_
 
 // Fixed-order butterfly within each wave, then the four wave results in wave
 // order; every thread gets the result.  s_w holds four floats.
-template <typename F>
+template <int NW, typename F>
 __device__ __forceinline__ float block_reduce(float v, float *s_w, F op) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o));
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = v;
     __syncthreads();
-    return op(op(s_w[0], s_w[1]), op(s_w[2], s_w[3]));
+    float x = s_w[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) x = op(x, s_w[w]);
+    return x;
 }
 
 constexpr int MAX_SPLITS = 4096;
+constexpr int WIDE_NW = 8;  // waves of a merge of more splits than merge_fast_max
 
-// Exclusive prefix sum of one int per thread over the workgroup (256
-// threads); *total gets the sum.  s holds four ints and is free again on return.
+// Exclusive prefix sum of one int per thread over the workgroup (NW waves);
+// *total gets the sum.  s holds NW ints and is free again on return.
+template <int NW>
 __device__ __forceinline__ int block_excl_scan(int v, int *s, int *total) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int x = v;
@@ -627,7 +632,7 @@ __device__ __forceinline__ int block_excl_scan(int v, int *s, int *total) {
     __syncthreads();
     int off = 0, tot = 0;
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
+    for (int w = 0; w < NW; w++) {
         const int t = s[w];
         off += w < wv ? t : 0;
         tot += t;
@@ -637,43 +642,127 @@ __device__ __forceinline__ int block_excl_scan(int v, int *s, int *total) {
     return off + x - v;
 }
 
-// The merge of one head's splits (one workgroup of 256 threads), over the
+// The terms one wave takes back out of a merge: of the listed (straddling)
+// splits first, first + 1, .. first + 256 / P - 1, then the same from
+// first + stride, ..., the positions whose weight w = e^{s - M} * inv is under
+// 1e-8 and not 0, each w times its value row's float4 d4 + lane % NQ; summed
+// over the positions a lane group lane / NQ took.  256 scores a load, four
+// loads in flight; the positions pass through the wave's queue in LDS, so
+// there is no barrier and a chain of two loads while it holds them.
+constexpr int QCAP = 512;  // queued positions at most
+template <int NQ, typename VRow>
+__device__ __forceinline__ float4 skipped_terms(const uint16_t *list, int nlist, int first, int stride, const float *psc,
+                                                int n_head, int h, int P, int L, float M, float inv, int d4,
+                                                VRow vrow, int2 *queue, int lane) {
+    constexpr int GW = 64 / NQ, RB = 4;
+    const int lp = __builtin_ctz(P), grp = lane / NQ, dq = lane % NQ;
+    const unsigned long long below = (1ull << lane) - 1;
+    float4 fix = make_float4(0.f, 0.f, 0.f, 0.f);
+    int nk = 0;  // queued (the same in every lane)
+    auto flush = [&]() {
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own queue
+        for (int k0 = grp; k0 < nk; k0 += 8 * GW) {
+            float4 vv[8];
+            float ww[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int kk = k0 + u * GW;
+                const int2 q = queue[kk < nk ? kk : k0];
+                vv[u] = vrow(q.x, d4 + dq);
+                ww[u] = kk < nk ? __builtin_bit_cast(float, q.y) : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                fix.x = fmaf(ww[u], vv[u].x, fix.x);
+                fix.y = fmaf(ww[u], vv[u].y, fix.y);
+                fix.z = fmaf(ww[u], vv[u].z, fix.z);
+                fix.w = fmaf(ww[u], vv[u].w, fix.w);
+            }
+        }
+        nk = 0;
+        __asm__ volatile("" ::: "memory");
+    };
+    for (int r0 = first; r0 < nlist; r0 += RB * stride) {
+        float4 sc4[RB];
+        int t0[RB];
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            const int e = r0 + r * stride + ((4 * lane) >> lp), k = (4 * lane) & (P - 1);
+            const int j = list[e < nlist ? e : r0];
+            t0[r] = e < nlist ? j * P + k : L;  // past the end: none
+            sc4[r] = *reinterpret_cast<const float4 *>(psc + ((size_t)j * n_head + h) * P + k);
+        }
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            if (nk > QCAP - 256) flush();
+            const float sc[4] = {sc4[r].x, sc4[r].y, sc4[r].z, sc4[r].w};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float w = 0.0f;
+                if (t0[r] + u < L && sc[u] != -INFINITY) {
+                    w = expf(sc[u] - M);
+                    w = w * inv;
+                    // kept (a weight that underflows to 0 adds nothing either)
+                    w = w < 1e-8f ? w : 0.0f;
+                }
+                const unsigned long long hit = __builtin_amdgcn_ballot_w64(w > 0.0f);
+                if (w > 0.0f)
+                    queue[nk + __builtin_popcountll(hit & below)] = make_int2(t0[r] + u, __builtin_bit_cast(int, w));
+                nk += __builtin_popcountll(hit);
+            }
+        }
+    }
+    flush();
+    return fix;
+}
+
+// The merge of one head's splits (one workgroup of NW waves), over the
 // head's dims [d0, d0 + D):
 //   M = max m_j,  S = sum_j l_j e^{m_j - M},  out = sum_j e^{m_j - M} acc_j / S,
 // less the terms the reference skips, w_t = e^{s_t - M} * (1/S) < 1e-8
 // (mod.rs:807).  Decided per split from its extremes: a split whose largest
 // weight is under 1e-8 is left out whole; one whose smallest is not is taken
-// whole; the straddling ones have their stored scores read, 1024 candidates
-// at a time, and the value rows of just the skipped positions are gathered,
-// all loads in flight together, and taken back out.  The first splits'
-// partial values are loaded before M is known, so their latency overlaps the
-// reductions.  vrow(t, q) is float4 q of position t's value row for this
-// head.  Every list is compacted in index order and every sum has a fixed
-// order.
-template <int HD, int D, typename VRow>
+// whole; the straddling ones have their stored scores read and the value rows
+// of just the skipped positions are gathered and taken back out.  The first
+// splits' partial values are loaded before M is known, so their latency
+// overlaps the reductions.  vrow(t, q) is float4 q of position t's value row
+// for this head.  Every list and every sum has a fixed order.
+//
+// Straddling splits are the rule over long caches: scores that spread by two
+// nats put one position in a thousand under the line at 20000 positions, so
+// every fourth split of 128 holds one or two.  Each wave takes straddling
+// splits of its own, 256 scores a load (P divides 256), queues the skipped
+// positions in its own LDS and gathers their rows: no barrier between the
+// list and the last sum, and a chain of two loads whatever the list's length
+// over NW waves.  Measured, scores spread by 2 (us per layer, split and merge,
+// before with the candidates scanned 1024 at a time
+// by a block of 256): 32 heads of 128 over 20001 positions 52 -> 45, over 32768
+// 88 -> 73, 14 heads of 64 over 20001 / 32768 25 / 52 -> 17 / 24, 16 latent heads
+// over 32768 50 -> 42.
+template <int HD, int D, int NW, typename VRow>
 __device__ __forceinline__ void merge_head(const float *pm, const float *pl, const float *pmin, const float *pacc,
                                            const float *psc, int ns, int n_head, int h, int d0, int P, int L,
                                            VRow vrow, float *out) {
-    constexpr int NQ = D / 4, NSG = 256 / NQ;  // float4 slices of the dims; split (or position) groups
-    constexpr int PER = MAX_SPLITS / 256;      // splits per thread at most
-    constexpr int CAP = 2048;                  // skipped positions gathered per flush
-    constexpr int NB = 8;                      // partial values in flight per thread
-    const int tid = threadIdx.x;
-    __shared__ float s_w[2][4];
-    __shared__ int s_scan[4];
+    constexpr int NT = 64 * NW;
+    constexpr int NQ = D / 4, NSG = NT / NQ;  // float4 slices of the dims; split groups
+    constexpr int PER = MAX_SPLITS / NT;       // splits per thread at most
+    constexpr int NB = NW >= 16 ? 4 : 8;       // partial values in flight per thread
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ float s_w[2][NW];
+    __shared__ int s_scan[NW];
     __shared__ float s_c[MAX_SPLITS];           // e^{m_j - M}, or 0 for a split left out
-    __shared__ int s_list[MAX_SPLITS];          // straddling splits, in index order
-    __shared__ __align__(16) float s_acc[NSG][D];
-    __shared__ __align__(16) float s_fix[NSG][D];
-    __shared__ int s_kpos[CAP];
-    __shared__ float s_kw[CAP];
+    __shared__ uint16_t s_list[MAX_SPLITS];     // straddling splits, in index order
+    __shared__ __align__(16) float s_acc[NW][D];
+    __shared__ __align__(16) float s_fix[NW][D];
+    __shared__ int2 s_queue[NW][QCAP];          // a wave's skipped positions and their weights' bits
 
     const int sg = tid / NQ, dq = tid % NQ;
     // each thread a run of splits, its statistics held in registers: loaded
     // first (the reductions below wait on them, and loads complete in issue
     // order), as buffer loads that read zero past the last split, under a
     // bound uniform over the workgroup, so no load waits on a branch
-    const int per = (ns + 255) / 256, i0 = tid * per, n = min(ns - i0, per);
+    const int per = (ns + NT - 1) / NT, i0 = tid * per, n = min(ns - i0, per);
     const size_t sbytes = (size_t)ns * n_head * 4;
     const rsrc_t PM = rsrc(pm, sbytes), PL = rsrc(pl, sbytes), PN = rsrc(pmin, sbytes);
     float m[PER], l[PER], mn[PER];
@@ -699,7 +788,7 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
 #pragma unroll
     for (int u = 0; u < PER; u++)
         if (u < n) mx = fmaxf(mx, m[u]);
-    const float M = block_reduce(mx, s_w[0], [](float x, float y) { return fmaxf(x, y); });
+    const float M = block_reduce<NW>(mx, s_w[0], [](float x, float y) { return fmaxf(x, y); });
     float s = 0.0f;
     float c[PER];
 #pragma unroll
@@ -709,7 +798,7 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
             s = fmaf(l[u], c[u], s);
         }
     }
-    const float S = block_reduce(s, s_w[1], [](float x, float y) { return x + y; });
+    const float S = block_reduce<NW>(s, s_w[1], [](float x, float y) { return x + y; });
     const float inv = 1.0f / S;  // inv = 1 / sum, tensor.rs:304
 
     unsigned mask = 0;  // straddling splits of this thread's run
@@ -722,11 +811,11 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
         }
     }
     int nstr;
-    int at = block_excl_scan(__builtin_popcount(mask), s_scan, &nstr);  // its barrier publishes s_c
+    int at = block_excl_scan<NW>(__builtin_popcount(mask), s_scan, &nstr);  // its barrier publishes s_c
     if (nstr) {
 #pragma unroll
         for (int u = 0; u < PER; u++)
-            if (mask >> u & 1u) s_list[at++] = i0 + u;
+            if (mask >> u & 1u) s_list[at++] = (uint16_t)(i0 + u);
     }
 
     // acc[d] = sum_j c_j acc_j[d]: thread (split group sg, float4 slice dq)
@@ -743,82 +832,40 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
             x.w = fmaf(cu, v[u].w, x.w);
         }
         j0 += NB * NSG;
-        if (j0 >= ns) break;
+        if (j0 - sg >= ns) break;  // uniform: every thread of the workgroup alike
 #pragma unroll
         for (int u = 0; u < NB; u++) v[u] = pa_load(j0 + u * NSG);
     }
-    *reinterpret_cast<float4 *>(&s_acc[sg][4 * dq]) = x;
 
-    // the skipped terms of the straddling splits: 1024 candidates a batch,
-    // four consecutive positions of one split per thread
+    // the skipped terms of the straddling splits, a wave a run of them
     float4 fix = make_float4(0.f, 0.f, 0.f, 0.f);
     if (nstr) {
         __syncthreads();  // s_list
-        int nk = 0;       // listed skipped positions (the same in every thread)
-        const int ncand = nstr * P;
-        for (int c0 = 0; c0 < ncand; c0 += 1024) {
-            const int cand = c0 + 4 * tid;
-            float w4[4] = {0.f, 0.f, 0.f, 0.f};
-            int t0 = 0, cnt = 0;
-            if (cand < ncand) {
-                const int j = s_list[cand / P], k = cand % P;
-                t0 = j * P + k;
-                const float4 sc4 = *reinterpret_cast<const float4 *>(psc + ((size_t)j * n_head + h) * P + k);
-                const float sc[4] = {sc4.x, sc4.y, sc4.z, sc4.w};
+        const int ew = 256 / P;
+        fix = skipped_terms<NQ>(s_list, nstr, wave * ew, NW * ew, psc, n_head, h, P, L, M, inv, d0 / 4, vrow,
+                                s_queue[wave], lane);
+    }
+    // the wave's groups by butterfly, then the waves in order
+    auto over_groups = [&](float4 &f) {
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    if (t0 + u < L && sc[u] != -INFINITY) {
-                        float w = expf(sc[u] - M);
-                        w = w * inv;
-                        // kept (a weight that underflows to 0 adds nothing either)
-                        w4[u] = w < 1e-8f ? w : 0.0f;
-                        cnt += w4[u] > 0.0f;
-                    }
-                }
-            }
-            int added;
-            int o = nk + block_excl_scan(cnt, s_scan, &added);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                if (w4[u] > 0.0f) {
-                    s_kpos[o] = t0 + u;
-                    s_kw[o] = w4[u];
-                    o++;
-                }
-            }
-            nk += added;
-            __syncthreads();
-            if (nk > CAP - 1024 || c0 + 1024 >= ncand) {
-                // gather: thread (group sg, slice dq) takes listed positions sg, sg + NSG, ...
-                for (int k0 = sg; k0 < nk; k0 += 4 * NSG) {
-                    float4 vv[4];
-                    float ww[4];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int kk = k0 + u * NSG;
-                        const bool ok = kk < nk;
-                        vv[u] = vrow(s_kpos[ok ? kk : 0], d0 / 4 + dq);
-                        ww[u] = ok ? s_kw[kk] : 0.0f;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        fix.x = fmaf(ww[u], vv[u].x, fix.x);
-                        fix.y = fmaf(ww[u], vv[u].y, fix.y);
-                        fix.z = fmaf(ww[u], vv[u].z, fix.z);
-                        fix.w = fmaf(ww[u], vv[u].w, fix.w);
-                    }
-                }
-                nk = 0;
-                __syncthreads();
-            }
+        for (int o = NQ; o < 64; o <<= 1) {
+            f.x = f.x + __shfl_xor(f.x, o);
+            f.y = f.y + __shfl_xor(f.y, o);
+            f.z = f.z + __shfl_xor(f.z, o);
+            f.w = f.w + __shfl_xor(f.w, o);
         }
-        *reinterpret_cast<float4 *>(&s_fix[sg][4 * dq]) = fix;
+    };
+    over_groups(x);
+    if (lane < NQ) *reinterpret_cast<float4 *>(&s_acc[wave][4 * lane]) = x;
+    if (nstr) {
+        over_groups(fix);
+        if (lane < NQ) *reinterpret_cast<float4 *>(&s_fix[wave][4 * lane]) = fix;
     }
     __syncthreads();
     if (tid < NQ) {
         float4 x = *reinterpret_cast<const float4 *>(&s_acc[0][4 * tid]);
 #pragma unroll
-        for (int g = 1; g < NSG; g++) {
+        for (int g = 1; g < NW; g++) {
             const float4 y = *reinterpret_cast<const float4 *>(&s_acc[g][4 * tid]);
             x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
         }
@@ -826,7 +873,7 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
         if (nstr) {
             float4 f = *reinterpret_cast<const float4 *>(&s_fix[0][4 * tid]);
 #pragma unroll
-            for (int g = 1; g < NSG; g++) {
+            for (int g = 1; g < NW; g++) {
                 const float4 z = *reinterpret_cast<const float4 *>(&s_fix[g][4 * tid]);
                 f = make_float4(f.x + z.x, f.y + z.y, f.z + z.z, f.w + z.w);
             }
@@ -847,19 +894,25 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
 // partial values, D / 16 float4s a lane-row of 64 / (D / 16) splits), the maximum and the sum are
 // wave butterflies (each wave computes the same ones, in the same order),
 // the weights e^{m_j - M} pass through the wave's own LDS row, and the
-// split groups' sums meet by butterfly.  Returns false, having written
-// nothing, when a split straddles the 1e-8 line (some but not all of its
-// weights skipped): the caller then runs merge_head, which handles those.
+// split groups' sums meet by butterfly.  The straddling splits' skipped terms
+// come after, each wave over all of them for its own dims (skipped_terms).
 // The most splits merge_head_fast takes for D dims: its partial values'
 // split groups and its statistics' four splits a lane both cover them, and
-// no more than 128: the more splits, the likelier one straddles the 1e-8
-// line, and a straddle costs the fast path's loads on top of merge_head's
-// (latent attention at L = 32768, 256 splits of random data: 40.8 -> 43.2 us
-// per layer when taken).
-constexpr int merge_fast_max(int d) { return 16 * 64 / (d / 16) < 128 ? 16 * 64 / (d / 16) : 128; }
-template <int HD, int D>
-__device__ __forceinline__ bool merge_head_fast(const float *pm, const float *pl, const float *pmin, const float *pacc,
-                                                int ns, int n_head, int h, int d0, float *out) {
+// no more than 128 (past that merge_head's waves share the partials out).
+__host__ __device__ constexpr int merge_fast_max(int d) { return 16 * 64 / (d / 16) < 128 ? 16 * 64 / (d / 16) : 128; }
+// Splits of 256 positions leave to merge_head, too: over a cache that long
+// (16384 positions on) a third of them and more straddle, which its eight
+// waves share and the fast path's each go through (14 heads of 64 over 32768
+// positions, scores spread by 2: 53-70 us fast, 24 shared; without a
+// straddling split 13.4 and 13.7).  The host asks for a launch's most splits,
+// the kernel for those of the length it finds.
+__host__ __device__ constexpr bool merge_takes_fast(int d, int ns, int P) {
+    return ns <= merge_fast_max(d) && P <= 128;
+}
+template <int HD, int D, typename VRow>
+__device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl, const float *pmin, const float *pacc,
+                                                const float *psc, int ns, int n_head, int h, int d0, int P, int L,
+                                                VRow vrow, float *out) {
     constexpr int NQ = D / 16;      // float4s of a wave's dims
     constexpr int SG = 64 / NQ;     // split groups a wave-row holds
     constexpr int PJ = 16;          // partial values a lane holds at most
@@ -900,16 +953,9 @@ __device__ __forceinline__ bool merge_head_fast(const float *pm, const float *pl
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum = sum + __shfl_xor(sum, o);
     const float inv = 1.0f / sum;  // inv = 1 / sum, tensor.rs:304
-    bool straddle = false;
 #pragma unroll
-    for (int u = 0; u < PS; u++) {
-        if (lane + 64 * u < ns) {
-            const bool out_whole = c[u] * inv < 1e-8f;  // every weight of the split is skipped
-            if (!out_whole && expf(mn[u] - mx) * inv < 1e-8f) straddle = true;
-            s_c[wave][lane + 64 * u] = out_whole ? 0.0f : c[u];
-        }
-    }
-    if (__builtin_amdgcn_ballot_w64(straddle)) return false;  // the same in every wave
+    for (int u = 0; u < PS; u++)  // a split whose every weight is skipped adds nothing
+        if (lane + 64 * u < ns) s_c[wave][lane + 64 * u] = c[u] * inv < 1e-8f ? 0.0f : c[u];
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the wave's own LDS row
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -928,13 +974,36 @@ __device__ __forceinline__ bool merge_head_fast(const float *pm, const float *pl
         x.z = x.z + __shfl_xor(x.z, o);
         x.w = x.w + __shfl_xor(x.w, o);
     }
-    if (sg == 0)
-        *reinterpret_cast<float4 *>(out + (size_t)h * HD + d) = make_float4(x.x * inv, x.y * inv, x.z * inv, x.w * inv);
-    return true;
+    x = make_float4(x.x * inv, x.y * inv, x.z * inv, x.w * inv);
+    __shared__ uint16_t s_list[4][PS * 64];  // straddling splits, in index order, a copy a wave
+    __shared__ int2 s_queue[4][QCAP];
+    int nstr = 0;
+#pragma unroll
+    for (int u = 0; u < PS; u++) {
+        const bool straddle =
+            lane + 64 * u < ns && !(c[u] * inv < 1e-8f) && expf(mn[u] - mx) * inv < 1e-8f;
+        const unsigned long long hit = __builtin_amdgcn_ballot_w64(straddle);
+        if (straddle) s_list[wave][nstr + __builtin_popcountll(hit & ((1ull << lane) - 1))] = (uint16_t)(lane + 64 * u);
+        nstr += __builtin_popcountll(hit);
+    }
+    if (nstr) {
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own list
+        float4 f = skipped_terms<NQ>(s_list[wave], nstr, 0, 256 / P, psc, n_head, h, P, L, mx, inv,
+                                     (d0 + (D / 4) * wave) / 4, vrow, s_queue[wave], lane);
+#pragma unroll
+        for (int o = NQ; o < 64; o <<= 1) {
+            f.x = f.x + __shfl_xor(f.x, o);
+            f.y = f.y + __shfl_xor(f.y, o);
+            f.z = f.z + __shfl_xor(f.z, o);
+            f.w = f.w + __shfl_xor(f.w, o);
+        }
+        x = make_float4(x.x - f.x, x.y - f.y, x.z - f.z, x.w - f.w);
+    }
+    if (sg == 0) *reinterpret_cast<float4 *>(out + (size_t)h * HD + d) = x;
 }
 
-template <int HD, bool ROWS>
-__global__ __launch_bounds__(256) void attn_merge_kernel(const int32_t *len_dev, float *pm0, float *pl0, float *pmin0,
+template <int HD, bool ROWS, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_merge_kernel(const int32_t *len_dev, float *pm0, float *pl0, float *pmin0,
                                                          float *pacc0, int L0, unsigned pn, unsigned hg,
                                                          AttnArgs a) {
     const int len_raw = len_dev ? *len_dev : 0;
@@ -954,9 +1023,13 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const int32_t *len_dev,
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               V, (unsigned)(((size_t)t * a.vstride + voff + 4 * d4) * 4), 0, 0));
     };
-    if (ns <= merge_fast_max(HD) && merge_head_fast<HD, HD>(a.pm, a.pl, a.pmin, a.pacc, ns, a.n_head, h, 0, a.out))
+    if (merge_takes_fast(HD, ns, a.P)) {
+        if (threadIdx.x < 256)  // no barrier in it
+            merge_head_fast<HD, HD>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
         return;
-    merge_head<HD, HD>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
+    }
+    if constexpr (NW > 4)  // (the host knows the most splits there can be)
+        merge_head<HD, HD, NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
 }
 
 // A prompt's pass (Rows::Following, run_rows llama.rs:258-271): n rows at
@@ -1313,9 +1386,16 @@ int run(kh_ctx *ctx, const AttnArgs &a, int head_dim, int nb = 1) {
         const unsigned pn = (unsigned)a.P | (a.plus_one ? 1u << 31 : 0u);
         const unsigned hg = (unsigned)a.n_head | (unsigned)a.group << 16;
         const bool rows = a.rows || a.n_head > 0xffff || a.group > 0xffff;
-#define KH_MERGE(HH, RW)                                                                                           \
-    hipLaunchKernelGGL((attn_merge_kernel<HH, RW>), mg, dim3(256), 0, ctx->stream, a.len_dev, a.pm, a.pl, a.pmin, \
-                       a.pacc, a.L, pn, hg, a)
+        const bool wide = !merge_takes_fast(head_dim, a.nsplit, a.P);
+#define KH_MERGE(HH, RW)                                                                                       \
+    do {                                                                                                       \
+        if (wide)                                                                                              \
+            hipLaunchKernelGGL((attn_merge_kernel<HH, RW, WIDE_NW>), mg, dim3(64 * WIDE_NW), 0, ctx->stream, a.len_dev,     \
+                               a.pm, a.pl, a.pmin, a.pacc, a.L, pn, hg, a);                                    \
+        else                                                                                                   \
+            hipLaunchKernelGGL((attn_merge_kernel<HH, RW, 4>), mg, dim3(256), 0, ctx->stream, a.len_dev, a.pm, \
+                               a.pl, a.pmin, a.pacc, a.L, pn, hg, a);                                          \
+    } while (0)
         if (head_dim == 64) {
             if (rows) KH_MERGE(64, true);
             else KH_MERGE(64, false);
@@ -1765,19 +1845,21 @@ __global__ __launch_bounds__(64 * NW) void mla_split_kernel(MlaArgs a) {
 }
 
 // Merge, one workgroup per head and 128 dims (merge_head): the value row of position t is c_t.
-template <int D>
-__global__ __launch_bounds__(256) void mla_merge_kernel(MlaArgs a) {
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW) void mla_merge_kernel(MlaArgs a) {
     const int h = blockIdx.x;
     const rsrc_t C = rsrc(a.c, (size_t)a.L * a.cstride * 4);
     auto vrow = [&](int t, int d4) {
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               C, (unsigned)(((size_t)t * a.cstride + 4 * d4) * 4), 0, 0));
     };
-    if (a.nsplit <= merge_fast_max(D) &&
-        merge_head_fast<MLA_LAT, D>(a.pm, a.pl, a.pmin, a.pacc, a.nsplit, a.n_head, h, D * blockIdx.y, a.out))
-        return;
-    merge_head<MLA_LAT, D>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
-                           vrow, a.out);
+    // (the host knows the splits: four waves are the fast path's launch)
+    if constexpr (NW == 4)
+        merge_head_fast<MLA_LAT, D>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
+                                    vrow, a.out);
+    else
+        merge_head<MLA_LAT, D, NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
+                                   vrow, a.out);
 }
 
 }  // namespace
@@ -1824,12 +1906,18 @@ int launch_mla(kh_ctx *ctx, int n_head, const float *q_lat, const float *q_pe, c
     KH_HIP(hipGetLastError());
     if (a.nsplit > 1) {
         const int fd = mla_merge_dims(a.nsplit);
-        if (fd == 32)
-            hipLaunchKernelGGL((mla_merge_kernel<32>), dim3(n_head, MLA_LAT / 32), dim3(256), 0, ctx->stream, a);
-        else if (fd == 64)
-            hipLaunchKernelGGL((mla_merge_kernel<64>), dim3(n_head, MLA_LAT / 64), dim3(256), 0, ctx->stream, a);
-        else
-            hipLaunchKernelGGL((mla_merge_kernel<128>), dim3(n_head, MLA_LAT / 128), dim3(256), 0, ctx->stream, a);
+        const bool wide = !merge_takes_fast(fd, a.nsplit, a.P);
+#define KH_MERGE(D)                                                                                                   \
+    do {                                                                                                              \
+        if (wide)                                                                                                     \
+            hipLaunchKernelGGL((mla_merge_kernel<D, WIDE_NW>), dim3(n_head, MLA_LAT / D), dim3(64 * WIDE_NW), 0, ctx->stream, a);  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((mla_merge_kernel<D, 4>), dim3(n_head, MLA_LAT / D), dim3(256), 0, ctx->stream, a);    \
+    } while (0)
+        if (fd == 32) KH_MERGE(32);
+        else if (fd == 64) KH_MERGE(64);
+        else KH_MERGE(128);
+#undef KH_MERGE
         KH_HIP(hipGetLastError());
     }
     return KH_OK;

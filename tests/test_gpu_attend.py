@@ -200,3 +200,31 @@ def test_attend_skip_across_many_splits(ctx, monkeypatch, n_head, n_kv, L, mode)
     got = K.attend(ctx, spec, q.ravel(), cache, 0, L)
     want = O.attend(n_head, n_kv, 64, q.ravel(), k.ravel(), v.ravel(), L)
     close(got, want)
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,L", [(8, 2, 128, 500), (8, 2, 128, 8192), (32, 8, 128, 20000),
+                                              (14, 2, 64, 9000), (14, 2, 64, 33000)])
+@pytest.mark.parametrize("spread", ["few", "half"])
+def test_merge_takes_back_skipped_terms(ctx, n_head, n_kv, hd, L, spread):
+    # The merge's two forms (up to 128 splits of at most 128 positions, else
+    # shared by eight waves) with one straddling split in a few and a skipped
+    # position or two in each, and with half the positions skipped (the queue
+    # of skipped positions filling many times).
+    say("merge skipped terms", n_head, n_kv, hd, L, spread)
+    spec = K.Spec(n_head, n_kv, hd)
+    kvd = n_kv * hd
+    rng = np.random.default_rng(L + hd)
+    q = np.zeros((n_head, hd), np.float32)
+    q[:, 0] = np.sqrt(hd)  # score_t = k_t[0] of the head's KV head
+    k = np.zeros((L, kvd), np.float32)
+    for h in range(n_kv):
+        if spread == "few":
+            k[:, hd * h] = 2.0 * rng.standard_normal(L)
+        else:
+            k[:, hd * h] = rng.uniform(0.0, 11.0, L)
+            k[rng.choice(L, 3, replace=False), hd * h] = 24.0
+    v = (rng.standard_normal((L, kvd)) * 100.0).astype(np.float32)
+    cache = K.KvCache(ctx, 1, kvd, kvd)
+    cache.push(0, k.ravel(), v.ravel())
+    got = K.attend(ctx, spec, q.ravel(), cache, 0, L)
+    close(got, O.attend(n_head, n_kv, hd, q.ravel(), k.ravel(), v.ravel(), L))
