@@ -308,6 +308,12 @@ int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, co
 int launch_matmul_q(kh_ctx *ctx, const kh_weight *w, const QAct &q, size_t m, const float *bias, float *y,
                     int accumulate = 0);
 
+// Up to three weights of one precision and width over the same quantised rows
+// in one GEMM launch: y[i] = x W_i^T (+ bias[i]).  KH_DECLINED where the
+// operands are past its 32-bit offsets.
+int launch_matmul_jobs(kh_ctx *ctx, int k, const kh_weight *const *w, const QAct &q, size_t m,
+                       const float *const *bias, float *const *y);
+
 // GEMM over activations already quantised (QActBatch form), optionally
 // grouped by expert: with `tiles` set, workgroup row y of the grid takes tile
 // tiles[1 + 3y .. 3 + 3y] = (expert, first row, rows) of tiles[0] tiles, its
@@ -333,15 +339,16 @@ struct GemmArgs {
     // the splits in order, then bias and residual
     int ksplit;
     float *part;
-    // a second weight of the same shape over the same activations (gate and
-    // up): when y2 is set the grid holds both weights' row tiles, the first
-    // weight's then the second's, and the second writes y2 (split-K partials
-    // of the second take the plane after the first's)
-    const void *w2;
-    const float *ws2;
+    // a second and a third weight of the same width and precision over the
+    // same activations (gate and up; q, k and v): where y2 (y3) is set the grid
+    // holds their row tiles after the first weight's, and split-K partials of
+    // theirs take the planes after the first's
+    const void *w2, *w3;
+    const float *ws2, *ws3, *bias2, *bias3;
+    int N2, N3;
     const void *const *wtab2;
     const float *const *wstab2;
-    float *y2;
+    float *y2, *y3;
 };
 // tile_n: weight rows per tile (128, or 64 with 64-token tiles, ungrouped)
 int launch_gemm_q(kh_ctx *ctx, int precision, const GemmArgs &a, int max_tiles, int tile_m, int tile_n = 128);

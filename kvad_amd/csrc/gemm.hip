@@ -264,14 +264,21 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_kernel(GemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr0 = (wave / WT) * RT * 32, wm0 = (wave % WT) * TT * 32;
     const int K = a.K, nb = K / BLOCK;
-    // a paired launch: row tiles past the first weight's are the second's
-    const int nx = (a.N + BN - 1) / BN;
-    const bool second = a.y2 && (int)blockIdx.x >= nx;
-    const int n0 = ((int)blockIdx.x - (second ? nx : 0)) * BN;
-    if (second) {
-        a.w = a.w2, a.ws = a.ws2, a.wtab = a.wtab2, a.wstab = a.wstab2, a.y = a.y2;
-        if (a.ksplit > 1) a.part += (size_t)a.ksplit * a.M * a.N;
+    // row tiles past the first weight's are the second's, then the third's
+    int bx = (int)blockIdx.x;
+    if (a.y2) {
+        const int nx = (a.N + BN - 1) / BN, nx2 = (a.N2 + BN - 1) / BN;
+        const size_t planes = a.ksplit > 1 ? (size_t)a.ksplit * a.M : 0;
+        if (bx >= nx + nx2) {
+            bx -= nx + nx2, a.part += planes * (size_t)(a.N + a.N2);
+            a.w = a.w3, a.ws = a.ws3, a.bias = a.bias3, a.y = a.y3, a.N = a.N3;
+        } else if (bx >= nx) {
+            bx -= nx, a.part += planes * (size_t)a.N;
+            a.w = a.w2, a.ws = a.ws2, a.bias = a.bias2, a.y = a.y2, a.N = a.N2;
+            a.wtab = a.wtab2, a.wstab = a.wstab2;
+        }
     }
+    const int n0 = bx * BN;
 
     // the workgroup's rows of activations (and, grouped, its expert)
     int m0, m_end;
@@ -688,19 +695,19 @@ Shape pick_shape(int M, int N, int cu) {
     if (forced == 6464) return T64x64;
     if (forced == 128 || forced == 64 || forced == 32) return forced == 128 ? T128x128 : forced == 64 ? T128x64 : T128x32;
     const long long nt = (N + 127) / 128;
-    // 128 x 128 tiles while they give four workgroups per CU; below that,
-    // from 128 tokens, 64 x 64 tiles while they give one per two CUs (more,
-    // smaller workgroups hide the k-stages' load latency: (512, 896, 4864)
-    // 31.0 -> 28.3 us, (1024, 896, 4864) 45.0 -> 41.2, (512, 2048, 1408)
-    // 32.6 -> 31.0; at (2048, 4096, 14336) they lose, 461 -> 597, and at 16
-    // tokens over 14336x4096 29 -> 45 against 32-token tiles split over k)
+    // 128 x 128 tiles while they give four workgroups per CU; below that, past
+    // 64 tokens, 64 x 64 tiles: more, smaller workgroups hide the k-stages' load
+    // latency ((512, 896, 4864) 28.5 -> 27.4 us against 128-row 32-token tiles,
+    // (512, 4864, 896) 19.1 -> 17.8, (128, 896, 896) 10.9 -> 10.3, all split alike;
+    // at (2048, 4096, 14336) they lose, 461 -> 597, and at 16 tokens over
+    // 14336x4096 29 -> 45 against 32-token tiles split over k).
     // Token tiles no wider than the tokens need: a tall matrix at 16 or 32
     // tokens (a vocabulary head) gives enough workgroups with 32-token
     // tiles, and 128-token ones would leave three quarters of every tile idle.
     if (M > 64 && nt * ((M + 127) / 128) >= 4LL * cu) return T128x128;
-    if (M >= 128 && (long long)((N + 63) / 64) * ((M + 63) / 64) >= cu / 2) return T64x64;
-    if (M > 64 && nt * ((M + 127) / 128) >= cu) return T128x128;
-    if (M > 32 && nt * ((M + 63) / 64) >= cu) return T128x64;
+    if (M > 64 && M < 128 && nt >= cu) return T128x128;
+    if (M > 64) return T64x64;
+    if (M > 32 && nt >= cu) return T128x64;
     return T128x32;
 }
 
@@ -714,9 +721,16 @@ int gemm_tiles(kh_ctx *ctx, int M, int N, int *tile_n) {
 
 namespace {
 
+// Rows of every weight of a launch, and their tiles.
+long long all_rows(const GemmArgs &a) { return (long long)a.N + (a.y2 ? a.N2 : 0) + (a.y3 ? a.N3 : 0); }
+long long row_tiles(const GemmArgs &a, int tile_n) {
+    auto tiles = [&](int n) { return ((long long)n + tile_n - 1) / tile_n; };
+    return tiles(a.N) + (a.y2 ? tiles(a.N2) : 0) + (a.y3 ? tiles(a.N3) : 0);
+}
+
 template <int PREC>
 int launch_i8(kh_ctx *ctx, const GemmArgs &a, int max_tiles, int tile_m, int tile_n) {
-    const unsigned gx = (unsigned)((a.N + tile_n - 1) / tile_n) * (a.y2 ? 2u : 1u);
+    const unsigned gx = (unsigned)row_tiles(a, tile_n);
     const unsigned gy = a.tiles ? (unsigned)max_tiles : (unsigned)((a.M + tile_m - 1) / tile_m);
     if (gy == 0) return KH_OK;
     const dim3 grid(gx, gy, a.ksplit > 1 ? (unsigned)a.ksplit : 1u);
@@ -736,15 +750,14 @@ int launch_i8(kh_ctx *ctx, const GemmArgs &a, int max_tiles, int tile_m, int til
     }
     KH_HIP(hipGetLastError());
     if (a.ksplit > 1) {
-        const size_t quads = ((size_t)a.M * a.N + 3) / 4;
-        hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, ctx->stream,
-                           a.part, a.ksplit, a.M, a.N, a.bias, a.accumulate, a.y);
-        KH_HIP(hipGetLastError());
-        if (a.y2) {  // the second weight's splits, in the plane after the first's
-            hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
-                               ctx->stream, a.part + (size_t)a.ksplit * a.M * a.N, a.ksplit, a.M, a.N, a.bias,
-                               a.accumulate, a.y2);
-            KH_HIP(hipGetLastError());
+        const int ns[3] = {a.N, a.y2 ? a.N2 : 0, a.y3 ? a.N3 : 0};
+        const float *bias[3] = {a.bias, a.bias2, a.bias3};
+        float *y[3] = {a.y, a.y2, a.y3};
+        const float *part = a.part;
+        for (int i = 0; i < 3 && ns[i]; i++) {
+            const int rc = launch_split_reduce(ctx, part, a.ksplit, a.M, ns[i], bias[i], a.accumulate, y[i]);
+            if (rc) return rc;
+            part += (size_t)a.ksplit * a.M * ns[i];
         }
     }
     return KH_OK;
@@ -849,20 +862,24 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
 namespace {
 
 // Sets a's split-K fields: the k-stages (`stages` of them, at least `min_st`
-// a split) are split so that the grid comes to about SPLIT_PER_CU workgroups
-// per CU (a CU holds several: one's loads wait while another's MFMAs run), at
-// most SPLIT_MAX splits, and partials (4 M N bytes a split, written and read
-// again) of at most the weights' wbytes or 4 MiB, whichever is more (a small
-// weight such as a router's 64 rows would otherwise never split: 512 tokens x
-// 64 x 2048, 16 workgroups, 22.6 us unsplit).
-int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st, size_t wbytes) {
+// a split, none under `least`) are split so that the grid comes to about
+// SPLIT_PER_CU workgroups per CU (a CU holds several: one's loads wait while
+// another's MFMAs run), at most SPLIT_MAX splits, and partials (4 M N bytes a
+// split, written and read again) of at most the weights' wbytes or 4 MiB,
+// whichever is more (a small weight such as a router's 64 rows would otherwise
+// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); twice
+// that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
+// 4096) 36.3 -> 27.5 us in four splits instead of two, (512, 896, 4864) 27.5 ->
+// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two).
+int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st, int least, size_t wbytes) {
     a.ksplit = 0;
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const size_t plane = (size_t)a.M * a.N * 4 * (a.y2 ? 2 : 1);
-    long long ks = ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
+    const size_t plane = (size_t)a.M * all_rows(a) * 4;
+    const size_t most = std::max(wbytes, (size_t)4 << 20) * (2 * tiles <= cu ? 2 : 1);
+    long long ks = stages < least ? 1 : ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
     ks = std::min<long long>(ks, stages / min_st);
     ks = std::min<long long>(ks, SPLIT_MAX);
-    ks = std::min<long long>(ks, (long long)(std::max(wbytes, (size_t)4 << 20) / plane));
+    ks = std::min<long long>(ks, (long long)(most / plane));
     const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
     if (forced > 0) ks = std::min(forced, stages);
     ks = std::min<long long>(ks, (long long)(SPLIT_BYTES / plane));
@@ -887,7 +904,7 @@ int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st,
 // 126 -> 11.5; 512x512 at 16 15.7 -> 6.9 (at least four stages 8.5, eight 11.7).
 int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
     const long long tiles = (long long)((a.N + 127) / 128) * ((a.M + tile_m - 1) / tile_m);
-    return set_split(ctx, a, tiles, (a.K + FK - 1) / FK, 2, (size_t)a.N * a.K * 4);
+    return set_split(ctx, a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4);
 }
 
 }  // namespace
@@ -895,10 +912,11 @@ int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
 int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
     a.ksplit = 0;
     if (a.tiles) return KH_OK;  // grouped launches are not split
-    // a paired launch (a.y2) holds both weights' tiles and partial planes
-    const int pair = a.y2 ? 2 : 1;
-    const long long tiles = (long long)((a.N + tile_n - 1) / tile_n) * ((a.M + tile_m - 1) / tile_m) * pair;
-    return set_split(ctx, a, tiles, (a.K + BK - 1) / BK, SPLIT_MIN_STAGES, (size_t)a.N * a.K * pair);
+    // Under twelve stages of 128 the second launch costs more than the shorter
+    // chains save: (512 tokens, 896 rows, 896) 14.1 us in two splits, 11.2
+    // unsplit, (80, 4864, 896) 14.0 and 10.9.
+    return set_split(ctx, a, row_tiles(a, tile_n) * ((a.M + tile_m - 1) / tile_m), (a.K + BK - 1) / BK,
+                     SPLIT_MIN_STAGES, 12, (size_t)all_rows(a) * a.K);
 }
 
 int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y,
@@ -978,6 +996,32 @@ int launch_gemm_q(kh_ctx *ctx, int precision, const GemmArgs &a, int max_tiles, 
         case KH_Q4K: return launch_i8<KH_Q4K>(ctx, a, max_tiles, tile_m, tile_n);
         default: return fail(KH_EINVAL, "gemm: the grouped kernel takes quantised weights");
     }
+}
+
+int launch_matmul_jobs(kh_ctx *ctx, int k, const kh_weight *const *w, const QAct &q, size_t m,
+                       const float *const *bias, float *const *y) {
+    if (k < 2 || k > 3) return fail(KH_EINVAL, "matmul: two or three weights per launch");
+    const size_t cols = w[0]->cols;
+    size_t rows = 0;
+    for (int i = 0; i < k; i++) {
+        if (w[i]->precision == KH_F32 || w[i]->precision != w[0]->precision || w[i]->cols != cols)
+            return fail(KH_EINVAL, "matmul: weights of one launch share a quantised precision and width");
+        if (w[i]->rows * cols + 4 * 128 * cols >= 0xffffffffull)
+            return fail(KH_DECLINED, "matmul: operands of 4 GiB or more are not addressed here");
+        rows += w[i]->rows;
+    }
+    if (m * cols + 4 * 128 * cols >= 0xffffffffull || rows > 0x7fffffff || m > 0x7fffffff)
+        return fail(KH_DECLINED, "matmul: operands of 4 GiB or more are not addressed here");
+    GemmArgs a{};
+    a.M = (int)m, a.K = (int)cols;
+    a.xq = q.qs, a.xs = q.scales, a.xsum = q.sums;
+    a.w = w[0]->qs, a.ws = w[0]->scales, a.bias = bias[0], a.y = y[0], a.N = (int)w[0]->rows;
+    a.w2 = w[1]->qs, a.ws2 = w[1]->scales, a.bias2 = bias[1], a.y2 = y[1], a.N2 = (int)w[1]->rows;
+    if (k == 3) a.w3 = w[2]->qs, a.ws3 = w[2]->scales, a.bias3 = bias[2], a.y3 = y[2], a.N3 = (int)w[2]->rows;
+    int tn;
+    const int tm = gemm_tiles(ctx, a.M, (int)rows, &tn);
+    const int rc = plan_split(ctx, a, tm, tn);
+    return rc ? rc : launch_gemm_q(ctx, w[0]->precision, a, 0, tm, tn);
 }
 
 }  // namespace kh

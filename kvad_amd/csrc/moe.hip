@@ -447,7 +447,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     a.w = gate->qs, a.ws = gate->scales, a.N = (int)gate->rows, a.y = g;
     if (gate->precision == up->precision && gate->rows == up->rows && gate->cols == up->cols) {
         // gate and up in one launch over the same activation tiles
-        a.w2 = up->qs, a.ws2 = up->scales, a.y2 = u;
+        a.w2 = up->qs, a.ws2 = up->scales, a.y2 = u, a.N2 = a.N;
         if ((rc = plan_split(ctx, a, tm, tn)) || (rc = launch_gemm_q(ctx, gate->precision, a, 0, tm, tn))) return rc;
     } else {
         if ((rc = plan_split(ctx, a, tm, tn)) || (rc = launch_gemm_q(ctx, gate->precision, a, 0, tm, tn))) return rc;
@@ -581,7 +581,7 @@ int moe_prefill(kh_ctx *ctx, kh_moe *moe, const float *hs, size_t m, float *out)
     // and up in the same launch (the second weight table)
     a.wtab2 = const_cast<const void *const *>(moe->tab + n);
     a.wstab2 = const_cast<const float *const *>(moe->stab + n);
-    a.y2 = u;
+    a.y2 = u, a.N2 = a.N;
     if ((rc = launch_gemm_q(ctx, moe->precision, a, (int)max_tiles, tile_m))) return rc;
     if ((rc = launch_swiglu_qact(ctx, g, u, total, inter, rq))) return rc;
     // each expert's down over its rows of swiglu(gate, up)

@@ -482,10 +482,8 @@ int ensure_pass(kh_llm *m, size_t n, size_t max_len) {
 // ones from the rows' codes in qa (matmul_bt, quant.rs:751; tensor.rs:102);
 // with accumulate the product is added into y (the residual add).
 // Projections of the same input (q/k/v, gate/up) take one multi-token GEMV
-// launch up to this many rows (the weights stream once per launch; the GEMM
-// would take a launch per weight, and at decode's small matrices its
-// 128-row tiles leave most CUs idle).  A single projection (o, down, the
-// head) follows kh_matmul's rule.
+// launch up to this many rows.  A single projection (o, down, the head)
+// follows kh_matmul's rule.
 size_t rows_multi_max() {
     static const size_t v = (size_t)env_int("KVAD_ROWS_MULTI", 64);  // tuning knob
     return v;
@@ -505,14 +503,21 @@ bool any_f32(std::initializer_list<const kh_weight *> ws) {
     return false;
 }
 
-// Projections of the same input: one multi-token launch when they are all
-// quantised alike and the rows are few, else one projection at a time.
+// Projections of the same input, all quantised alike, in one launch: the
+// multi-token GEMV while the rows are few, else the GEMM over all their row
+// tiles (k and v alone are four 64-row tiles of a 896-wide model: q, k and v of
+// a 512-token pass 8.2 + 5.9 + 5.9 us and a reduction of 4-5 each -> one launch
+// of 7); else one projection at a time.
 int project_all(kh_ctx *ctx, int k, const kh_weight *const *w, const float *xs, const QAct &qa, size_t n,
                 const float *const *bias, float *const *y) {
-    bool one = n <= rows_multi_max();
+    bool one = true;
     for (int i = 0; i < k; i++)
         one = one && w[i]->precision != KH_F32 && w[i]->precision == w[0]->precision && w[i]->cols == w[0]->cols;
-    if (one) return launch_gemv_multi_jobs(ctx, k, w, bias, y, nullptr, qa, n);
+    if (one && n <= rows_multi_max()) return launch_gemv_multi_jobs(ctx, k, w, bias, y, nullptr, qa, n);
+    if (one) {
+        const int rc = launch_matmul_jobs(ctx, k, w, qa, n, bias, y);
+        if (rc != KH_DECLINED) return rc;
+    }
     for (int i = 0; i < k; i++) {
         int rc = project(ctx, w[i], xs, qa, n, bias[i], y[i]);
         if (rc) return rc;
