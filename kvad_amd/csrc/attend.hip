@@ -1040,13 +1040,19 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(const int32_t *len_
 // them, wave w taking the 16-position tiles w, w + NW, ..., on the matrix
 // cores in the split kernel's layouts (v_mfma_f32_16x16x4f32: S = K Q^T
 // lands as lane (c, j) holding positions 4c .. 4c + 3 of column j; O += P V
-// with V rows 4c + r).  Two passes over the positions: the column's maximum
-// M and sum S = sum e^{s - M} (per wave a running maximum with the sum
-// rescaled when it rises; the waves' (M, S) combined in LDS in wave order),
-// then the reference's weights w = e^{s - M} * (1/S), w < 1e-8 dropped
-// (mod.rs:805-812), times the values, the waves' sums added in LDS in wave
-// order.  Every column's whole sequence is in one workgroup: no partials in
-// memory and no merge launch.  Scores are dot(q, k) * scale (mod.rs:802).
+// with V rows 4c + r).  One pass over the positions: e^{s - R} against a
+// reference R near the column's maximum and their products with the values,
+// the column's smallest score kept beside them; the waves' (R, S) and sums
+// meet in LDS in wave order.  Where the smallest weight of some column is under
+// the reference's 1e-8 line (mod.rs:807) the workgroup goes over the positions
+// twice more, for M and S = sum e^{s - M} and then the weights themselves,
+// w = e^{s - M} * (1/S), w < 1e-8 dropped, times the values (normal scores
+// spread by 2: four columns in a thousand at 1500 positions).  Every column's
+// whole sequence is in one workgroup: no partials in memory and no merge launch.  Scores are
+// dot(q, k) * scale (mod.rs:802).  Bound by the matrix cores' f32 rate and the
+// exponentials between its products: over
+// 512 rows of 14 heads of 64 at 1000 positions and 476 at 1500 the two passes
+// alone took 43 and 60 us, the one pass 28 and 40.
 struct PassArgs {
     const float *q;        // [n][n_head][HD]
     const AttnRow *rows;   // [n]: the cache (the same for every row) and each row's length
@@ -1110,10 +1116,126 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
             s[r] = t0 + 4 * c4 + r <= last ? sc : -INFINITY;
         }
     };
-    // Both passes keep the wave's next tile in flight while one is worked
+    // Every pass keeps the wave's next tile in flight while one is worked
     // (tiles past L read zeros: the buffers' range ends at L).
+    f4v acc[NT];
+#pragma unroll
+    for (int q = 0; q < NT; q++) acc[q] = f4v{0.f, 0.f, 0.f, 0.f};
+    __shared__ float s_on[3][NW][16];                    // each wave's reference, sum, smallest score
+    __shared__ __align__(16) float s_acc[NW][16][HD];    // the waves' sums
+    __shared__ float s_f[NW][16];
+    // One pass: e^{s - R} against a reference R, the first tile's maximum,
+    // raised (and the sums rescaled) only when a score passes it by 8, which
+    // few sequences do again: no maximum across lanes per tile.
+    {
+        float R = 0.0f, S = 0.0f, mn = INFINITY;
+        bool started = false;  // R is a score of the column's
+        auto online = [&](int t0, const f4v (&kq)[NQ4], const f4v (&vv)[4][VT]) {
+            float s[4];
+            scores(t0, kq, s);
+            const float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+            if (__builtin_amdgcn_ballot_w64(mx > (started ? R + 8.0f : -INFINITY))) {
+                const float m = rows_max(mx);  // the column's, in all its lanes
+                const bool up = m > (started ? R + 8.0f : -INFINITY);
+                const float c = up && started ? expf(R - m) : 1.0f;  // sums are zero before the start
+                R = up ? m : R;
+                started = started || up;
+                S = S * c;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float ci = __shfl(c, 4 * c4 + i);  // of column 4 c4 + i
+#pragma unroll
+                    for (int q = 0; q < NT; q++) acc[q][i] = acc[q][i] * ci;
+                }
+            }
+            float p[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[r] = expf(s[r] - R);  // 0 where masked: R is finite
+                S += p[r];
+                mn = s[r] == -INFINITY ? mn : fminf(mn, s[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int q = 0; q < NT; q++)
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], vv[r][q >> 2][q & 3], acc[q], 0, 0, 0);
+        };
+        f4v ka[NQ4], kb[NQ4], va[4][VT], vb[4][VT];
+        load_k(16 * wave, ka);
+        load_v(16 * wave, va);
+        for (int t0 = 16 * wave; t0 < L; t0 += 2 * STEP) {
+            load_k(t0 + STEP, kb);
+            load_v(t0 + STEP, vb);
+            online(t0, ka, va);
+            if (t0 + STEP >= L) break;
+            load_k(t0 + 2 * STEP, ka);
+            load_v(t0 + 2 * STEP, va);
+            online(t0 + STEP, kb, vb);
+        }
+        S = rows_sum(S);
+        mn = rows_min(mn);
+        if (c4 == 0) {
+            s_on[0][wave][j16] = started ? R : -INFINITY;
+            s_on[1][wave][j16] = S;
+            s_on[2][wave][j16] = mn;
+        }
+    }
+    // acc[q][i] is column 4 c4 + i, dim 4 j16 + (q & 3) + 64 (q >> 2)
+    auto store_acc = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int v = 0; v < VT; v++)
+                *reinterpret_cast<float4 *>(&s_acc[wave][4 * c4 + i][64 * v + 4 * j16]) =
+                    make_float4(acc[4 * v][i], acc[4 * v + 1][i], acc[4 * v + 2][i], acc[4 * v + 3][i]);
+    };
+    // out = the waves' sums, wave w's times s_f[w], in wave order
+    auto finish = [&]() {
+        __syncthreads();
+        for (int i = tid; i < 16 * HD / 4; i += 64 * NW) {
+            const int col = i / (HD / 4), d = 4 * (i % (HD / 4)), row = r0 + col / gc, head = h0 + col % gc;
+            if (col >= rpt * gc || row >= a.n) continue;
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const float4 y = *reinterpret_cast<const float4 *>(&s_acc[w][col][d]);
+                const float f = s_f[w][col];
+                x = make_float4(fmaf(y.x, f, x.x), fmaf(y.y, f, x.y), fmaf(y.z, f, x.z), fmaf(y.w, f, x.w));
+            }
+            *reinterpret_cast<float4 *>(a.out + ((size_t)row * a.n_head + head) * HD + d) = x;
+        }
+    };
+    store_acc();
+    __syncthreads();
+    float M = -INFINITY, S = 0.0f;  // the column's, over the waves in order
+    {
+        float mn = INFINITY;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            M = fmaxf(M, s_on[0][w][j16]);
+            mn = fminf(mn, s_on[2][w][j16]);
+        }
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float rw = s_on[0][w][j16];
+            S = rw == -INFINITY ? S : fmaf(s_on[1][w][j16], expf(rw - M), S);
+        }
+        const float inv = 1.0f / S;
+        // the smallest weight kept: the same in every wave
+        const bool skips = hv && expf(mn - M) * inv < 1e-8f;
+        if (!__builtin_amdgcn_ballot_w64(skips)) {
+            if (c4 == 0) {
+                const float rw = s_on[0][wave][j16];
+                s_f[wave][j16] = rw == -INFINITY ? 0.0f : expf(rw - M) * inv;
+            }
+            finish();
+            return;
+        }
+    }
+    // Some column has weights the reference drops: its own two passes.
     // pass 1: the maximum M and the sum of e^{s - M}
-    float M = -INFINITY, S = 0.0f;
+    M = -INFINITY, S = 0.0f;
     auto stats = [&](int t0, const f4v (&kq)[NQ4]) {
         float s[4];
         scores(t0, kq, s);
@@ -1156,7 +1278,6 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
     }
     const float inv = 1.0f / S;  // inv = 1 / sum, tensor.rs:304
     // pass 2: the weights times the values
-    f4v acc[NT];
 #pragma unroll
     for (int q = 0; q < NT; q++) acc[q] = f4v{0.f, 0.f, 0.f, 0.f};
     auto accumulate = [&](int t0, const f4v (&kq)[NQ4], const f4v (&vv)[4][VT]) {
@@ -1188,39 +1309,10 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
             accumulate(t0 + STEP, kb, vb);
         }
     }
-    // acc[q][i] is column 4 c4 + i, dim 4 j16 + (q & 3) + 64 (q >> 2)
-    if constexpr (NW == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int col = 4 * c4 + i, row = r0 + col / gc, head = h0 + col % gc;
-            if (col >= rpt * gc || row >= a.n) continue;
-            float *o = a.out + ((size_t)row * a.n_head + head) * HD;
-#pragma unroll
-            for (int v = 0; v < VT; v++)
-                *reinterpret_cast<float4 *>(o + 64 * v + 4 * j16) =
-                    make_float4(acc[4 * v][i], acc[4 * v + 1][i], acc[4 * v + 2][i], acc[4 * v + 3][i]);
-        }
-    } else {  // the waves' sums, added in wave order
-        __shared__ __align__(16) float s_acc[NW][16][HD];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int v = 0; v < VT; v++)
-                *reinterpret_cast<float4 *>(&s_acc[wave][4 * c4 + i][64 * v + 4 * j16]) =
-                    make_float4(acc[4 * v][i], acc[4 * v + 1][i], acc[4 * v + 2][i], acc[4 * v + 3][i]);
-        __syncthreads();
-        for (int i = tid; i < 16 * HD / 4; i += 64 * NW) {
-            const int col = i / (HD / 4), d = 4 * (i % (HD / 4)), row = r0 + col / gc, head = h0 + col % gc;
-            if (col >= rpt * gc || row >= a.n) continue;
-            float4 x = *reinterpret_cast<const float4 *>(&s_acc[0][col][d]);
-#pragma unroll
-            for (int w = 1; w < NW; w++) {
-                const float4 y = *reinterpret_cast<const float4 *>(&s_acc[w][col][d]);
-                x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
-            }
-            *reinterpret_cast<float4 *>(a.out + ((size_t)row * a.n_head + head) * HD + d) = x;
-        }
-    }
+    if (c4 == 0) s_f[wave][j16] = 1.0f;
+    __syncthreads();  // s_acc's first use is over in every wave
+    store_acc();
+    finish();
 }
 
 // P = 16 R nw positions per workgroup of nw waves: four waves with R in

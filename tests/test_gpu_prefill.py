@@ -291,3 +291,39 @@ def test_each_stage_of_a_pass(ctx, monkeypatch, case):
     logits = proj(ref.head, s["vocab"], e, O.rms_norm(X[n - 1], ref.final_norm, eps))
     note("head", close(tr["logits"], logits, "head of the last row"))
     say("prefill stages worst", case, {k: f"{v:.1e}" for k, v in worst.items()})
+
+
+@pytest.mark.parametrize("variant,attn", [("qwen3_q8", "pass"), ("qwen3_q8", "pass:4"), ("qwen3_q8", "pass:8"),
+                                          ("qwen3_hd128_q8", "pass:2")])
+@pytest.mark.parametrize("spread", [1.0, 2.5, 6.0])
+def test_a_pass_over_widely_spread_scores(ctx, monkeypatch, variant, attn, spread):
+    # The query norms scaled so that scores spread by about `spread`: by 2.5 a
+    # later tile's maximum passes the first's by more than 8 now and then (the
+    # running sums are rescaled), by 6 weights fall under 1e-8 as well and the
+    # workgroup drops them as the reference does, in two passes of its own.
+    kw = dict(VARIANTS["qwen3_q8"], **({"n_head": 8, "n_kv_head": 2, "head_dim": 128, "n_embd": 256}
+                                       if variant == "qwen3_hd128_q8" else {}))
+    attention_path(monkeypatch, attn)
+    say("pass, spread scores", variant, attn, spread)
+    n = 150
+    m, mk = build(ctx, 360, n_layer=1, n_ctx=192, **kw)
+    ref = mk()
+    s, L = ref.s, ref.layers[0]
+    hd, nh, nkv, half, eps = s["head_dim"], s["n_head"], s["n_kv_head"], s["head_dim"] // 2, s["eps"]
+    qd, kvd = nh * hd, nkv * hd
+    L["q_norm"] = (np.asarray(L["q_norm"]) * spread).astype(np.float32)
+    m.set_layer(0, *m._keep[0], L["attn_norm"], L["mlp_norm"], L.get("q_b"), L.get("k_b"), L.get("v_b"), L["q_norm"],
+                L["k_norm"])
+    tr = m.trace_pass([(i * 29 + 7) % 512 for i in range(n)])
+    kc, vc, dropped = tr["k_cache"][0], tr["v_cache"][0], 0
+    for i in range(n):
+        q = tr["qkv"][0][i][:qd].copy()
+        for head in range(nh):
+            seg = O.rms_norm(q[head * hd:(head + 1) * hd], L["q_norm"], eps)
+            rope = O.rope_apply_interleaved if s.get("rope_interleaved") else O.rope_apply
+            q[head * hd:(head + 1) * hd] = rope(ref.cos, ref.sin, half, seg, i)
+            sc = kc[:i + 1].reshape(i + 1, nkv, hd)[:, head // (nh // nkv)] @ q[head * hd:(head + 1) * hd] / np.sqrt(hd)
+            dropped += int(np.sum(np.exp(sc - sc.max()) / np.sum(np.exp(sc - sc.max())) < 1e-8))
+        att = O.attend(nh, nkv, hd, q, kc[:i + 1].ravel(), vc[:i + 1].ravel(), i + 1)
+        close(tr["att"][0][i], att, f"row {i} attention")
+    assert dropped == 0 if spread == 1.0 else spread < 6.0 or dropped > 0, dropped
