@@ -615,7 +615,7 @@ __device__ __forceinline__ float block_reduce(float v, float *s_w, F op) {
 }
 
 constexpr int MAX_SPLITS = 4096;
-constexpr int WIDE_NW = 8;  // waves of a merge of more splits than merge_fast_max
+constexpr int WIDE_NW = 8;  // waves of a merge the fast path does not take
 
 // Exclusive prefix sum of one int per thread over the workgroup (NW waves);
 // *total gets the sum.  s holds NW ints and is free again on return.
@@ -888,35 +888,36 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
 // past 16 bits) takes them from the struct and the row table.  pn: P |
 // plus_one << 31; hg: n_head | group << 16.
 // The merge of dims d0 .. d0 + D of one head (rows of HD) without barriers,
-// for up to merge_fast_max(D) splits (128 for 64 or 128 dims): every
+// for up to MAXNS splits: every
 // load is issued at once (each wave reads every split's max, sum and
-// minimum, four splits a lane, and its quarter of the dims of every split's
+// minimum, MAXNS / 64 splits a lane, and its quarter of the dims of every split's
 // partial values, D / 16 float4s a lane-row of 64 / (D / 16) splits), the maximum and the sum are
 // wave butterflies (each wave computes the same ones, in the same order),
 // the weights e^{m_j - M} pass through the wave's own LDS row, and the
 // split groups' sums meet by butterfly.  The straddling splits' skipped terms
 // come after, each wave over all of them for its own dims (skipped_terms).
-// The most splits merge_head_fast takes for D dims: its partial values'
-// split groups and its statistics' four splits a lane both cover them, and
-// no more than 128 (past that merge_head's waves share the partials out).
-__host__ __device__ constexpr int merge_fast_max(int d) { return 16 * 64 / (d / 16) < 128 ? 16 * 64 / (d / 16) : 128; }
-// Splits of 256 positions leave to merge_head, too: over a cache that long
-// (16384 positions on) a third of them and more straddle, which its eight
-// waves share and the fast path's each go through (14 heads of 64 over 32768
-// positions, scores spread by 2: 53-70 us fast, 24 shared; without a
-// straddling split 13.4 and 13.7).  The host asks for a launch's most splits,
+// The most splits merge_head_fast takes: 128, or 256 for latent attention's
+// 64-dim slices (whose launches know their splits: a bound the compiler sees
+// in the code it serves, 7.0 -> 7.5 us per short layer where it was 256).
+// Splits of 256 positions, and more than 128 of more than 32, leave to
+// merge_head: over a cache that long a third of them and more straddle, which
+// its eight waves share and the fast path's each go through (14 heads of 64
+// over 32768 positions, scores spread by 2: 53-70 us fast, 24 shared; without
+// a straddling split 13.4 and 14.8).  The host asks for a launch's most splits,
 // the kernel for those of the length it finds.
-__host__ __device__ constexpr bool merge_takes_fast(int d, int ns, int P) {
-    return ns <= merge_fast_max(d) && P <= 128;
+__host__ __device__ constexpr bool merge_takes_fast(int maxns, int ns, int P) {
+    return ns <= maxns && P <= 128 && (ns <= 128 || P <= 32);
 }
-template <int HD, int D, typename VRow>
+constexpr int MERGE_NS = 128;                                              // grouped-query attention's
+__host__ __device__ constexpr int mla_merge_ns(int d) { return d <= 64 ? 256 : 128; }
+template <int HD, int D, int MAXNS, typename VRow>
 __device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl, const float *pmin, const float *pacc,
                                                 const float *psc, int ns, int n_head, int h, int d0, int P, int L,
                                                 VRow vrow, float *out) {
     constexpr int NQ = D / 16;      // float4s of a wave's dims
     constexpr int SG = 64 / NQ;     // split groups a wave-row holds
-    constexpr int PJ = 16;          // partial values a lane holds at most
-    constexpr int PS = 4;           // splits of statistics a lane holds
+    constexpr int PJ = (MAXNS + SG - 1) / SG;  // partial values a lane holds at most
+    constexpr int PS = MAXNS / 64;             // splits of statistics a lane holds
     __shared__ float s_c[4][PS * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int dq = lane % NQ, sg = lane / NQ;
@@ -1023,9 +1024,9 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(const int32_t *len_
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               V, (unsigned)(((size_t)t * a.vstride + voff + 4 * d4) * 4), 0, 0));
     };
-    if (merge_takes_fast(HD, ns, a.P)) {
+    if (merge_takes_fast(MERGE_NS, ns, a.P)) {
         if (threadIdx.x < 256)  // no barrier in it
-            merge_head_fast<HD, HD>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
+            merge_head_fast<HD, HD, MERGE_NS>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
         return;
     }
     if constexpr (NW > 4)  // (the host knows the most splits there can be)
@@ -1478,7 +1479,7 @@ int run(kh_ctx *ctx, const AttnArgs &a, int head_dim, int nb = 1) {
         const unsigned pn = (unsigned)a.P | (a.plus_one ? 1u << 31 : 0u);
         const unsigned hg = (unsigned)a.n_head | (unsigned)a.group << 16;
         const bool rows = a.rows || a.n_head > 0xffff || a.group > 0xffff;
-        const bool wide = !merge_takes_fast(head_dim, a.nsplit, a.P);
+        const bool wide = !merge_takes_fast(MERGE_NS, a.nsplit, a.P);
 #define KH_MERGE(HH, RW)                                                                                       \
     do {                                                                                                       \
         if (wide)                                                                                              \
@@ -1735,7 +1736,7 @@ namespace {
 
 constexpr int MLA_LAT = 512, MLA_ROPE = 64, MLA_K = MLA_LAT + MLA_ROPE;
 constexpr int MLA_QSTR = MLA_K + 4;  // LDS row stride (floats) of the staged queries
-constexpr int MLA_P = 64;            // positions per workgroup: one tile of 16 per wave
+constexpr int MLA_ONE = 32;          // the longest sequence taken in one launch
 // dims per merge workgroup: 128 (four per head) for a few splits, 64 from
 // 64 splits on, where each workgroup's partials are what it waits for
 // (measured at L = 1024 / 8192 / 32768: 18.9 / 24.6 / 44.2 us per layer at
@@ -1754,10 +1755,14 @@ struct MlaArgs {
     float scale;
     float *pm, *pl, *pmin, *pacc, *psc;  // per split: [nsplit][n_head]; acc [..][512]; scores [..][P]
     float *out;                    // [n_head][512]
-    int P;                         // positions per split: 16 per wave
+    int P;                         // positions per split
 };
 
-// Split kernel.  Wave w scores positions t0 + 16w .. +15 for the 16 heads:
+// A sequence of up to MLA_ONE positions in one launch (NW waves of 16
+// positions, so NW - 2 of them score rows past the end, as zeros, and take their
+// share of the value dims: 11.5 us against 12.1 on two waves):
+// the reference's weights in one launch.  Wave w scores positions
+// 16w .. + 15 for the 16 heads:
 // S = K' Q'^T on v_mfma_f32_16x16x4_f32 over 36 products of 16 dims (32 of
 // c, 4 of pe, so each reads one array); in product 4k + i k-slot c takes
 // dims 64k + 16i + 4c .. + 3, so one load instruction reads 64 contiguous
@@ -1767,21 +1772,20 @@ struct MlaArgs {
 // share it; the probabilities go to LDS and wave w then forms
 // O[heads][dims 128w .. 128w + 127] = P V over all 64 positions.
 template <int NW>
-__global__ __launch_bounds__(64 * NW) void mla_split_kernel(MlaArgs a) {
+__global__ __launch_bounds__(64 * NW) void mla_one_kernel(MlaArgs a) {
     constexpr int P = 16 * NW;       // positions: one tile of 16 per wave
     constexpr int DW = MLA_LAT / NW;  // value dims each wave forms
     constexpr int VG = DW / 64;       // 64-dim groups of them
-    const int split = blockIdx.x, h0 = blockIdx.y * 16;
+    const int h0 = blockIdx.y * 16;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j16 = lane & 15, c4 = lane >> 4;
     const int L = a.L;
-    const int t0 = split * P, n = min(L - t0, P);
-    const bool whole = a.nsplit == 1;
+    const int t0 = 0, n = min(L, P);
     const int H = min(a.n_head - h0, 16);
     __shared__ __align__(16) float sQ[16 * MLA_QSTR];
     __shared__ float sP[16][P + 4];
-    __shared__ float s_st[3][NW][16];
+    __shared__ float s_st[2][NW][16];
     const rsrc_t C = rsrc(a.c, (size_t)L * a.cstride * 4), PE = rsrc(a.pe, (size_t)L * a.pestride * 4);
 
     // the tile's key rows (the long-latency loads) first
@@ -1840,21 +1844,16 @@ __global__ __launch_bounds__(64 * NW) void mla_split_kernel(MlaArgs a) {
                 vv[u][r][v] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(C, off, 256 * v, 0));
         }
     __builtin_amdgcn_sched_barrier(0);
-    float s[4], mx = -INFINITY, mn = INFINITY;
+    float s[4], mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const bool ok = j16 < H && 16 * wave + 4 * c4 + r < n;
         const float sc = d[r] * a.scale;  // (dot(q_lat, c) + dot(q_pe, pe)) * scale, deepseek.rs:567-570
         s[r] = ok ? sc : -INFINITY;
         mx = fmaxf(mx, s[r]);
-        mn = ok ? fminf(mn, sc) : mn;
     }
     mx = rows_max(mx);
-    mn = rows_min(mn);
-    if (c4 == 0) {
-        s_st[0][wave][j16] = mx;
-        s_st[2][wave][j16] = mn;
-    }
+    if (c4 == 0) s_st[0][wave][j16] = mx;
     __syncthreads();
     auto wmax = [&](int st, int h) {
         float x = s_st[st][0][h];
@@ -1879,15 +1878,13 @@ __global__ __launch_bounds__(64 * NW) void mla_split_kernel(MlaArgs a) {
     if (c4 == 0) s_st[1][wave][j16] = l;
     __syncthreads();
     const float S = wsum(j16);
-    if (whole) {
-        // the reference's own weights: w = exp(s - M) * (1/S), dropping w < 1e-8
-        // (softmax_inplace, tensor.rs:297-308; deepseek.rs:576-579)
-        const float inv = 1.0f / S;
+    // the reference's own weights: w = exp(s - M) * (1/S), dropping w < 1e-8
+    // (softmax_inplace, tensor.rs:297-308; deepseek.rs:576-579)
+    const float inv = 1.0f / S;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float w = e[r] * inv;
-            e[r] = w < 1e-8f ? 0.0f : w;
-        }
+    for (int r = 0; r < 4; r++) {
+        const float w = e[r] * inv;
+        e[r] = w < 1e-8f ? 0.0f : w;
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) sP[j16][16 * wave + 4 * c4 + r] = e[r];
@@ -1914,26 +1911,161 @@ __global__ __launch_bounds__(64 * NW) void mla_split_kernel(MlaArgs a) {
     for (int i = 0; i < 4; i++) {
         const int h = 4 * c4 + i;
         if (h >= H) continue;
-        float *dst = whole ? a.out + (size_t)(h0 + h) * MLA_LAT
-                           : a.pacc + ((size_t)split * a.n_head + h0 + h) * MLA_LAT;
+        float *dst = a.out + (size_t)(h0 + h) * MLA_LAT;
 #pragma unroll
         for (int v = 0; v < VG; v++)
             *reinterpret_cast<float4 *>(dst + D0 + 64 * v + 4 * j16) =
                 make_float4(acc[4 * v][i], acc[4 * v + 1][i], acc[4 * v + 2][i], acc[4 * v + 3][i]);
     }
-    if (!whole && tid < H) {
-        const int h = tid;
-        const size_t o = (size_t)split * a.n_head + h0 + h;
-        a.pm[o] = wmax(0, h);
-        a.pl[o] = wsum(h);
-        float mnv = s_st[2][0][h];
+}
+
+// Split kernel: P = 32 R positions by eight waves, 32 at a time.  The tile's
+// latent rows come in coalesced, a tile ahead in registers, and lie in LDS (64
+// KB, rows 4 banks apart) for both uses, as keys and as values.  Scores: wave
+// (pg, dg) takes positions 16 pg .. + 15 over dims 128 dg .. + 127 of c and 16
+// dg .. + 15 of pe, the queries' share of those dims held in registers,
+// S = K' Q'^T on v_mfma_f32_16x16x4_f32; the four dim groups' sums meet in LDS,
+// and every wave reads them in the layout its value products want, so each
+// takes the maxima and exponentials of all 32 positions itself and no weight
+// passes through memory.  Values: wave w forms O[heads][dims 64 w .. + 63].
+// Between tiles the sums are rescaled to the running maximum.
+//
+// Bound by the f32 matrix cores (68 products of 32 cycles a wave and tile, two
+// waves a SIMD) and by the chain load - scores - exchange - values of the first
+// tile.  One wave per 16 positions over all 576 dims, which read the rows from
+// memory twice, had both chains four times as long: 16 heads over 1000 / 3000 / 6001 / 20000 /
+// 32768 positions (scores spread by 2, split and merge) 16.2 / 20.5 / 24.0 /
+// 36.3 / 50 -> 12.0 / 15.5 / 18.4 / 32.3 / 37.5 us, 128 heads over 20000 150 ->
+// 130.  Held to 128 registers for a second workgroup a CU it spills: 19.6 at 6001.
+constexpr int MLA_CSTR = MLA_LAT + 4, MLA_TILE = 32;
+__global__ __launch_bounds__(512) void mla_split_kernel(MlaArgs a) {
+    __shared__ __align__(16) float sC[MLA_TILE * MLA_CSTR];
+    __shared__ __align__(16) float sS[4][16][MLA_TILE + 4];  // [dim group][head][position]
+    const int split = blockIdx.x, h0 = blockIdx.y * 16;
+    const int tid = threadIdx.x, lane = tid & 63, j16 = lane & 15, c4 = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int pg = wave & 1, dg = wave >> 1;
+    const int L = a.L, P = a.P, t0 = split * P;
+    const int H = min(a.n_head - h0, 16);
+    const bool hv = j16 < H;
+    const rsrc_t C = rsrc(a.c, (size_t)L * a.cstride * 4), PE = rsrc(a.pe, (size_t)L * a.pestride * 4);
+    // rows 4 w .. 4 w + 3 of a tile, a KB a load; and this wave's pe operand
+    f4v rc[8], rp;
+    auto load = [&](int t) {
 #pragma unroll
-        for (int w = 1; w < NW; w++) mnv = fminf(mnv, s_st[2][w][h]);
-        a.pmin[o] = mnv;
+        for (int i = 0; i < 8; i++)
+            rc[i] = __builtin_bit_cast(
+                f4v, __builtin_amdgcn_raw_buffer_load_b128(
+                         C, (unsigned)(((size_t)(t + 4 * wave + i / 2) * a.cstride + 256 * (i % 2) + 4 * lane) * 4), 0, 0));
+        rp = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                         PE, (unsigned)(((size_t)(t + 16 * pg + j16) * a.pestride + 16 * dg + 4 * c4) * 4),
+                                         0, 0));
+    };
+    load(t0);
+    f4v q[9];  // head j16's dims 128 dg + 16 m + 4 c4 .. + 3, then pe's
+    {
+        const float *ql = a.q_lat + (size_t)(h0 + (hv ? j16 : 0)) * MLA_LAT + 128 * dg + 4 * c4;
+        const float *qp = a.q_pe + (size_t)(h0 + (hv ? j16 : 0)) * MLA_ROPE + 16 * dg + 4 * c4;
+#pragma unroll
+        for (int m = 0; m < 9; m++) {
+            const float4 f = *reinterpret_cast<const float4 *>(m < 8 ? ql + 16 * m : qp);
+            q[m] = hv ? f4v{f.x, f.y, f.z, f.w} : f4v{0.f, 0.f, 0.f, 0.f};
+        }
     }
-    if (!whole && j16 < H)  // the scores, for the merge's decision on the 1e-8 skip (stored last)
-        *reinterpret_cast<float4 *>(a.psc + ((size_t)split * a.n_head + h0 + j16) * P + 16 * wave + 4 * c4) =
-            make_float4(s[0], s[1], s[2], s[3]);
+    f4v acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = f4v{0.f, 0.f, 0.f, 0.f};
+    float M = -INFINITY, S = 0.0f, mn = INFINITY;
+    const int end = min(t0 + P, L);
+    for (int t = t0; t < end; t += MLA_TILE) {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            *reinterpret_cast<f4v *>(&sC[(4 * wave + i / 2) * MLA_CSTR + 256 * (i % 2) + 4 * lane]) = rc[i];
+        const f4v pe = rp;
+        __syncthreads();
+        f4v d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            const f4v k = *reinterpret_cast<const f4v *>(&sC[(16 * pg + j16) * MLA_CSTR + 128 * dg + 16 * m + 4 * c4]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], q[m][e], d, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(pe[e], q[8][e], d, 0, 0, 0);
+        *reinterpret_cast<f4v *>(&sS[dg][j16][16 * pg + 4 * c4]) = d;
+        __syncthreads();
+        if (t + MLA_TILE < end) load(t + MLA_TILE);
+        // positions 16 u + 4 c4 + r of head j16
+        f4v s[2];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            f4v x = *reinterpret_cast<const f4v *>(&sS[0][j16][16 * u + 4 * c4]);
+#pragma unroll
+            for (int g = 1; g < 4; g++) x += *reinterpret_cast<const f4v *>(&sS[g][j16][16 * u + 4 * c4]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const bool ok = hv && t + 16 * u + 4 * c4 + r < L;
+                const float sc = x[r] * a.scale;  // (dot(q_lat, c) + dot(q_pe, pe)) * scale, deepseek.rs:567-570
+                s[u][r] = ok ? sc : -INFINITY;
+                mx = fmaxf(mx, s[u][r]);
+                mn = ok ? fminf(mn, sc) : mn;
+            }
+        }
+        mx = rows_max(mx);
+        if (t > t0) {  // rescaled to the running maximum
+            const float Mn = fmaxf(M, mx), c = M == -INFINITY ? 0.0f : expf(M - Mn);
+            S = S * c;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float ci = __shfl(c, 4 * c4 + i);  // of head 4 c4 + i
+#pragma unroll
+                for (int k = 0; k < 4; k++) acc[k][i] = acc[k][i] * ci;
+            }
+            M = Mn;
+        } else {
+            M = mx;
+        }
+        f4v p[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[u][r] = s[u][r] == -INFINITY ? 0.0f : expf(s[u][r] - M);
+                S += p[u][r];
+            }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const f4v v = *reinterpret_cast<const f4v *>(&sC[(16 * u + 4 * c4 + r) * MLA_CSTR + 64 * wave + 4 * j16]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[u][r], v[k], acc[k], 0, 0, 0);
+            }
+        // the scores, for the merge's decision on the 1e-8 skip
+        if (wave == 0 && hv) {
+            float *ps = a.psc + ((size_t)split * a.n_head + h0 + j16) * P + (t - t0) + 4 * c4;
+#pragma unroll
+            for (int u = 0; u < 2; u++) *reinterpret_cast<f4v *>(ps + 16 * u) = s[u];
+        }
+        __syncthreads();  // the tile's rows and scores are read
+    }
+    S = rows_sum(S);
+    mn = rows_min(mn);
+    // acc[k][i]: head 4 c4 + i, dim 64 w + 4 j16 + k
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int h = 4 * c4 + i;
+        if (h < H)
+            *reinterpret_cast<float4 *>(a.pacc + ((size_t)split * a.n_head + h0 + h) * MLA_LAT + 64 * wave + 4 * j16) =
+                make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]);
+    }
+    if (tid < H) {  // lanes c4 = 0 of wave 0
+        const size_t o = (size_t)split * a.n_head + h0 + tid;
+        a.pm[o] = M;
+        a.pl[o] = S;
+        a.pmin[o] = mn;
+    }
 }
 
 // Merge, one workgroup per head and 128 dims (merge_head): the value row of position t is c_t.
@@ -1947,7 +2079,7 @@ __global__ __launch_bounds__(64 * NW) void mla_merge_kernel(MlaArgs a) {
     };
     // (the host knows the splits: four waves are the fast path's launch)
     if constexpr (NW == 4)
-        merge_head_fast<MLA_LAT, D>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
+        merge_head_fast<MLA_LAT, D, mla_merge_ns(D)>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
                                     vrow, a.out);
     else
         merge_head<MLA_LAT, D, NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
@@ -1962,43 +2094,44 @@ int launch_mla(kh_ctx *ctx, int n_head, const float *q_lat, const float *q_pe, c
     if (n_positions == 0) return launch_fill(ctx, out, (size_t)n_head * MLA_LAT, 0.0f);
     if (cstride < MLA_LAT || pestride < MLA_ROPE || cstride % 4 || pestride % 4)
         return fail(KH_EINVAL, "mla_attend: row strides must hold a row and be multiples of 4 floats");
-    if ((n_positions + MLA_P) * cstride * 4 >= 0xffffffffull || (n_positions + MLA_P) * pestride * 4 >= 0xffffffffull)
+    if ((n_positions + 256) * cstride * 4 >= 0xffffffffull || (n_positions + 256) * pestride * 4 >= 0xffffffffull)
         return fail(KH_DECLINED, "mla_attend: caches of 4 GiB or more per layer are not addressed here");
     MlaArgs a{};
     a.q_lat = q_lat, a.q_pe = q_pe, a.c = c, a.pe = pe, a.cstride = cstride, a.pestride = pestride;
     a.n_head = n_head;
     a.L = (int)n_positions;
-    // positions per split: 128 (eight waves) while that still gives a
-    // workgroup per CU -- half the partials to write and merge; 32 (two
-    // waves) for short sequences past one split, twice the workgroups
-    // (measured at L = 1024 / 8192 / 32768: 18.9 / 24.4 / 40.8 us per layer
-    // by this rule, 17.7 / 27.2 / 51.0 with 32 everywhere); else 64
+    // One launch up to MLA_ONE positions (11.5 us; 33 to 64 took 12.9 there,
+    // 11.6 as two splits and a merge); past that splits of 32, 64 or 128
+    // positions, the least that keeps to a workgroup a CU (16 heads over 20000
+    // positions 28.7 us in 157 splits, 34.7 in 313), 256 where 128 make more than
+    // two.  A power of two: the merge reads 256 scores at a time.
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const int hg = (n_head + 15) / 16;
-    const int forced = env_int("KVAD_MLA_SPLIT", 0);  // tuning knob: positions per split (32 / 64 / 128)
-    a.P = forced == 32 || forced == 64 || forced == 128 ? forced
-          : (long long)((n_positions + 127) / 128) * hg >= cu ? 128
-          : n_positions > (size_t)MLA_P && n_positions <= 1024 ? 32
-                                                               : MLA_P;
+    const int forced = env_int("KVAD_MLA_SPLIT", 0);  // tuning knob: positions per split (32 / 64 / 128 / 256)
+    const bool one = n_positions <= (size_t)MLA_ONE && forced == 0;
+    a.P = one ? 64 : forced == 64 || forced == 128 || forced == 256 ? forced : MLA_TILE;
+    auto wgs = [&] { return (long long)((n_positions + a.P - 1) / a.P) * hg; };
+    if (!forced && !one) {
+        while (a.P < 128 && wgs() > cu) a.P *= 2;
+        if (wgs() > 2LL * cu) a.P = 256;
+    }
     a.nsplit = (int)((n_positions + a.P - 1) / a.P);
     if (a.nsplit > MAX_SPLITS) return fail(KH_DECLINED, "mla_attend: sequence longer than the split merge takes");
     a.scale = scale;
     a.out = out;
-    if (a.nsplit > 1) {
+    if (!one) {
         int rc = ensure(ctx, ctx->ws, 4 * partial_floats(a.nsplit, n_head, MLA_LAT, a.P) + 1024);
         if (rc) return rc;
         carve_partials(a, ctx->ws.ptr, MLA_LAT);
     }
-    if (a.P == 128)
-        hipLaunchKernelGGL((mla_split_kernel<8>), dim3(a.nsplit, hg), dim3(512), 0, ctx->stream, a);
-    else if (a.P == 32)
-        hipLaunchKernelGGL((mla_split_kernel<2>), dim3(a.nsplit, hg), dim3(128), 0, ctx->stream, a);
+    if (one)
+        hipLaunchKernelGGL((mla_one_kernel<4>), dim3(1, hg), dim3(256), 0, ctx->stream, a);
     else
-        hipLaunchKernelGGL((mla_split_kernel<4>), dim3(a.nsplit, hg), dim3(256), 0, ctx->stream, a);
+        hipLaunchKernelGGL(mla_split_kernel, dim3(a.nsplit, hg), dim3(512), 0, ctx->stream, a);
     KH_HIP(hipGetLastError());
-    if (a.nsplit > 1) {
+    if (!one) {
         const int fd = mla_merge_dims(a.nsplit);
-        const bool wide = !merge_takes_fast(fd, a.nsplit, a.P);
+        const bool wide = !merge_takes_fast(mla_merge_ns(fd), a.nsplit, a.P);
 #define KH_MERGE(D)                                                                                                   \
     do {                                                                                                              \
         if (wide)                                                                                                     \

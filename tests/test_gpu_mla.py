@@ -134,3 +134,19 @@ def test_128_position_splits_match_the_oracle(ctx, monkeypatch, L):
     got = _run(ctx, ql, qp, c, pe, H, L)
     want = O.mla_attend(H, 512, 64, ql, qp, c, pe, L, SCALE).reshape(H, 512)
     assert np.max(np.abs(got - want)) <= 1e-4 * np.max(np.abs(want)), L
+
+
+@pytest.mark.parametrize("P", ["32", "64", "256"])
+@pytest.mark.parametrize("H,L", [(16, 1), (16, 33), (17, 290), (5, 64), (16, 3000)])
+def test_split_widths_match_the_oracle(ctx, monkeypatch, P, H, L):
+    # splits of one, two and eight 32-position tiles, the sums carried over the
+    # tiles at a running maximum: part-filled last tiles and splits, head
+    # groups of fewer than 16, and scores spread so that the maximum rises from
+    # tile to tile and the merge takes skipped terms back
+    monkeypatch.setenv("KVAD_MLA_SPLIT", P)
+    ql, qp, c, pe = _case(H * 17 + L, H, L)
+    for spread in (1.0, 4.0):
+        got = _run(ctx, ql * np.float32(spread), qp * np.float32(spread), c, pe, H, L)
+        want = O.mla_attend(H, 512, 64, ql * np.float32(spread), qp * np.float32(spread), c, pe, L, SCALE)
+        err = np.max(np.abs(got.ravel() - want.ravel()))
+        assert err <= 1e-4 * np.max(np.abs(want)), (P, H, L, spread, err)
