@@ -615,7 +615,7 @@ __device__ __forceinline__ float block_reduce(float v, float *s_w, F op) {
 }
 
 constexpr int MAX_SPLITS = 4096;
-constexpr int WIDE_NW = 8;  // waves of a merge the fast path does not take
+constexpr int WIDE_NW = 8;  // waves of a merge of long or many splits
 
 // Exclusive prefix sum of one int per thread over the workgroup (NW waves);
 // *total gets the sum.  s holds NW ints and is free again on return.
@@ -734,11 +734,10 @@ __device__ __forceinline__ float4 skipped_terms(const uint16_t *list, int nlist,
 // splits of its own, 256 scores a load (P divides 256), queues the skipped
 // positions in its own LDS and gathers their rows: no barrier between the
 // list and the last sum, and a chain of two loads whatever the list's length
-// over NW waves.  Measured, scores spread by 2 (us per layer, split and merge,
-// before with the candidates scanned 1024 at a time
-// by a block of 256): 32 heads of 128 over 20001 positions 52 -> 45, over 32768
-// 88 -> 73, 14 heads of 64 over 20001 / 32768 25 / 52 -> 17 / 24, 16 latent heads
-// over 32768 50 -> 42.
+// over NW waves.  For launches of more splits than merge_head_fast takes;
+// measured there, scores spread by 2 (us per layer, split and merge, before with
+// the candidates scanned 1024 at a time by a block of 256): 32 heads of 128 over
+// 40000 positions 135 -> 96, 16 latent heads over 70000 153 -> 104.
 template <int HD, int D, int NW, typename VRow>
 __device__ __forceinline__ void merge_head(const float *pm, const float *pl, const float *pmin, const float *pacc,
                                            const float *psc, int ns, int n_head, int h, int d0, int P, int L,
@@ -887,38 +886,40 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
 // (preloaded, as the split kernel's): ROWS (batched rows, or head counts
 // past 16 bits) takes them from the struct and the row table.  pn: P |
 // plus_one << 31; hg: n_head | group << 16.
-// The merge of dims d0 .. d0 + D of one head (rows of HD) without barriers,
-// for up to MAXNS splits: every
-// load is issued at once (each wave reads every split's max, sum and
-// minimum, MAXNS / 64 splits a lane, and its quarter of the dims of every split's
-// partial values, D / 16 float4s a lane-row of 64 / (D / 16) splits), the maximum and the sum are
-// wave butterflies (each wave computes the same ones, in the same order),
-// the weights e^{m_j - M} pass through the wave's own LDS row, and the
-// split groups' sums meet by butterfly.  The straddling splits' skipped terms
-// come after, each wave over all of them for its own dims (skipped_terms).
+// The merge of dims d0 .. d0 + D of one head (rows of HD) by NW waves, for up
+// to MAXNS splits: every load is issued at once (each wave reads every split's
+// max, sum and minimum, MAXNS / 64 splits a lane, and its share of the dims of
+// every split's partial values, D / (4 NW) float4s a lane-row of splits), the
+// maximum and the sum are wave butterflies (each wave computes the same ones,
+// in the same order), the weights e^{m_j - M} pass through the wave's own LDS
+// row, and the split groups' sums meet by butterfly.  The straddling splits'
+// skipped terms come after (skipped_terms): four waves take all of them each,
+// for their own dims, without a barrier; eight share the splits, over all
+// dims, and meet in LDS once.
 // The most splits merge_head_fast takes: 128, or 256 for latent attention's
 // 64-dim slices (whose launches know their splits: a bound the compiler sees
 // in the code it serves, 7.0 -> 7.5 us per short layer where it was 256).
-// Splits of 256 positions, and more than 128 of more than 32, leave to
-// merge_head: over a cache that long a third of them and more straddle, which
-// its eight waves share and the fast path's each go through (14 heads of 64
-// over 32768 positions, scores spread by 2: 53-70 us fast, 24 shared; without
-// a straddling split 13.4 and 14.8).  The host asks for a launch's most splits,
-// the kernel for those of the length it finds.
-__host__ __device__ constexpr bool merge_takes_fast(int maxns, int ns, int P) {
+// Splits of 256 positions, and more than 128 of more than 32, go to the eight
+// waves: over a cache that long a third of them and more straddle, which four
+// each go through in full (14 heads of 64 over 32768 positions, scores spread
+// by 2: 53-70 us, shared 22.7; without a straddling split 13.4 and 12.6).
+// merge_head, which had taken these, came to 24 and 14.8; more splits than
+// maxns are still its own.  The host asks for a launch's most splits, the
+// kernel for those of the length it finds.
+__host__ __device__ constexpr bool merge_takes_four(int maxns, int ns, int P) {
     return ns <= maxns && P <= 128 && (ns <= 128 || P <= 32);
 }
 constexpr int MERGE_NS = 128;                                              // grouped-query attention's
 __host__ __device__ constexpr int mla_merge_ns(int d) { return d <= 64 ? 256 : 128; }
-template <int HD, int D, int MAXNS, typename VRow>
+template <int HD, int D, int MAXNS, int NW, typename VRow>
 __device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl, const float *pmin, const float *pacc,
                                                 const float *psc, int ns, int n_head, int h, int d0, int P, int L,
                                                 VRow vrow, float *out) {
-    constexpr int NQ = D / 16;      // float4s of a wave's dims
+    constexpr int NQ = D / (4 * NW);  // float4s of a wave's dims
     constexpr int SG = 64 / NQ;     // split groups a wave-row holds
     constexpr int PJ = (MAXNS + SG - 1) / SG;  // partial values a lane holds at most
     constexpr int PS = MAXNS / 64;             // splits of statistics a lane holds
-    __shared__ float s_c[4][PS * 64];
+    __shared__ float s_c[NW][PS * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int dq = lane % NQ, sg = lane / NQ;
     const size_t sb = (size_t)ns * n_head * 4;
@@ -933,7 +934,7 @@ __device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl
         mn[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(PN, o, 0, 0));
     }
     float4 v[PJ];
-    const int d = d0 + (D / 4) * wave + 4 * dq;
+    const int d = d0 + (D / NW) * wave + 4 * dq;
 #pragma unroll
     for (int k = 0; k < PJ; k++) {  // split sg + SG k
         const unsigned o = (unsigned)((((size_t)(sg + SG * k) * n_head + h) * HD + d) * 4);
@@ -976,8 +977,8 @@ __device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl
         x.w = x.w + __shfl_xor(x.w, o);
     }
     x = make_float4(x.x * inv, x.y * inv, x.z * inv, x.w * inv);
-    __shared__ uint16_t s_list[4][PS * 64];  // straddling splits, in index order, a copy a wave
-    __shared__ int2 s_queue[4][QCAP];
+    __shared__ uint16_t s_list[NW][PS * 64];  // straddling splits, in index order, a copy a wave
+    __shared__ int2 s_queue[NW][QCAP];
     int nstr = 0;
 #pragma unroll
     for (int u = 0; u < PS; u++) {
@@ -989,14 +990,28 @@ __device__ __forceinline__ void merge_head_fast(const float *pm, const float *pl
     }
     if (nstr) {
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own list
-        float4 f = skipped_terms<NQ>(s_list[wave], nstr, 0, 256 / P, psc, n_head, h, P, L, mx, inv,
-                                     (d0 + (D / 4) * wave) / 4, vrow, s_queue[wave], lane);
+        constexpr bool SHARE = NW > 4;
+        constexpr int FQ = SHARE ? D / 4 : NQ;  // float4s a wave's skipped terms span
+        const int ew = 256 / P;
+        float4 f = skipped_terms<FQ>(s_list[wave], nstr, SHARE ? wave * ew : 0, SHARE ? NW * ew : ew, psc, n_head, h, P, L,
+                                     mx, inv, SHARE ? d0 / 4 : (d0 + (D / NW) * wave) / 4, vrow, s_queue[wave], lane);
 #pragma unroll
-        for (int o = NQ; o < 64; o <<= 1) {
+        for (int o = FQ; o < 64; o <<= 1) {
             f.x = f.x + __shfl_xor(f.x, o);
             f.y = f.y + __shfl_xor(f.y, o);
             f.z = f.z + __shfl_xor(f.z, o);
             f.w = f.w + __shfl_xor(f.w, o);
+        }
+        if constexpr (SHARE) {  // (nstr is the same in every wave)
+            __shared__ __align__(16) float s_fix[NW][D];
+            if (lane < FQ) *reinterpret_cast<float4 *>(&s_fix[wave][4 * lane]) = f;
+            __syncthreads();
+            f = *reinterpret_cast<const float4 *>(&s_fix[0][(D / NW) * wave + 4 * dq]);
+#pragma unroll
+            for (int g = 1; g < NW; g++) {
+                const float4 y = *reinterpret_cast<const float4 *>(&s_fix[g][(D / NW) * wave + 4 * dq]);
+                f = make_float4(f.x + y.x, f.y + y.y, f.z + y.z, f.w + y.w);
+            }
         }
         x = make_float4(x.x - f.x, x.y - f.y, x.z - f.z, x.w - f.w);
     }
@@ -1024,9 +1039,8 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(const int32_t *len_
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               V, (unsigned)(((size_t)t * a.vstride + voff + 4 * d4) * 4), 0, 0));
     };
-    if (merge_takes_fast(MERGE_NS, ns, a.P)) {
-        if (threadIdx.x < 256)  // no barrier in it
-            merge_head_fast<HD, HD, MERGE_NS>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
+    if (ns <= MERGE_NS) {
+        merge_head_fast<HD, HD, MERGE_NS, NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, ns, a.n_head, h, 0, a.P, L, vrow, a.out);
         return;
     }
     if constexpr (NW > 4)  // (the host knows the most splits there can be)
@@ -1479,7 +1493,7 @@ int run(kh_ctx *ctx, const AttnArgs &a, int head_dim, int nb = 1) {
         const unsigned pn = (unsigned)a.P | (a.plus_one ? 1u << 31 : 0u);
         const unsigned hg = (unsigned)a.n_head | (unsigned)a.group << 16;
         const bool rows = a.rows || a.n_head > 0xffff || a.group > 0xffff;
-        const bool wide = !merge_takes_fast(MERGE_NS, a.nsplit, a.P);
+        const bool wide = !merge_takes_four(MERGE_NS, a.nsplit, a.P);
 #define KH_MERGE(HH, RW)                                                                                       \
     do {                                                                                                       \
         if (wide)                                                                                              \
@@ -2077,11 +2091,11 @@ __global__ __launch_bounds__(64 * NW) void mla_merge_kernel(MlaArgs a) {
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               C, (unsigned)(((size_t)t * a.cstride + 4 * d4) * 4), 0, 0));
     };
-    // (the host knows the splits: four waves are the fast path's launch)
-    if constexpr (NW == 4)
-        merge_head_fast<MLA_LAT, D, mla_merge_ns(D)>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
-                                    vrow, a.out);
-    else
+    // (the host knows the splits: four waves are never given more)
+    if (NW == 4 || a.nsplit <= mla_merge_ns(D))
+        merge_head_fast<MLA_LAT, D, mla_merge_ns(D), NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h,
+                                                         D * blockIdx.y, a.P, a.L, vrow, a.out);
+    else if constexpr (NW > 4)
         merge_head<MLA_LAT, D, NW>(a.pm, a.pl, a.pmin, a.pacc, a.psc, a.nsplit, a.n_head, h, D * blockIdx.y, a.P, a.L,
                                    vrow, a.out);
 }
@@ -2131,7 +2145,7 @@ int launch_mla(kh_ctx *ctx, int n_head, const float *q_lat, const float *q_pe, c
     KH_HIP(hipGetLastError());
     if (!one) {
         const int fd = mla_merge_dims(a.nsplit);
-        const bool wide = !merge_takes_fast(mla_merge_ns(fd), a.nsplit, a.P);
+        const bool wide = !merge_takes_four(mla_merge_ns(fd), a.nsplit, a.P);
 #define KH_MERGE(D)                                                                                                   \
     do {                                                                                                              \
         if (wide)                                                                                                     \

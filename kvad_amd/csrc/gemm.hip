@@ -943,7 +943,7 @@ int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, co
         a.xf = xs;
         return launch_f32gemm(ctx, a);
     }
-    // up to eight rows: the multi-token GEMV quantises them as it stages them
+    // a few rows: the VALU multi-token GEMV quantises them as it stages them
     // (QActBatch::new's codes, one launch fewer) while they are few values
     const bool multi = matmul_takes_multi(w->precision, m, rows, cols) && !matmul_force_gemm();
     if (multi && multi_stages_f32(w->precision, m, rows, cols))

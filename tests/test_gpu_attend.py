@@ -228,3 +228,21 @@ def test_merge_takes_back_skipped_terms(ctx, n_head, n_kv, hd, L, spread):
     cache.push(0, k.ravel(), v.ravel())
     got = K.attend(ctx, spec, q.ravel(), cache, 0, L)
     close(got, O.attend(n_head, n_kv, hd, q.ravel(), k.ravel(), v.ravel(), L))
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,L", [(14, 2, 64, 1030), (14, 2, 64, 32768), (4, 2, 128, 32768), (14, 2, 64, 32769)])
+@pytest.mark.parametrize("spread", [0.5, 2.0])
+def test_eight_wave_merge(ctx, monkeypatch, n_head, n_kv, hd, L, spread):
+    # 256-position splits: the fewest that straddle, the most the barrier-free
+    # merge's eight waves take (128) and one past them (the list-based merge),
+    # without a straddling split and with some
+    monkeypatch.setenv("KVAD_ATTN_SPLIT", "256")
+    say("eight-wave merge", n_head, n_kv, hd, L, spread)
+    spec, kvd = K.Spec(n_head, n_kv, hd), n_kv * hd
+    rng = np.random.default_rng(L + hd)
+    q = rng.standard_normal(n_head * hd).astype(np.float32) * np.float32(spread)
+    k, v = rng.standard_normal((2, L * kvd)).astype(np.float32)
+    cache = K.KvCache(ctx, 1, kvd, kvd)
+    cache.push(0, k, v)
+    got = K.attend(ctx, spec, q, cache, 0, L)
+    close(got, O.attend(n_head, n_kv, hd, q, k, v, L))

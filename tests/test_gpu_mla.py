@@ -150,3 +150,16 @@ def test_split_widths_match_the_oracle(ctx, monkeypatch, P, H, L):
         want = O.mla_attend(H, 512, 64, ql * np.float32(spread), qp * np.float32(spread), c, pe, L, SCALE)
         err = np.max(np.abs(got.ravel() - want.ravel()))
         assert err <= 1e-4 * np.max(np.abs(want)), (P, H, L, spread, err)
+
+
+@pytest.mark.parametrize("L", [8200, 16384, 16385])
+def test_eight_wave_merge(ctx, monkeypatch, L):
+    # 64-position splits past 128: shared by eight waves to 256, then the
+    # list-based merge; spread so that splits straddle the 1e-8 line
+    monkeypatch.setenv("KVAD_MLA_SPLIT", "64")
+    ql, qp, c, pe = _case(L, 4, L)
+    for spread in (1.0, 4.0):
+        got = _run(ctx, ql * np.float32(spread), qp * np.float32(spread), c, pe, 4, L)
+        want = O.mla_attend(4, 512, 64, ql * np.float32(spread), qp * np.float32(spread), c, pe, L, SCALE)
+        err = np.max(np.abs(got.ravel() - want.ravel()))
+        assert err <= 1e-4 * np.max(np.abs(want)), (L, spread, err)
