@@ -690,13 +690,44 @@ __global__ __launch_bounds__(THREADS) void gemm_f32_kernel(GemmArgs a) {
 // workgroup, else the smallest.
 enum Shape { T128x128, T128x64, T128x32, T64x64 };
 
-Shape pick_shape(int M, int N, int cu) {
+// The split-K workspace: one fixed allocation for the partials, made on the
+// first split launch and never moved, so graphs captured over later launches
+// stay valid; a split whose partials do not fit is cut to what fits.
+constexpr size_t SPLIT_BYTES = 64u << 20;
+
+// Whether 128 x 128 tiles, of which a CU holds two, fill their rounds of the
+// chip over rows long enough to pay for a workgroup's start.  They need half
+// the LDS and scale traffic of 64 x 64 tiles, but a round that is short of
+// workgroups costs a whole one.  Measured (us, rows' quantisation included, 64 x
+// 64 tiles / 128 x 128): Q4_K 14336x4096 at 512 / 700 / 1000 tokens, 448 / 672 /
+// 896 tiles, 157 / 210 / 282 and 138 / 226 / 268; q8 115 / 160 / 221 and 107 / 165 /
+// 208; 8192x2048 at 700 / 1000 / 1500, 384 / 512 / 768 tiles, 53 / 70 / 99 and 60 /
+// 63 / 92; q8 9728x896 at 700, 456 tiles of seven stages, 32.5 and 33.5.  Fewer
+// tiles fill a round split along k, from 13 stages a split of 8192 columns or
+// more: 4096x14336 at 256 / 384 / 512 / 700 / 1000 tokens, 512 / 480 / 512 / 576 / 512
+// workgroups, Q4_K 107 / 189 / 189 / 225 / 353 and 80 / 116 / 141 / 273 / 266, q8 75 /
+// 124 / 130 / 164 / 231 and 65 / 93 / 112 / 202 / 206; shorter
+// splits go both ways (4096x4096 at 512 tokens, eight stages, 43.6 and 47.9,
+// 2048x8192 at 700, 12.8, 76 and 64).  Token tiles more than an
+// eighth empty are left to the smaller ones.
+bool fills_rounds(long long M, long long N, long long K, long long cu) {
+    const long long t = (N + 127) / 128 * ((M + 127) / 128), stages = (K + BK - 1) / BK;
+    if (M < 128 || 8 * ((M + 127) / 128 * 128) > 9 * M) return false;
+    if (t > cu) return stages >= 16 && (t >= 3 * cu || (4 * t >= 7 * cu && t <= 2 * cu));
+    if (stages < 64) return false;
+    // the split that set_split comes to
+    long long ks = (2 * cu + t / 2) / t;
+    ks = std::min(ks, K / (4 * M) * (2 * t <= cu ? 2 : 1));
+    ks = std::min(ks, (long long)SPLIT_BYTES / (4 * M * N));
+    return ks >= 2 && stages >= 13 * ks && 4 * t * ks >= 7 * cu && t * ks <= 2 * cu;
+}
+Shape pick_shape(int M, int N, int K, int cu) {
     const int forced = env_int("KVAD_GEMM_TILE_M", 0);  // tuning knob: tokens per tile (6464: 64 x 64)
     if (forced == 6464) return T64x64;
     if (forced == 128 || forced == 64 || forced == 32) return forced == 128 ? T128x128 : forced == 64 ? T128x64 : T128x32;
     const long long nt = (N + 127) / 128;
-    // 128 x 128 tiles while they give four workgroups per CU; below that, past
-    // 64 tokens, 64 x 64 tiles: more, smaller workgroups hide the k-stages' load
+    // 128 x 128 tiles while they give four workgroups per CU, or fill their
+    // rounds of the chip; else, past 64 tokens, 64 x 64 tiles: more, smaller workgroups hide the k-stages' load
     // latency ((512, 896, 4864) 28.5 -> 27.4 us against 128-row 32-token tiles,
     // (512, 4864, 896) 19.1 -> 17.8, (128, 896, 896) 10.9 -> 10.3, all split alike;
     // at (2048, 4096, 14336) they lose, 461 -> 597, and at 16 tokens over
@@ -705,6 +736,7 @@ Shape pick_shape(int M, int N, int cu) {
     // tokens (a vocabulary head) gives enough workgroups with 32-token
     // tiles, and 128-token ones would leave three quarters of every tile idle.
     if (M > 64 && nt * ((M + 127) / 128) >= 4LL * cu) return T128x128;
+    if (fills_rounds(M, N, K, cu)) return T128x128;
     if (M > 64 && M < 128 && nt >= cu) return T128x128;
     if (M > 64) return T64x64;
     if (M > 32 && nt >= cu) return T128x64;
@@ -713,8 +745,8 @@ Shape pick_shape(int M, int N, int cu) {
 
 }  // namespace
 
-int gemm_tiles(kh_ctx *ctx, int M, int N, int *tile_n) {
-    const Shape sh = pick_shape(M, N, ctx->cu_count > 0 ? ctx->cu_count : 256);
+int gemm_tiles(kh_ctx *ctx, int M, int N, int K, int *tile_n) {
+    const Shape sh = pick_shape(M, N, K, ctx->cu_count > 0 ? ctx->cu_count : 256);
     *tile_n = sh == T64x64 ? 64 : 128;
     return sh == T128x128 ? 128 : sh == T128x32 ? 32 : 64;
 }
@@ -826,10 +858,6 @@ bool matmul_force_gemm() { return env_int("KVAD_MATMUL_GEMM", 0) == 1; }
 }  // namespace
 
 namespace {
-// The split-K workspace: one fixed allocation for the partials, made on the
-// first split launch and never moved, so graphs captured over later launches
-// stay valid; a split whose partials do not fit is cut to what fits.
-constexpr size_t SPLIT_BYTES = 64u << 20;
 const int SPLIT_MIN_STAGES = env_int("KVAD_GEMM_SPLIT_MIN", 2);  // tuning knobs
 const int SPLIT_MAX = env_int("KVAD_GEMM_SPLIT_MAX", 32);
 const int SPLIT_PER_CU = env_int("KVAD_GEMM_SPLIT_PER_CU", 2);
@@ -981,7 +1009,7 @@ int launch_matmul_q(kh_ctx *ctx, const kh_weight *w, const QAct &q, size_t m, co
     a.xs = q.scales;
     a.xsum = q.sums;
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const Shape sh = pick_shape(a.M, a.N, cu);
+    const Shape sh = pick_shape(a.M, a.N, a.K, cu);
     const int tile_m = sh == T128x128 ? 128 : sh == T128x32 ? 32 : 64, tile_n = sh == T64x64 ? 64 : 128;
     int rc = plan_split(ctx, a, tile_m, tile_n);
     if (rc) return rc;
@@ -1019,7 +1047,7 @@ int launch_matmul_jobs(kh_ctx *ctx, int k, const kh_weight *const *w, const QAct
     a.w2 = w[1]->qs, a.ws2 = w[1]->scales, a.bias2 = bias[1], a.y2 = y[1], a.N2 = (int)w[1]->rows;
     if (k == 3) a.w3 = w[2]->qs, a.ws3 = w[2]->scales, a.bias3 = bias[2], a.y3 = y[2], a.N3 = (int)w[2]->rows;
     int tn;
-    const int tm = gemm_tiles(ctx, a.M, (int)rows, &tn);
+    const int tm = gemm_tiles(ctx, a.M, (int)rows, a.K, &tn);
     const int rc = plan_split(ctx, a, tm, tn);
     return rc ? rc : launch_gemm_q(ctx, w[0]->precision, a, 0, tm, tn);
 }

@@ -442,7 +442,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     a.xq = xq.qs, a.xs = xq.scales, a.xsum = xq.sums;
     a.M = (int)m, a.K = (int)gate->cols;
     int tn;
-    const int tm = gemm_tiles(ctx, (int)m, (int)gate->rows, &tn);
+    const int tm = gemm_tiles(ctx, (int)m, (int)gate->rows, (int)gate->cols, &tn);
     int rc;
     a.w = gate->qs, a.ws = gate->scales, a.N = (int)gate->rows, a.y = g;
     if (gate->precision == up->precision && gate->rows == up->rows && gate->cols == up->cols) {
@@ -460,7 +460,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     d.M = (int)m, d.K = (int)down->cols, d.N = (int)down->rows;
     d.w = down->qs, d.ws = down->scales, d.y = y;
     int tdn;
-    const int td = gemm_tiles(ctx, (int)m, (int)down->rows, &tdn);
+    const int td = gemm_tiles(ctx, (int)m, (int)down->rows, (int)down->cols, &tdn);
     if ((rc = plan_split(ctx, d, td, tdn))) return rc;
     return launch_gemm_q(ctx, down->precision, d, 0, td, tdn);
 }

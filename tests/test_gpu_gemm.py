@@ -275,3 +275,20 @@ def test_few_tokens_over_a_wide_activation(ctx, prec, m):
     w, parts = make(ctx, prec, rows, cols, seed=rows + m)
     xs = O.normal(m + 99, m * cols)
     close(w.matmul_bt(xs, m), oracle_matmul(prec, parts, rows, cols, xs, m))
+
+
+@pytest.mark.parametrize("prec,rows,cols,m", [("q8", 7165, 2080, 1000), ("q4k", 7165, 2048, 1000), ("q4", 7165, 2048, 897),
+                                              ("q8", 2045, 8224, 1000), ("q4k", 2045, 8192, 1000), ("q4", 2045, 8192, 1000)])
+def test_tiles_that_fill_rounds(ctx, prec, rows, cols, m):
+    # 128 x 128 tiles below four a CU: 448 of 16 stages, and 128 in four splits
+    # of 16, ragged in rows, tokens and (q8) k; the edge tiles against the oracle
+    say("matmul full rounds", prec, rows, cols, m)
+    r_idx = np.r_[0:8, 120:136, rows - 8:rows]
+    t_idx = np.r_[0:8, 120:136, m - 8:m]
+    w, parts = make(ctx, prec, rows, cols, seed=rows + cols)
+    xs = O.normal(m + 7, m * cols)
+    got = w.matmul_bt(xs, m).reshape(m, rows)
+    sub = tuple(np.ascontiguousarray(np.asarray(p).reshape(rows, -1)[r_idx]).ravel() for p in parts)
+    want = oracle_matmul(prec, sub, len(r_idx), cols, xs.reshape(m, cols)[t_idx].ravel(), len(t_idx))
+    close(got[np.ix_(t_idx, r_idx)], want.reshape(len(t_idx), len(r_idx)))
+    assert np.all(np.isfinite(got))
