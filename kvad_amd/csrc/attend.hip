@@ -1059,15 +1059,27 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(const int32_t *len_
 // reference R near the column's maximum and their products with the values,
 // the column's smallest score kept beside them; the waves' (R, S) and sums
 // meet in LDS in wave order.  Where the smallest weight of some column is under
-// the reference's 1e-8 line (mod.rs:807) the workgroup goes over the positions
-// twice more, for M and S = sum e^{s - M} and then the weights themselves,
-// w = e^{s - M} * (1/S), w < 1e-8 dropped, times the values (normal scores
-// spread by 2: four columns in a thousand at 1500 positions).  Every column's
-// whole sequence is in one workgroup: no partials in memory and no merge launch.  Scores are
-// dot(q, k) * scale (mod.rs:802).  Bound by the matrix cores' f32 rate and the
-// exponentials between its products: over
-// 512 rows of 14 heads of 64 at 1000 positions and 476 at 1500 the two passes
-// alone took 43 and 60 us, the one pass 28 and 40.
+// the reference's 1e-8 line (mod.rs:807) the sums are not used: by then M and S
+// are known, and a second pass takes the weights themselves,
+// w = e^{s - M} * (1/S), w < 1e-8 dropped, times the values.  The first pass
+// leaves the values out from the point where it foresees that.  Every column's
+// whole sequence is in one workgroup: no partials in memory and no merge launch.
+// Scores are dot(q, k) * scale (mod.rs:802).
+//
+// Bound by the keys and values each workgroup reads from L2 (512 rows of 14
+// heads of 64 over 8000 positions: 2 GB in 172 us) and, over short sequences, by
+// the chain of a tile.  A prompt's passes of 512 rows (us, all of them) where no
+// weight is dropped / where most workgroups drop some (normal scores spread by 1
+// / by 3), against two passes everywhere and against a dropped weight found
+// only at the end and paid with two passes more:
+//   14 heads of 64 over 512, 1500, 8000:   18 / 27, 92 / 140, 1660 / 2700
+//                         two everywhere   25 / 25, 137 / 132, 2780 / 2750
+//                         found at the end 18 / 40, 94 / 213, 1710 / 4450
+//   32 heads of 128 over 512, 1500, 8000:  50 / 86, 254 / 446, 5020 / 9980
+//                         two everywhere   87 / 84, 454 / 453, 10180 / 10140
+//                         found at the end 52 / 125, 263 / 678, 5480 / 16260
+// Where a workgroup in two drops one (spread by 2 over 3000) 463 and 1670, two
+// passes everywhere 445 and 1580.
 struct PassArgs {
     const float *q;        // [n][n_head][HD]
     const AttnRow *rows;   // [n]: the cache (the same for every row) and each row's length
@@ -1077,8 +1089,11 @@ struct PassArgs {
     float scale;
 };
 
+// A barrier over the workgroup's LDS accesses; loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <int HD, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
+__global__ __launch_bounds__(64 * NW, HD == 64 ? 4 : 2) void attn_pass_kernel(PassArgs a) {
     constexpr int NQ4 = HD / 16, VT = HD / 64, NT = HD / 16;
     constexpr int STEP = 16 * NW;  // positions between one wave's tiles
     const int tid = threadIdx.x, lane = tid & 63, j16 = lane & 15, c4 = lane >> 4;
@@ -1139,13 +1154,15 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
     __shared__ float s_on[3][NW][16];                    // each wave's reference, sum, smallest score
     __shared__ __align__(16) float s_acc[NW][16][HD];    // the waves' sums
     __shared__ float s_f[NW][16];
+    __shared__ int s_skips;  // a wave foresees a weight under the line
     // One pass: e^{s - R} against a reference R, the first tile's maximum,
     // raised (and the sums rescaled) only when a score passes it by 8, which
     // few sequences do again: no maximum across lanes per tile.
     {
         float R = 0.0f, S = 0.0f, mn = INFINITY;
         bool started = false;  // R is a score of the column's
-        auto online = [&](int t0, const f4v (&kq)[NQ4], const f4v (&vv)[4][VT]) {
+        float p[4];            // the tile's e^{s - R}
+        auto online = [&](int t0, const f4v (&kq)[NQ4]) {
             float s[4];
             scores(t0, kq, s);
             const float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
@@ -1163,30 +1180,71 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
                     for (int q = 0; q < NT; q++) acc[q][i] = acc[q][i] * ci;
                 }
             }
-            float p[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 p[r] = expf(s[r] - R);  // 0 where masked: R is finite
                 S += p[r];
                 mn = s[r] == -INFINITY ? mn : fminf(mn, s[r]);
             }
+        };
+        auto values = [&](const f4v (&vv)[4][VT]) {
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int q = 0; q < NT; q++)
                     acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], vv[r][q >> 2][q & 3], acc[q], 0, 0, 0);
         };
-        f4v ka[NQ4], kb[NQ4], va[4][VT], vb[4][VT];
-        load_k(16 * wave, ka);
-        load_v(16 * wave, va);
-        for (int t0 = 16 * wave; t0 < L; t0 += 2 * STEP) {
+        int t0 = 16 * wave;
+        f4v ka[NQ4], kb[NQ4];
+        load_k(t0, ka);
+        if (tid == 0) s_skips = 0;
+        lds_barrier();
+        {
+            f4v va[4][VT], vb[4][VT];
+            load_v(t0, va);
+            // Whether a weight under 1e-8 is in sight after 1, 2, 4, 6, ... tiles
+            // of the wave: a score under the line that the column is heading for,
+            // its sum so far grown to L positions, and half a unit more per e-fold
+            // of positions the waves have yet to see (drawn anew at 1, 2, 4, 8,
+            // ...).  A whole unit foresees too much: 32 heads of 128 over 8000
+            // positions spread by 1, where none is dropped, 5020 -> 6580 us.
+            float line = -INFINITY;
+            constexpr float LN2 = 0.69314718f, LOG2_NW = NW == 8 ? 3.0f : NW == 4 ? 2.0f : NW == 2 ? 1.0f : 0.0f;
+            auto foresees = [&](int done) {
+                if ((done & (done - 1)) == 0) {
+                    const float f = __log2f((float)L) - __log2f((float)(16 * done));  // log2 of the growth
+                    line = fmaf(LN2, __log2f(rows_sum(S)) + f + 0.5f * fmaxf(f - LOG2_NW, 0.0f), R - 18.420681f);
+                }
+                const bool skips = __builtin_amdgcn_ballot_w64(mn < line);
+                if (skips) __hip_atomic_store(&s_skips, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                return skips;
+            };
+            // (whether some wave foresees it does not depend on when another
+            // leaves the values out: R, S and mn go on alike)
+            for (int i = 2; t0 < L; i += 2) {
+                bool told = __hip_atomic_load(&s_skips, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                load_k(t0 + STEP, kb);
+                load_v(t0 + STEP, vb);
+                online(t0, ka);
+                if (i == 2) told = foresees(1);
+                if (!told) values(va);
+                t0 += STEP;
+                if (t0 >= L) break;
+                load_k(t0 + STEP, ka);
+                load_v(t0 + STEP, va);
+                online(t0, kb);
+                if (!told) values(vb);
+                t0 += STEP;
+                if (foresees(i) || told) break;
+            }
+        }
+        // the rest without the values, if any
+        for (; t0 < L; t0 += 2 * STEP) {
             load_k(t0 + STEP, kb);
-            load_v(t0 + STEP, vb);
-            online(t0, ka, va);
+            online(t0, ka);
             if (t0 + STEP >= L) break;
             load_k(t0 + 2 * STEP, ka);
-            load_v(t0 + 2 * STEP, va);
-            online(t0 + STEP, kb, vb);
+            online(t0 + STEP, kb);
         }
         S = rows_sum(S);
         mn = rows_min(mn);
@@ -1221,8 +1279,15 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
             *reinterpret_cast<float4 *>(a.out + ((size_t)row * a.n_head + head) * HD + d) = x;
         }
     };
-    store_acc();
-    __syncthreads();
+    f4v ka[NQ4], va[4][VT];
+    const bool again = __hip_atomic_load(&s_skips, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (again) {  // the second pass's first tile
+        load_k(16 * wave, ka);
+        load_v(16 * wave, va);
+    } else {
+        store_acc();
+    }
+    lds_barrier();
     float M = -INFINITY, S = 0.0f;  // the column's, over the waves in order
     {
         float mn = INFINITY;
@@ -1237,9 +1302,9 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
             S = rw == -INFINITY ? S : fmaf(s_on[1][w][j16], expf(rw - M), S);
         }
         const float inv = 1.0f / S;
-        // the smallest weight kept: the same in every wave
+        // the smallest weight kept, and all values taken: the same in every wave
         const bool skips = hv && expf(mn - M) * inv < 1e-8f;
-        if (!__builtin_amdgcn_ballot_w64(skips)) {
+        if (!s_skips && !__builtin_amdgcn_ballot_w64(skips)) {
             if (c4 == 0) {
                 const float rw = s_on[0][wave][j16];
                 s_f[wave][j16] = rw == -INFINITY ? 0.0f : expf(rw - M) * inv;
@@ -1248,51 +1313,9 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
             return;
         }
     }
-    // Some column has weights the reference drops: its own two passes.
-    // pass 1: the maximum M and the sum of e^{s - M}
-    M = -INFINITY, S = 0.0f;
-    auto stats = [&](int t0, const f4v (&kq)[NQ4]) {
-        float s[4];
-        scores(t0, kq, s);
-        const float mx = rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
-        const float Mn = fmaxf(M, mx);
-        float e = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; r++) e += s[r] == -INFINITY ? 0.0f : expf(s[r] - Mn);
-        e = rows_sum(e);
-        S = (M == -INFINITY ? 0.0f : S * expf(M - Mn)) + e;
-        M = Mn;
-    };
-    {
-        f4v ka[NQ4], kb[NQ4];
-        load_k(16 * wave, ka);
-        for (int t0 = 16 * wave; t0 < L; t0 += 2 * STEP) {
-            load_k(t0 + STEP, kb);
-            stats(t0, ka);
-            if (t0 + STEP >= L) break;
-            load_k(t0 + 2 * STEP, ka);
-            stats(t0 + STEP, kb);
-        }
-    }
-    if constexpr (NW > 1) {  // the waves' statistics, in wave order
-        __shared__ float s_st[2][NW][16];
-        if (c4 == 0) {
-            s_st[0][wave][j16] = M;
-            s_st[1][wave][j16] = S;
-        }
-        __syncthreads();
-        M = s_st[0][0][j16];
-#pragma unroll
-        for (int w = 1; w < NW; w++) M = fmaxf(M, s_st[0][w][j16]);
-        S = 0.0f;
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const float mw = s_st[0][w][j16];
-            S = mw == -INFINITY ? S : fmaf(s_st[1][w][j16], expf(mw - M), S);
-        }
-    }
+    // Some column has weights the reference drops: a second pass, by M and S.
     const float inv = 1.0f / S;  // inv = 1 / sum, tensor.rs:304
-    // pass 2: the weights times the values
+    // the weights times the values
 #pragma unroll
     for (int q = 0; q < NT; q++) acc[q] = f4v{0.f, 0.f, 0.f, 0.f};
     auto accumulate = [&](int t0, const f4v (&kq)[NQ4], const f4v (&vv)[4][VT]) {
@@ -1311,9 +1334,11 @@ __global__ __launch_bounds__(64 * NW) void attn_pass_kernel(PassArgs a) {
                 acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], vv[r][q >> 2][q & 3], acc[q], 0, 0, 0);
     };
     {
-        f4v ka[NQ4], kb[NQ4], va[4][VT], vb[4][VT];
-        load_k(16 * wave, ka);
-        load_v(16 * wave, va);
+        f4v kb[NQ4], vb[4][VT];
+        if (!again) {
+            load_k(16 * wave, ka);
+            load_v(16 * wave, va);
+        }
         for (int t0 = 16 * wave; t0 < L; t0 += 2 * STEP) {
             load_k(t0 + STEP, kb);
             load_v(t0 + STEP, vb);
