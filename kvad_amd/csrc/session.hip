@@ -481,12 +481,26 @@ int ensure_pass(kh_llm *m, size_t n, size_t max_len) {
 // y[n][rows] (+)= xs W^T (+bias): f32 weights on the f32 GEMM, quantised
 // ones from the rows' codes in qa (matmul_bt, quant.rs:751; tensor.rs:102);
 // with accumulate the product is added into y (the residual add).
-// Projections of the same input (q/k/v, gate/up) take one multi-token GEMV
-// launch up to this many rows.  A single projection (o, down, the head)
-// follows kh_matmul's rule.
+// Projections take the multi-token GEMV up to this many rows at most.
 size_t rows_multi_max() {
     static const size_t v = (size_t)env_int("KVAD_ROWS_MULTI", 64);  // tuning knob
     return v;
+}
+
+// Whether projections of the same input (q/k/v, gate/up) take one multi-token
+// GEMV launch.  (A single projection -- o, down, the head -- follows kh_matmul's
+// rule.)  Up to 16 rows, and over 4096 columns at most up to all of them.  A
+// launch of several weights is not split over the grid, so past 16 rows wider
+// weights are streamed once per 16 rows: ahead of the GEMM's one launch for
+// Q4_K up to three times, behind it for q8 and q4.  A layer's pass (us, GEMV /
+// GEMM for q/k/v and gate/up): q8 5120 wide (13824 ff) at 24 / 33 / 64 rows 211
+// / 205, 251 / 230, 293 / 241, 8192 wide (28672 ff) 409 / 328, 554 / 400, 693 /
+// 419; q4 5120 191 / 190, 235 / 228, 269 / 235; Q4_K 5120 194 / 207, 250 / 265,
+// 289 / 277 and at 48 254 / 267, 8192 305 / 349, 421 / 469, 488 / 479 and 427 /
+// 469; 4096 wide (14336 ff) at 64 rows q8 203 / 206, q4 196 / 207, Q4_K 212 / 233.
+bool joint_takes_multi(int precision, size_t n, size_t cols) {
+    if (n > rows_multi_max()) return false;
+    return n <= 16 || cols <= 4096 || (precision == KH_Q4K && n <= 48);
 }
 
 int project(kh_ctx *ctx, const kh_weight *w, const float *xs, const QAct &qa, size_t n, const float *bias, float *y,
@@ -513,7 +527,8 @@ int project_all(kh_ctx *ctx, int k, const kh_weight *const *w, const float *xs, 
     bool one = true;
     for (int i = 0; i < k; i++)
         one = one && w[i]->precision != KH_F32 && w[i]->precision == w[0]->precision && w[i]->cols == w[0]->cols;
-    if (one && n <= rows_multi_max()) return launch_gemv_multi_jobs(ctx, k, w, bias, y, nullptr, qa, n);
+    if (one && joint_takes_multi(w[0]->precision, n, w[0]->cols))
+        return launch_gemv_multi_jobs(ctx, k, w, bias, y, nullptr, qa, n);
     if (one) {
         const int rc = launch_matmul_jobs(ctx, k, w, qa, n, bias, y);
         if (rc != KH_DECLINED) return rc;

@@ -39,8 +39,18 @@ import kvad_amd as K  # noqa: E402
 
 from test_gpu_gemv import say  # noqa: E402
 from test_gpu_llm import LOGIT_RTOL, build  # noqa: E402
-from test_gpu_llm_stages import close_residual, proj  # noqa: E402
+from test_gpu_llm_stages import close_residual, proj as proj_q8  # noqa: E402
 from test_gpu_moe_stages import close  # noqa: E402
+
+
+def proj(w, rows, cols, x, bias=None):
+    """y = x W^T (+ bias) of one row: q8 in f64 over exact block dots, q4 and
+    Q4_K as the oracle's matmul gives it."""
+    if not isinstance(w[0], str):
+        return proj_q8(w, rows, cols, x, bias)
+    x = np.ascontiguousarray(x, np.float32)
+    return O.matmul_q4k(w[1], rows, cols, x, 1, bias) if w[0] == "q4k" else O.matmul_q4(w[1], w[2], rows, cols, x, 1, bias)
+
 
 VARIANTS = {
     # batched_decode.rs:264: ("llama", F32), ("qwen3", Q8)
@@ -393,3 +403,32 @@ def test_widely_spread_scores_cost_a_second_pass_at_most(ctx):
         best[spread] = min(times)
     say("pass, time of spread scores, ms", {k: round(1e3 * v, 2) for k, v in best.items()})
     assert best[4.0] <= 1.55 * best[0.5], best
+
+
+@pytest.mark.parametrize("prec,n_embd,n,multi", [("q8", 4128, 40, False), ("q4", 4128, 17, False), ("q4k", 4352, 49, False),
+                                                 ("q8", 4128, 16, True), ("q8", 4096, 40, True), ("q4k", 4352, 48, True)])
+def test_joint_projections_of_wide_rows(ctx, monkeypatch, prec, n_embd, n, multi):
+    # q/k/v of one pass past 16 rows: on the GEMM where the multi-token GEMV,
+    # which cannot split several weights over the grid, would stream them once
+    # per 16 rows.  The GEMM's sums of a row (its k-stages unsplit) do not
+    # depend on the rows beside it: bit for bit those of 70 rows, which always
+    # take it; the GEMV's run in another order.
+    monkeypatch.setenv("KVAD_GEMM_KSPLIT", "1")
+    say("joint projections", prec, n_embd, n)
+    m, mk = build(ctx, 390, n_layer=1, n_ctx=96, n_embd=n_embd, n_head=4, n_kv_head=1, head_dim=64, n_ff=256, prec=prec)
+    m.reading(70)
+    ref = mk()
+    s, L = ref.s, ref.layers[0]
+    toks = [(i * 19 + 6) % 512 for i in range(70)]
+    few = m.trace_pass(toks[:n])
+    m.truncate(0)
+    many = m.trace_pass(toks)["qkv"][0][:n]
+    same = np.array_equal(few["qkv"][0], many)
+    assert same != multi
+    qd, kvd = 256, 64
+    for i in (0, n // 2, n - 1):
+        h = O.rms_norm(few["x_embed"][i], L["attn_norm"], s["eps"])
+        for at, name, rows in ((0, "q", qd), (qd, "k", kvd), (qd + kvd, "v", kvd)):
+            want = proj(L[name], rows, n_embd, h, L.get(name + "_b"))
+            for got in (few["qkv"][0], many):
+                close(got[i, at:at + rows], want, f"row {i} {name}")
