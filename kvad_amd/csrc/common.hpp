@@ -365,8 +365,8 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
 // splitting its k-stages pays (ksplit 0: no split).
 int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n = 128);
 // Tokens per tile (returned) and weight rows per tile (*tile_n) for an
-// ungrouped M x N launch of the int8 GEMM.
-int gemm_tiles(kh_ctx *ctx, int M, int N, int K, int *tile_n);
+// ungrouped launch of the int8 GEMM over a's weights.
+int gemm_tiles(kh_ctx *ctx, int precision, const GemmArgs &a, int *tile_n);
 
 // Operator bodies on device pointers (abi.hip), for the layers built on them.
 int matvec_device(kh_ctx *ctx, const kh_weight *w, const float *x, const float *bias, float *y, int32_t *dots);

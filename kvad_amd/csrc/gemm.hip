@@ -695,10 +695,54 @@ enum Shape { T128x128, T128x64, T128x32, T64x64 };
 // stay valid; a split whose partials do not fit is cut to what fits.
 constexpr size_t SPLIT_BYTES = 64u << 20;
 
-// Whether 128 x 128 tiles, of which a CU holds two, fill their rounds of the
-// chip over rows long enough to pay for a workgroup's start.  They need half
+const int SPLIT_MIN_STAGES = env_int("KVAD_GEMM_SPLIT_MIN", 2);  // tuning knobs
+const int SPLIT_MAX = env_int("KVAD_GEMM_SPLIT_MAX", 32);
+const int SPLIT_PER_CU = env_int("KVAD_GEMM_SPLIT_PER_CU", 2);
+// Under twelve stages of 128 the second launch costs more than the shorter
+// chains save: (512 tokens, 896 rows, 896) 14.1 us in two splits, 11.2
+// unsplit, (80, 4864, 896) 14.0 and 10.9.
+constexpr int SPLIT_LEAST = 12;
+
+// Rows of every weight of a launch, and their tiles.
+long long all_rows(const GemmArgs &a) { return (long long)a.N + (a.y2 ? a.N2 : 0) + (a.y3 ? a.N3 : 0); }
+long long row_tiles(const GemmArgs &a, int tile_n) {
+    auto tiles = [&](int n) { return ((long long)n + tile_n - 1) / tile_n; };
+    return tiles(a.N) + (a.y2 ? tiles(a.N2) : 0) + (a.y3 ? tiles(a.N3) : 0);
+}
+
+// How many splits a launch's k-stages are cut into (under 2: none): `stages` of
+// them, at least `min_st` a split, none under `least`, so that the grid comes to
+// about SPLIT_PER_CU workgroups per CU (a CU holds several: one's loads wait while
+// another's MFMAs run), at most SPLIT_MAX splits, and partials (4 M N bytes a
+// split, written and read again) of at most the weights' wbytes or 4 MiB,
+// whichever is more (a small weight such as a router's 64 rows would otherwise
+// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); twice
+// that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
+// 4096) 36.3 -> 27.5 us in four splits instead of two, (512, 896, 4864) 27.5 ->
+// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two).
+long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st, int least, size_t wbytes, int cu) {
+    const size_t plane = (size_t)a.M * all_rows(a) * 4;
+    const size_t most = std::max(wbytes, (size_t)4 << 20) * (2 * tiles <= cu ? 2 : 1);
+    long long ks = stages < least ? 1 : ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
+    ks = std::min<long long>(ks, stages / min_st);
+    ks = std::min<long long>(ks, SPLIT_MAX);
+    ks = std::min<long long>(ks, (long long)(most / plane));
+    const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
+    if (forced > 0) ks = std::min(forced, stages);
+    return std::min<long long>(ks, (long long)(SPLIT_BYTES / plane));
+}
+// The int8 GEMM's, in tiles of tile_m tokens by tile_n rows.
+long long split_count_i8(const GemmArgs &a, int tile_m, int tile_n, int cu) {
+    return split_count(a, row_tiles(a, tile_n) * ((a.M + tile_m - 1) / tile_m), (a.K + BK - 1) / BK, SPLIT_MIN_STAGES,
+                       SPLIT_LEAST, (size_t)all_rows(a) * a.K, cu);
+}
+
+// Whether 128 x 128 tiles, of which a CU holds two, use the chip well enough
+// over rows long enough to pay for a workgroup's start.  They need half
 // the LDS and scale traffic of 64 x 64 tiles, but a round that is short of
-// workgroups costs a whole one.  Measured (us, rows' quantisation included, 64 x
+// workgroups costs a whole one: taken from seven eighths of a round of two a CU,
+// and from a round and a half on, where the sweep had them ahead whether the last
+// one is full or not.  Measured (us, rows' quantisation included, 64 x
 // 64 tiles / 128 x 128): Q4_K 14336x4096 at 512 / 700 / 1000 tokens, 448 / 672 /
 // 896 tiles, 157 / 210 / 282 and 138 / 226 / 268; q8 115 / 160 / 221 and 107 / 165 /
 // 208; 8192x2048 at 700 / 1000 / 1500, 384 / 512 / 768 tiles, 53 / 70 / 99 and 60 /
@@ -709,23 +753,28 @@ constexpr size_t SPLIT_BYTES = 64u << 20;
 // 124 / 130 / 164 / 231 and 65 / 93 / 112 / 202 / 206; shorter
 // splits go both ways (4096x4096 at 512 tokens, eight stages, 43.6 and 47.9,
 // 2048x8192 at 700, 12.8, 76 and 64).  Token tiles more than an
-// eighth empty are left to the smaller ones.
-bool fills_rounds(long long M, long long N, long long K, long long cu) {
-    const long long t = (N + 127) / 128 * ((M + 127) / 128), stages = (K + BK - 1) / BK;
-    if (M < 128 || 8 * ((M + 127) / 128 * 128) > 9 * M) return false;
+// eighth empty are left to the smaller ones, and so are six splits and more of
+// q8 and q4 rows that are no multiple of four, whose partials go value by value
+// (574 tokens, 1082 rows, 18528 columns, eleven splits, 76 and 112; 586, 1152,
+// 18688, eleven, 82 and 74; over 24 shapes of six to eleven splits 0.68 to 1.01 of
+// the smaller tiles' speed, of rows in fours 0.96 to 1.27; Q4_K 0.93 to 1.48 over
+// either).
+bool fills_rounds(kh_ctx *ctx, int precision, const GemmArgs &a, long long cu) {
+    const long long M = a.M, mt = (M + 127) / 128, t = row_tiles(a, 128) * mt, stages = (a.K + BK - 1) / BK;
+    if (M < 128 || 8 * 128 * mt > 9 * M) return false;
     if (t > cu) return stages >= 16 && (t >= 3 * cu || (4 * t >= 7 * cu && t <= 2 * cu));
     if (stages < 64) return false;
-    // the split that set_split comes to
-    long long ks = (2 * cu + t / 2) / t;
-    ks = std::min(ks, K / (4 * M) * (2 * t <= cu ? 2 : 1));
-    ks = std::min(ks, (long long)SPLIT_BYTES / (4 * M * N));
-    return ks >= 2 && stages >= 13 * ks && 4 * t * ks >= 7 * cu && t * ks <= 2 * cu;
+    const long long ks = split_count_i8(a, 128, 128, (int)cu);
+    const bool fours = !(a.N % 4 || (a.y2 && a.N2 % 4) || (a.y3 && a.N3 % 4));
+    if (ks > 5 && !fours && precision != KH_Q4K) return false;
+    return ks >= 2 && stages >= 13 * ks && 4 * t * ks >= 7 * cu && t * ks <= 2 * cu && split_partials(ctx, 0);
 }
-Shape pick_shape(int M, int N, int K, int cu) {
+Shape pick_shape(kh_ctx *ctx, int precision, const GemmArgs &a) {
     const int forced = env_int("KVAD_GEMM_TILE_M", 0);  // tuning knob: tokens per tile (6464: 64 x 64)
     if (forced == 6464) return T64x64;
     if (forced == 128 || forced == 64 || forced == 32) return forced == 128 ? T128x128 : forced == 64 ? T128x64 : T128x32;
-    const long long nt = (N + 127) / 128;
+    const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256, M = a.M;
+    const long long nt = row_tiles(a, 128);
     // 128 x 128 tiles while they give four workgroups per CU, or fill their
     // rounds of the chip; else, past 64 tokens, 64 x 64 tiles: more, smaller workgroups hide the k-stages' load
     // latency ((512, 896, 4864) 28.5 -> 27.4 us against 128-row 32-token tiles,
@@ -736,7 +785,7 @@ Shape pick_shape(int M, int N, int K, int cu) {
     // tokens (a vocabulary head) gives enough workgroups with 32-token
     // tiles, and 128-token ones would leave three quarters of every tile idle.
     if (M > 64 && nt * ((M + 127) / 128) >= 4LL * cu) return T128x128;
-    if (fills_rounds(M, N, K, cu)) return T128x128;
+    if (fills_rounds(ctx, precision, a, cu)) return T128x128;
     if (M > 64 && M < 128 && nt >= cu) return T128x128;
     if (M > 64) return T64x64;
     if (M > 32 && nt >= cu) return T128x64;
@@ -745,20 +794,13 @@ Shape pick_shape(int M, int N, int K, int cu) {
 
 }  // namespace
 
-int gemm_tiles(kh_ctx *ctx, int M, int N, int K, int *tile_n) {
-    const Shape sh = pick_shape(M, N, K, ctx->cu_count > 0 ? ctx->cu_count : 256);
+int gemm_tiles(kh_ctx *ctx, int precision, const GemmArgs &a, int *tile_n) {
+    const Shape sh = pick_shape(ctx, precision, a);
     *tile_n = sh == T64x64 ? 64 : 128;
     return sh == T128x128 ? 128 : sh == T128x32 ? 32 : 64;
 }
 
 namespace {
-
-// Rows of every weight of a launch, and their tiles.
-long long all_rows(const GemmArgs &a) { return (long long)a.N + (a.y2 ? a.N2 : 0) + (a.y3 ? a.N3 : 0); }
-long long row_tiles(const GemmArgs &a, int tile_n) {
-    auto tiles = [&](int n) { return ((long long)n + tile_n - 1) / tile_n; };
-    return tiles(a.N) + (a.y2 ? tiles(a.N2) : 0) + (a.y3 ? tiles(a.N3) : 0);
-}
 
 template <int PREC>
 int launch_i8(kh_ctx *ctx, const GemmArgs &a, int max_tiles, int tile_m, int tile_n) {
@@ -857,12 +899,6 @@ namespace {
 bool matmul_force_gemm() { return env_int("KVAD_MATMUL_GEMM", 0) == 1; }
 }  // namespace
 
-namespace {
-const int SPLIT_MIN_STAGES = env_int("KVAD_GEMM_SPLIT_MIN", 2);  // tuning knobs
-const int SPLIT_MAX = env_int("KVAD_GEMM_SPLIT_MAX", 32);
-const int SPLIT_PER_CU = env_int("KVAD_GEMM_SPLIT_PER_CU", 2);
-}  // namespace
-
 int gemm_split_reserve(kh_ctx *ctx) {
     if (ctx->gemm.ptr) return KH_OK;
     KH_HIP(hipMalloc(&ctx->gemm.ptr, SPLIT_BYTES));
@@ -889,28 +925,9 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
 
 namespace {
 
-// Sets a's split-K fields: the k-stages (`stages` of them, at least `min_st`
-// a split, none under `least`) are split so that the grid comes to about
-// SPLIT_PER_CU workgroups per CU (a CU holds several: one's loads wait while
-// another's MFMAs run), at most SPLIT_MAX splits, and partials (4 M N bytes a
-// split, written and read again) of at most the weights' wbytes or 4 MiB,
-// whichever is more (a small weight such as a router's 64 rows would otherwise
-// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); twice
-// that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
-// 4096) 36.3 -> 27.5 us in four splits instead of two, (512, 896, 4864) 27.5 ->
-// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two).
-int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st, int least, size_t wbytes) {
+// Sets a's split-K fields for ks splits, none under two or without a workspace.
+int set_split(kh_ctx *ctx, GemmArgs &a, long long ks) {
     a.ksplit = 0;
-    const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const size_t plane = (size_t)a.M * all_rows(a) * 4;
-    const size_t most = std::max(wbytes, (size_t)4 << 20) * (2 * tiles <= cu ? 2 : 1);
-    long long ks = stages < least ? 1 : ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
-    ks = std::min<long long>(ks, stages / min_st);
-    ks = std::min<long long>(ks, SPLIT_MAX);
-    ks = std::min<long long>(ks, (long long)(most / plane));
-    const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
-    if (forced > 0) ks = std::min(forced, stages);
-    ks = std::min<long long>(ks, (long long)(SPLIT_BYTES / plane));
     if (ks < 2) return KH_OK;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     KH_HIP(hipStreamIsCapturing(ctx->stream, &cap));
@@ -932,7 +949,8 @@ int set_split(kh_ctx *ctx, GemmArgs &a, long long tiles, int stages, int min_st,
 // 126 -> 11.5; 512x512 at 16 15.7 -> 6.9 (at least four stages 8.5, eight 11.7).
 int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
     const long long tiles = (long long)((a.N + 127) / 128) * ((a.M + tile_m - 1) / tile_m);
-    return set_split(ctx, a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4);
+    const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    return set_split(ctx, a, split_count(a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4, cu));
 }
 
 }  // namespace
@@ -940,11 +958,7 @@ int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
 int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
     a.ksplit = 0;
     if (a.tiles) return KH_OK;  // grouped launches are not split
-    // Under twelve stages of 128 the second launch costs more than the shorter
-    // chains save: (512 tokens, 896 rows, 896) 14.1 us in two splits, 11.2
-    // unsplit, (80, 4864, 896) 14.0 and 10.9.
-    return set_split(ctx, a, row_tiles(a, tile_n) * ((a.M + tile_m - 1) / tile_m), (a.K + BK - 1) / BK,
-                     SPLIT_MIN_STAGES, 12, (size_t)all_rows(a) * a.K);
+    return set_split(ctx, a, split_count_i8(a, tile_m, tile_n, ctx->cu_count > 0 ? ctx->cu_count : 256));
 }
 
 int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y,
@@ -1008,9 +1022,8 @@ int launch_matmul_q(kh_ctx *ctx, const kh_weight *w, const QAct &q, size_t m, co
     a.xq = q.qs;
     a.xs = q.scales;
     a.xsum = q.sums;
-    const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const Shape sh = pick_shape(a.M, a.N, a.K, cu);
-    const int tile_m = sh == T128x128 ? 128 : sh == T128x32 ? 32 : 64, tile_n = sh == T64x64 ? 64 : 128;
+    int tile_n;
+    const int tile_m = gemm_tiles(ctx, w->precision, a, &tile_n);
     int rc = plan_split(ctx, a, tile_m, tile_n);
     if (rc) return rc;
     return launch_gemm_q(ctx, w->precision, a, 0, tile_m, tile_n);
@@ -1047,7 +1060,7 @@ int launch_matmul_jobs(kh_ctx *ctx, int k, const kh_weight *const *w, const QAct
     a.w2 = w[1]->qs, a.ws2 = w[1]->scales, a.bias2 = bias[1], a.y2 = y[1], a.N2 = (int)w[1]->rows;
     if (k == 3) a.w3 = w[2]->qs, a.ws3 = w[2]->scales, a.bias3 = bias[2], a.y3 = y[2], a.N3 = (int)w[2]->rows;
     int tn;
-    const int tm = gemm_tiles(ctx, a.M, (int)rows, a.K, &tn);
+    const int tm = gemm_tiles(ctx, w[0]->precision, a, &tn);
     const int rc = plan_split(ctx, a, tm, tn);
     return rc ? rc : launch_gemm_q(ctx, w[0]->precision, a, 0, tm, tn);
 }

@@ -441,18 +441,21 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     GemmArgs a{};
     a.xq = xq.qs, a.xs = xq.scales, a.xsum = xq.sums;
     a.M = (int)m, a.K = (int)gate->cols;
-    int tn;
-    const int tm = gemm_tiles(ctx, (int)m, (int)gate->rows, (int)gate->cols, &tn);
-    int rc;
+    int tn, rc;
+    auto launch = [&](const kh_weight *w) {
+        const int tm = gemm_tiles(ctx, w->precision, a, &tn);
+        if ((rc = plan_split(ctx, a, tm, tn))) return rc;
+        return launch_gemm_q(ctx, w->precision, a, 0, tm, tn);
+    };
     a.w = gate->qs, a.ws = gate->scales, a.N = (int)gate->rows, a.y = g;
     if (gate->precision == up->precision && gate->rows == up->rows && gate->cols == up->cols) {
         // gate and up in one launch over the same activation tiles
         a.w2 = up->qs, a.ws2 = up->scales, a.y2 = u, a.N2 = a.N;
-        if ((rc = plan_split(ctx, a, tm, tn)) || (rc = launch_gemm_q(ctx, gate->precision, a, 0, tm, tn))) return rc;
+        if ((rc = launch(gate))) return rc;
     } else {
-        if ((rc = plan_split(ctx, a, tm, tn)) || (rc = launch_gemm_q(ctx, gate->precision, a, 0, tm, tn))) return rc;
+        if ((rc = launch(gate))) return rc;
         a.w = up->qs, a.ws = up->scales, a.N = (int)up->rows, a.y = u;
-        if ((rc = plan_split(ctx, a, tm, tn)) || (rc = launch_gemm_q(ctx, up->precision, a, 0, tm, tn))) return rc;
+        if ((rc = launch(up))) return rc;
     }
     if ((rc = launch_swiglu_qact(ctx, g, u, m, gate->rows, hq))) return rc;
     GemmArgs d{};
@@ -460,7 +463,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     d.M = (int)m, d.K = (int)down->cols, d.N = (int)down->rows;
     d.w = down->qs, d.ws = down->scales, d.y = y;
     int tdn;
-    const int td = gemm_tiles(ctx, (int)m, (int)down->rows, (int)down->cols, &tdn);
+    const int td = gemm_tiles(ctx, down->precision, d, &tdn);
     if ((rc = plan_split(ctx, d, td, tdn))) return rc;
     return launch_gemm_q(ctx, down->precision, d, 0, td, tdn);
 }

@@ -292,3 +292,29 @@ def test_tiles_that_fill_rounds(ctx, prec, rows, cols, m):
     want = oracle_matmul(prec, sub, len(r_idx), cols, xs.reshape(m, cols)[t_idx].ravel(), len(t_idx))
     close(got[np.ix_(t_idx, r_idx)], want.reshape(len(t_idx), len(r_idx)))
     assert np.all(np.isfinite(got))
+
+
+@pytest.mark.parametrize("m,rows,cols,tile", [(896, 1408, 12544, "6464"), (1071, 908, 15904, "128"),
+                                              (574, 1082, 18528, "6464")])
+def test_tile_rule_knows_the_split(ctx, monkeypatch, m, rows, cols, tile):
+    # 128 x 128 tiles are taken for a split that fills a round of the chip only
+    # where the launch is then split that way: 77 tiles in seven splits are 27
+    # workgroups past a round of 512 (64 x 64 tiles, in two splits), 72 in seven
+    # are 504; 45 in eleven of rows that are no multiple of four store their
+    # partials value by value.  A split's sums have their own order, so the bits
+    # show it.
+    say("matmul tile rule", m, rows, cols)
+    rng = np.random.default_rng(rows)
+    q = rng.integers(-127, 128, rows * cols, dtype=np.int8)
+    sc = rng.uniform(1e-4, 3e-4, rows * cols // 32).astype(np.float32)
+    w = K.Weight.from_q8(ctx, rows, cols, sc, q)
+    xs = rng.standard_normal(m * cols, dtype=np.float32)
+    got = w.matmul_bt(xs, m)
+    monkeypatch.setenv("KVAD_GEMM_TILE_M", tile)
+    np.testing.assert_array_equal(w.matmul_bt(xs, m), got)
+    monkeypatch.setenv("KVAD_GEMM_TILE_M", "128" if tile == "6464" else "6464")
+    assert not np.array_equal(w.matmul_bt(xs, m), got)
+    r_idx, t_idx = np.r_[0:4, rows - 4:rows], np.r_[0:4, m - 4:m]
+    sub = tuple(np.ascontiguousarray(p.reshape(rows, -1)[r_idx]).ravel() for p in (sc, q))
+    want = oracle_matmul("q8", sub, len(r_idx), cols, xs.reshape(m, cols)[t_idx].ravel(), len(t_idx))
+    close(got.reshape(m, rows)[np.ix_(t_idx, r_idx)], want.reshape(len(t_idx), len(r_idx)))
