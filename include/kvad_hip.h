@@ -67,8 +67,10 @@ int kh_free(kh_ctx *ctx);
  * restores the own stream.  The caller keeps ownership of the stream. */
 int kh_set_stream(kh_ctx *ctx, void *hip_stream);
 int kh_synchronize(kh_ctx *ctx);
-/* Grow the context's device scratch to `bytes` up front, so that later calls
- * do not allocate. */
+/* Grow the context's device scratch to `bytes` up front, and make its fixed
+ * workspace for split matmuls (64 MiB), so that later calls do not allocate.
+ * Without that workspace (no room, or a first call under graph capture)
+ * matmuls run unsplit. */
 int kh_reserve(kh_ctx *ctx, size_t bytes);
 
 /* ---- weights ---------------------------------------------------------- */

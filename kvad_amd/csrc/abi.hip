@@ -224,6 +224,7 @@ int kh_synchronize(kh_ctx *ctx) {
 int kh_reserve(kh_ctx *ctx, size_t bytes) {
     if (!ctx) return fail(KH_EINVAL, "null context");
     Guard g(ctx);
+    gemm_split_reserve(ctx);
     return ensure(ctx, ctx->ws, bytes);
 }
 

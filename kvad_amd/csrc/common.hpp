@@ -352,9 +352,9 @@ struct GemmArgs {
 };
 // tile_n: weight rows per tile (128, or 64 with 64-token tiles, ungrouped)
 int launch_gemm_q(kh_ctx *ctx, int precision, const GemmArgs &a, int max_tiles, int tile_m, int tile_n = 128);
-// Allocates the split-K workspace now (a GEMM captured into a graph splits
-// only when it was allocated before the capture).
-int gemm_split_reserve(kh_ctx *ctx);
+// Allocates the split-K workspace now, if the device has room for it (a GEMM
+// captured into a graph splits only when it was allocated before the capture).
+void gemm_split_reserve(kh_ctx *ctx);
 // The split-K workspace for `bytes` of partials, or null where it does not
 // hold them (or was not allocated before a capture).
 float *split_partials(kh_ctx *ctx, size_t bytes);
@@ -363,7 +363,7 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
                         float *y);
 // Sets a's split-K fields for an ungrouped launch of tile_m-token tiles when
 // splitting its k-stages pays (ksplit 0: no split).
-int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n = 128);
+void plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n = 128);
 // Tokens per tile (returned) and weight rows per tile (*tile_n) for an
 // ungrouped launch of the int8 GEMM over a's weights.
 int gemm_tiles(kh_ctx *ctx, int precision, const GemmArgs &a, int *tile_n);

@@ -692,8 +692,9 @@ enum Shape { T128x128, T128x64, T128x32, T64x64 };
 
 // The split-K workspace: one fixed allocation for the partials, made on the
 // first split launch and never moved, so graphs captured over later launches
-// stay valid; a split whose partials do not fit is cut to what fits.
-constexpr size_t SPLIT_BYTES = 64u << 20;
+// stay valid; a split whose partials do not fit is cut to what fits, and where
+// the device has no room for it nothing is split.
+size_t split_bytes() { return (size_t)env_int("KVAD_GEMM_SPLIT_MIB", 64) << 20; }  // tuning knob (0: no splits)
 
 const int SPLIT_MIN_STAGES = env_int("KVAD_GEMM_SPLIT_MIN", 2);  // tuning knobs
 const int SPLIT_MAX = env_int("KVAD_GEMM_SPLIT_MAX", 32);
@@ -729,7 +730,7 @@ long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st
     ks = std::min<long long>(ks, (long long)(most / plane));
     const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
     if (forced > 0) ks = std::min(forced, stages);
-    return std::min<long long>(ks, (long long)(SPLIT_BYTES / plane));
+    return std::min<long long>(ks, (long long)(split_bytes() / plane));
 }
 // The int8 GEMM's, in tiles of tile_m tokens by tile_n rows.
 long long split_count_i8(const GemmArgs &a, int tile_m, int tile_n, int cu) {
@@ -837,7 +838,7 @@ int launch_i8(kh_ctx *ctx, const GemmArgs &a, int max_tiles, int tile_m, int til
     return KH_OK;
 }
 
-int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m);
+void plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m);
 
 // The f32 GEMM runs best on shorter token tiles than the int8 one (swept at
 // both prefill shapes): 64 tokens while that still gives two workgroups per
@@ -853,8 +854,7 @@ int launch_f32gemm(kh_ctx *ctx, GemmArgs a) {
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const Shape sh = pick_shape_f32(a.M, a.N, cu);
     const int tile_m = sh == T128x128 ? 128 : sh == T128x64 ? 64 : 32;
-    const int rc = plan_split_f32(ctx, a, tile_m);
-    if (rc) return rc;
+    plan_split_f32(ctx, a, tile_m);
     const dim3 grid((unsigned)((a.N + 127) / 128), (unsigned)((a.M + tile_m - 1) / tile_m),
                     a.ksplit > 1 ? (unsigned)a.ksplit : 1u);
     switch (sh) {
@@ -899,19 +899,24 @@ namespace {
 bool matmul_force_gemm() { return env_int("KVAD_MATMUL_GEMM", 0) == 1; }
 }  // namespace
 
-int gemm_split_reserve(kh_ctx *ctx) {
-    if (ctx->gemm.ptr) return KH_OK;
-    KH_HIP(hipMalloc(&ctx->gemm.ptr, SPLIT_BYTES));
-    ctx->gemm.bytes = SPLIT_BYTES;
-    return KH_OK;
+void gemm_split_reserve(kh_ctx *ctx) {
+    if (ctx->gemm.ptr || !split_bytes()) return;
+    if (hipMalloc(&ctx->gemm.ptr, split_bytes()) == hipSuccess) {
+        ctx->gemm.bytes = split_bytes();
+    } else {
+        ctx->gemm.ptr = nullptr;
+        (void)hipGetLastError();  // the unsplit launch's check must not find it
+    }
 }
 
 float *split_partials(kh_ctx *ctx, size_t bytes) {
-    if (bytes > SPLIT_BYTES) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) return nullptr;
-    if (cap == hipStreamCaptureStatusNone && gemm_split_reserve(ctx) != KH_OK) return nullptr;  // no allocation under capture
-    return static_cast<float *>(ctx->gemm.ptr);
+    if (!ctx->gemm.ptr) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) return nullptr;
+        if (cap != hipStreamCaptureStatusNone) return nullptr;  // no allocation under capture
+        gemm_split_reserve(ctx);
+    }
+    return bytes <= ctx->gemm.bytes ? static_cast<float *>(ctx->gemm.ptr) : nullptr;
 }
 
 int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, const float *bias, int accumulate,
@@ -926,19 +931,11 @@ int launch_split_reduce(kh_ctx *ctx, const float *part, int ks, int M, int N, co
 namespace {
 
 // Sets a's split-K fields for ks splits, none under two or without a workspace.
-int set_split(kh_ctx *ctx, GemmArgs &a, long long ks) {
+void set_split(kh_ctx *ctx, GemmArgs &a, long long ks) {
     a.ksplit = 0;
-    if (ks < 2) return KH_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    KH_HIP(hipStreamIsCapturing(ctx->stream, &cap));
-    if (cap == hipStreamCaptureStatusNone) {  // no allocation under capture
-        const int rc = gemm_split_reserve(ctx);
-        if (rc) return rc;
-    }
-    if (!ctx->gemm.ptr) return KH_OK;
-    a.ksplit = (int)ks;
-    a.part = static_cast<float *>(ctx->gemm.ptr);
-    return KH_OK;
+    if (ks < 2) return;
+    a.part = split_partials(ctx, (size_t)ks * a.M * all_rows(a) * 4);
+    if (a.part) a.ksplit = (int)ks;
 }
 
 // The f32 GEMM's split, at least two stages of 32 k-values each.  A few
@@ -947,18 +944,18 @@ int set_split(kh_ctx *ctx, GemmArgs &a, long long ks) {
 // workgroups of 65 stages, 56 -> 22 us; 4096x4096 at 2 / 32 / 128 tokens 114 ->
 // 20 / 21 / 50; a 64x2048 router at 4 / 512 54 -> 6.3 / 10.8; 896x4864 at 16
 // 126 -> 11.5; 512x512 at 16 15.7 -> 6.9 (at least four stages 8.5, eight 11.7).
-int plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
+void plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
     const long long tiles = (long long)((a.N + 127) / 128) * ((a.M + tile_m - 1) / tile_m);
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    return set_split(ctx, a, split_count(a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4, cu));
+    set_split(ctx, a, split_count(a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4, cu));
 }
 
 }  // namespace
 
-int plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
+void plan_split(kh_ctx *ctx, GemmArgs &a, int tile_m, int tile_n) {
     a.ksplit = 0;
-    if (a.tiles) return KH_OK;  // grouped launches are not split
-    return set_split(ctx, a, split_count_i8(a, tile_m, tile_n, ctx->cu_count > 0 ? ctx->cu_count : 256));
+    if (a.tiles) return;  // grouped launches are not split
+    set_split(ctx, a, split_count_i8(a, tile_m, tile_n, ctx->cu_count > 0 ? ctx->cu_count : 256));
 }
 
 int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y,
@@ -1024,8 +1021,7 @@ int launch_matmul_q(kh_ctx *ctx, const kh_weight *w, const QAct &q, size_t m, co
     a.xsum = q.sums;
     int tile_n;
     const int tile_m = gemm_tiles(ctx, w->precision, a, &tile_n);
-    int rc = plan_split(ctx, a, tile_m, tile_n);
-    if (rc) return rc;
+    plan_split(ctx, a, tile_m, tile_n);
     return launch_gemm_q(ctx, w->precision, a, 0, tile_m, tile_n);
 }
 
@@ -1061,8 +1057,8 @@ int launch_matmul_jobs(kh_ctx *ctx, int k, const kh_weight *const *w, const QAct
     if (k == 3) a.w3 = w[2]->qs, a.ws3 = w[2]->scales, a.bias3 = bias[2], a.y3 = y[2], a.N3 = (int)w[2]->rows;
     int tn;
     const int tm = gemm_tiles(ctx, w[0]->precision, a, &tn);
-    const int rc = plan_split(ctx, a, tm, tn);
-    return rc ? rc : launch_gemm_q(ctx, w[0]->precision, a, 0, tm, tn);
+    plan_split(ctx, a, tm, tn);
+    return launch_gemm_q(ctx, w[0]->precision, a, 0, tm, tn);
 }
 
 }  // namespace kh

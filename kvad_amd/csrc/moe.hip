@@ -444,7 +444,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     int tn, rc;
     auto launch = [&](const kh_weight *w) {
         const int tm = gemm_tiles(ctx, w->precision, a, &tn);
-        if ((rc = plan_split(ctx, a, tm, tn))) return rc;
+        plan_split(ctx, a, tm, tn);
         return launch_gemm_q(ctx, w->precision, a, 0, tm, tn);
     };
     a.w = gate->qs, a.ws = gate->scales, a.N = (int)gate->rows, a.y = g;
@@ -464,7 +464,7 @@ int ffn_rows(kh_ctx *ctx, const kh_weight *gate, const kh_weight *up, const kh_w
     d.w = down->qs, d.ws = down->scales, d.y = y;
     int tdn;
     const int td = gemm_tiles(ctx, down->precision, d, &tdn);
-    if ((rc = plan_split(ctx, d, td, tdn))) return rc;
+    plan_split(ctx, d, td, tdn);
     return launch_gemm_q(ctx, down->precision, d, 0, td, tdn);
 }
 

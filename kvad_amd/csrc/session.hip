@@ -820,7 +820,7 @@ int run_pass(kh_ctx *ctx, kh_llm *m, const int32_t *tokens, size_t n, const kh_l
         const std::pair<size_t, size_t> key{n, bm};
         auto it = m->pass_graphs.find(key);
         if (it == m->pass_graphs.end()) {
-            if ((rc = gemm_split_reserve(ctx))) return rc;
+            gemm_split_reserve(ctx);
             KH_HIP(hipStreamSynchronize(ctx->stream));
             hipGraph_t g = nullptr;
             KH_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
@@ -1264,7 +1264,7 @@ int kh_llm_forward_each(kh_ctx *ctx, kh_llm *m, size_t n, const int32_t *tokens,
     const std::pair<size_t, size_t> key{n, bm};
     auto it = m->rows_graphs.find(key);
     if (it == m->rows_graphs.end()) {
-        if ((rc = gemm_split_reserve(ctx))) return rc;
+        gemm_split_reserve(ctx);
         KH_HIP(hipStreamSynchronize(ctx->stream));
         hipGraph_t g = nullptr;
         KH_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));

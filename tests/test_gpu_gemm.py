@@ -318,3 +318,38 @@ def test_tile_rule_knows_the_split(ctx, monkeypatch, m, rows, cols, tile):
     sub = tuple(np.ascontiguousarray(p.reshape(rows, -1)[r_idx]).ravel() for p in (sc, q))
     want = oracle_matmul("q8", sub, len(r_idx), cols, xs.reshape(m, cols)[t_idx].ravel(), len(t_idx))
     close(got.reshape(m, rows)[np.ix_(t_idx, r_idx)], want.reshape(len(t_idx), len(r_idx)))
+
+
+@pytest.mark.parametrize("mib", ["0", str(1 << 30)])
+def test_matmuls_run_unsplit_without_a_split_workspace(ctx, monkeypatch, mib):
+    # a context that makes no workspace for partials, or has no room for it (a
+    # pebibyte): what would have been split runs unsplit, and the allocation's
+    # error is not reported by the launch after it.  f32, the int8 GEMM, and
+    # the few-row kernel past 16 rows of a width its registers do not hold.
+    c = K.Context(0)
+    try:
+        for prec, m, rows, cols in [("f32", 90, 300, 2052), ("q8", 100, 257, 2048), ("q8", 40, 70, 2080 * 2),
+                                    ("q4", 33, 70, 4128), ("q4k", 40, 70, 8448), ("q8", 512, 4096, 14336)]:
+            say("matmul without a split workspace", mib, prec, m, rows, cols)
+            monkeypatch.setenv("KVAD_MULTI_TOKENS", "64" if 16 < m <= 64 else "")
+            if rows * cols > 1 << 24:  # 128 x 128 tiles if split: the tile rule asks for the workspace
+                rng = np.random.default_rng(9)
+                parts = (rng.uniform(1e-4, 3e-4, rows * cols // 32).astype(np.float32),
+                         rng.integers(-127, 128, rows * cols, dtype=np.int8))
+                w = K.Weight.from_q8(c, rows, cols, *parts)
+                r_idx, t_idx = np.r_[0:4, rows - 4:rows], np.r_[0:4, m - 4:m]
+            else:
+                w, parts = make(c, prec, rows, cols, seed=rows + cols)
+                r_idx, t_idx = np.arange(rows), np.arange(m)
+            xs = O.normal(m + cols, m * cols) if m < 512 else rng.standard_normal(m * cols, dtype=np.float32)
+            bias = O.normal(rows + 1, rows)
+            monkeypatch.setenv("KVAD_GEMM_SPLIT_MIB", mib)
+            got = w.matmul_bt(xs, m, bias).reshape(m, rows)
+            monkeypatch.delenv("KVAD_GEMM_SPLIT_MIB")
+            sub = tuple(np.ascontiguousarray(np.asarray(p).reshape(rows, -1)[r_idx]).ravel() for p in parts)
+            want = oracle_matmul(prec, sub, len(r_idx), cols, np.ascontiguousarray(xs.reshape(m, cols)[t_idx]).ravel(),
+                                 len(t_idx), bias[r_idx])
+            close(got[np.ix_(t_idx, r_idx)], want.reshape(len(t_idx), len(r_idx)))
+            del w
+    finally:
+        c.close()
