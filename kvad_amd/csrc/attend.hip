@@ -1775,7 +1775,7 @@ namespace {
 
 constexpr int MLA_LAT = 512, MLA_ROPE = 64, MLA_K = MLA_LAT + MLA_ROPE;
 constexpr int MLA_QSTR = MLA_K + 4;  // LDS row stride (floats) of the staged queries
-constexpr int MLA_ONE = 32;          // the longest sequence taken in one launch
+constexpr int MLA_ONE = 32;          // the longest sequence taken in one launch (captured, twice as long)
 // dims per merge workgroup: 128 (four per head) for a few splits, 64 from
 // 64 splits on, where each workgroup's partials are what it waits for
 // (measured at L = 1024 / 8192 / 32768: 18.9 / 24.6 / 44.2 us per layer at
@@ -2140,14 +2140,16 @@ int launch_mla(kh_ctx *ctx, int n_head, const float *q_lat, const float *q_pe, c
     a.n_head = n_head;
     a.L = (int)n_positions;
     // One launch up to MLA_ONE positions (11.5 us; 33 to 64 took 12.9 there,
-    // 11.6 as two splits and a merge); past that splits of 32, 64 or 128
+    // 11.6 as two splits and a merge, but under capture one launch, which needs
+    // no scratch for partials); past that splits of 32, 64 or 128
     // positions, the least that keeps to a workgroup a CU (16 heads over 20000
     // positions 28.7 us in 157 splits, 34.7 in 313), 256 where 128 make more than
     // two.  A power of two: the merge reads 256 scores at a time.
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const int hg = (n_head + 15) / 16;
     const int forced = env_int("KVAD_MLA_SPLIT", 0);  // tuning knob: positions per split (32 / 64 / 128 / 256)
-    const bool one = n_positions <= (size_t)MLA_ONE && forced == 0;
+    const bool one = forced == 0 && (n_positions <= (size_t)MLA_ONE ||
+                                     (n_positions <= (size_t)2 * MLA_ONE && capturing(ctx->stream)));
     a.P = one ? 64 : forced == 64 || forced == 128 || forced == 256 ? forced : MLA_TILE;
     auto wgs = [&] { return (long long)((n_positions + a.P - 1) / a.P) * hg; };
     if (!forced && !one) {

@@ -32,6 +32,14 @@ int hip_fail(hipError_t e, const char *what);
         if (e_ != hipSuccess) return ::kh::hip_fail(e_, #call); \
     } while (0)
 
+// Whether work on the stream goes into a graph that is being captured: calls
+// that can do without the context's scratch take none then (it cannot be made
+// or grown under capture, and may move before a replay).
+inline bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
 // A launch-shape tuning knob from the environment (dflt when unset).
 inline int env_int(const char *name, int dflt) {
     const char *v = getenv(name);
@@ -286,6 +294,8 @@ inline unsigned multi_firsts(int njobs, int g1, int g2) {
 // (quantising them in every workgroup) rather than read codes quantised once
 // by a launch of their own: only while the stage is small.
 bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols);
+// Whether the VALU multi-token GEMV does, whichever kernel is ahead.
+bool valu_stages_f32(size_t m, size_t cols);
 // Whether the multi-token GEMV over `rows` weight rows in all runs on the
 // matrix cores (launch_gemv_mma) when it is given codes.
 bool mma_takes(size_t m, size_t rows, size_t cols);

@@ -911,9 +911,7 @@ void gemm_split_reserve(kh_ctx *ctx) {
 
 float *split_partials(kh_ctx *ctx, size_t bytes) {
     if (!ctx->gemm.ptr) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) return nullptr;
-        if (cap != hipStreamCaptureStatusNone) return nullptr;  // no allocation under capture
+        if (capturing(ctx->stream)) return nullptr;
         gemm_split_reserve(ctx);
     }
     return bytes <= ctx->gemm.bytes ? static_cast<float *>(ctx->gemm.ptr) : nullptr;
@@ -985,7 +983,8 @@ int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, co
     // a few rows: the VALU multi-token GEMV quantises them as it stages them
     // (QActBatch::new's codes, one launch fewer) while they are few values
     const bool multi = matmul_takes_multi(w->precision, m, rows, cols) && !matmul_force_gemm();
-    if (multi && multi_stages_f32(w->precision, m, rows, cols))
+    if (multi && (multi_stages_f32(w->precision, m, rows, cols) ||
+                  (m <= 4 && valu_stages_f32(m, cols) && capturing(ctx->stream))))  // no scratch for the codes
         return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, &accumulate, QAct{}, m, xs);
     // QActBatch::new (quant.rs:693-714): the activation rows quantised per block
     const size_t qb = (m * cols + 255) / 256 * 256, sb = (4 * m * cols / BLOCK + 255) / 256 * 256;

@@ -1267,11 +1267,15 @@ int launch_gemv_multi(kh_ctx *ctx, const kh_weight *w, const QAct &x, size_t m, 
 }
 
 bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols) {
+    // The matrix-core kernel takes the rows' codes.
+    return !(mma_takes(m, rows, cols) && mma_addresses(precision, rows, cols)) && valu_stages_f32(m, cols);
+}
+
+bool valu_stages_f32(size_t m, size_t cols) {
     // Every workgroup quantises its token slots' rows (2, 4 or 8 slots); past
     // about 12K values that costs more than a quantising launch of its own
     // plus a stage of codes (measured over q8 and Q4_K weights of 896 to
-    // 14336 columns at m = 2..8).  The matrix-core kernel takes the rows' codes.
-    if (mma_takes(m, rows, cols) && mma_addresses(precision, rows, cols)) return false;
+    // 14336 columns at m = 2..8).
     const size_t slots = m <= 2 ? 2 : m <= 4 ? 4 : 8;
     const int lim = env_int("KVAD_MULTI_STAGE_F32", 12288);  // tuning knob
     return slots * cols <= (size_t)lim;

@@ -1,7 +1,8 @@
 """The attention entry point that allocates nothing (kh_attend_dev_noalloc):
 its output equals kh_attend_dev's, bit for bit, on two calls in a row, the
 second with a smaller input; a call whose partials exceed the library's
-static scratch array is refused with a clear error."""
+static scratch array is refused with a clear error.  And calls that need no
+scratch of their context, captured into a graph on one that has made none."""
 import numpy as np
 import pytest
 
@@ -70,3 +71,92 @@ def test_noalloc_attention_refuses_what_exceeds_the_scratch(ctx):
     rc = run(ctx, K.lib.kh_attend_dev_noalloc, n_head, n_kv, hd, q, k, v, L, out)
     assert rc == -1  # KH_EINVAL
     assert b"bytes of scratch" in K.lib.kh_last_error()
+
+
+def captured(ctx, call):
+    """The call captured into a graph on a stream of its own, on a context
+    that has made no scratch yet."""
+    import torch
+
+    stream = torch.cuda.Stream()
+    ctx.set_stream(stream.cuda_stream)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=stream):
+        call()
+    return g, stream
+
+
+def replays_match(ctx, g, stream, out, want, tol):
+    """Several replays, the context's own eager work between them: a matmul
+    whose scratch grows past what was there, so that whatever the graph still
+    named would have moved."""
+    import torch
+
+    for i in range(4):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            g.replay()
+        torch.cuda.synchronize()
+        err = float((out - want).abs().max())
+        assert err <= tol * float(want.abs().max()), (i, err)
+        x = torch.randn((1 << i) * 500, 2048, device="cuda")
+        d, y = torch.randn(64, 2048, device="cuda"), torch.empty(x.shape[0], 64, device="cuda")
+        torch.cuda.synchronize()
+        w = K.Weight.quantize_dev(ctx, 64, 2048, d.data_ptr(), K.Q8)
+        w.matmul_bt_dev(x.data_ptr(), x.shape[0], y.data_ptr())
+        ctx.synchronize()
+
+
+@pytest.mark.parametrize("L", [20, 33, 64])
+def test_latent_attention_of_one_launch_is_captured_without_scratch(ctx, L):
+    import torch
+
+    say("mla under capture", L)
+    H = 16
+    g = torch.Generator(device="cuda")
+    g.manual_seed(L)
+    ql, qp, c, pe = (torch.randn(*s, device="cuda", generator=g) for s in ((H, 512), (H, 64), (L, 512), (L, 64)))
+    want, out = torch.empty(H, 512, device="cuda"), torch.empty(H, 512, device="cuda")
+
+    def call(cx, o):
+        K.mla_attend_dev(cx, H, ql.data_ptr(), qp.data_ptr(), c.data_ptr(), pe.data_ptr(), L, 192.0 ** -0.5, o.data_ptr())
+
+    torch.cuda.synchronize()
+    call(ctx, want)
+    ctx.synchronize()
+    fresh = K.Context(0)
+    try:
+        graph, stream = captured(fresh, lambda: call(fresh, out))
+        replays_match(fresh, graph, stream, out, want, 1e-5)
+    finally:
+        fresh.set_stream(None)
+        fresh.close()
+
+
+@pytest.mark.parametrize("prec,m,rows,cols", [("q8", 2, 65536, 256), ("q8", 3, 8960, 1536), ("q4", 4, 4096, 3072)])
+def test_few_rows_are_captured_without_scratch(ctx, prec, m, rows, cols):
+    import torch
+
+    say("matmul under capture", prec, m, rows, cols)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    data = torch.randn(rows, cols, device="cuda", generator=g) * 0.02
+    x = torch.randn(m, cols, device="cuda", generator=g)
+    want, out = torch.empty(m, rows, device="cuda"), torch.empty(m, rows, device="cuda")
+    torch.cuda.synchronize()
+    fresh = K.Context(0)
+    try:
+        for cx, o in ((ctx, want), (fresh, out)):
+            w = K.Weight.quantize_dev(cx, rows, cols, data.data_ptr(), K.Q8 if prec == "q8" else K.Q4)
+            cx.synchronize()
+            call = lambda: w.matmul_bt_dev(x.data_ptr(), m, o.data_ptr())  # noqa: E731
+            if cx is ctx:
+                call()
+                cx.synchronize()
+        graph, stream = captured(fresh, call)
+        replays_match(fresh, graph, stream, out, want, 1e-5)
+    finally:
+        fresh.set_stream(None)
+        fresh.close()
