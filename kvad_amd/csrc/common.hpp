@@ -294,11 +294,9 @@ inline unsigned multi_firsts(int njobs, int g1, int g2) {
 // (quantising them in every workgroup) rather than read codes quantised once
 // by a launch of their own: only while the stage is small.
 bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols);
-// Whether the VALU multi-token GEMV does, whichever kernel is ahead.
-bool valu_stages_f32(size_t m, size_t cols);
 // Whether the multi-token GEMV over `rows` weight rows in all runs on the
 // matrix cores (launch_gemv_mma) when it is given codes.
-bool mma_takes(size_t m, size_t rows, size_t cols);
+bool mma_takes(size_t m, size_t rows);
 // Whether the matrix-core multi-token GEMV addresses a weight (32-bit buffer
 // offsets for its rows, its scales and 32 tokens' outputs).
 bool mma_addresses(int prec, size_t rows, size_t cols);

@@ -983,8 +983,7 @@ int launch_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, co
     // a few rows: the VALU multi-token GEMV quantises them as it stages them
     // (QActBatch::new's codes, one launch fewer) while they are few values
     const bool multi = matmul_takes_multi(w->precision, m, rows, cols) && !matmul_force_gemm();
-    if (multi && (multi_stages_f32(w->precision, m, rows, cols) ||
-                  (m <= 4 && valu_stages_f32(m, cols) && capturing(ctx->stream))))  // no scratch for the codes
+    if (multi && multi_stages_f32(w->precision, m, rows, cols))
         return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, &accumulate, QAct{}, m, xs);
     // QActBatch::new (quant.rs:693-714): the activation rows quantised per block
     const size_t qb = (m * cols + 255) / 256 * 256, sb = (4 * m * cols / BLOCK + 255) / 256 * 256;

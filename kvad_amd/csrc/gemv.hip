@@ -1231,7 +1231,7 @@ int launch_gemv_multi_jobs(kh_ctx *ctx, int njobs, const kh_weight *const *w, co
         rows_total += w[i]->rows;
         fits = fits && mma_addresses(w[i]->precision, w[i]->rows, w[i]->cols);
     }
-    if (!xf && fits && w[0]->precision != KH_F32 && mma_takes(m, rows_total, w[0]->cols))
+    if (!xf && fits && w[0]->precision != KH_F32 && mma_takes(m, rows_total))
         return launch_gemv_mma(ctx, njobs, w, bias, y, accumulate, x, m);
     if (njobs < 1 || njobs > MULTI_JOBS) return fail(KH_EINVAL, "matmul: one to three weights per launch");
     MultiArgs a{};
@@ -1266,34 +1266,29 @@ int launch_gemv_multi(kh_ctx *ctx, const kh_weight *w, const QAct &x, size_t m, 
     return launch_gemv_multi_jobs(ctx, 1, &w, &bias, &y, nullptr, x, m);
 }
 
-bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols) {
-    // The matrix-core kernel takes the rows' codes.
-    return !(mma_takes(m, rows, cols) && mma_addresses(precision, rows, cols)) && valu_stages_f32(m, cols);
-}
+namespace {
+size_t mma_min_tokens() { return (size_t)env_int("KVAD_MMA_MIN", 5); }  // tuning knob
+}  // namespace
 
-bool valu_stages_f32(size_t m, size_t cols) {
+bool multi_stages_f32(int precision, size_t m, size_t rows, size_t cols) {
     // Every workgroup quantises its token slots' rows (2, 4 or 8 slots); past
     // about 12K values that costs more than a quantising launch of its own
     // plus a stage of codes (measured over q8 and Q4_K weights of 896 to
-    // 14336 columns at m = 2..8).
+    // 14336 columns at m = 2..8).  The matrix-core kernel takes the rows' codes.
+    if (m >= mma_min_tokens() && mma_addresses(precision, rows, cols)) return false;
     const size_t slots = m <= 2 ? 2 : m <= 4 ? 4 : 8;
     const int lim = env_int("KVAD_MULTI_STAGE_F32", 12288);  // tuning knob
     return slots * cols <= (size_t)lim;
 }
 
-bool mma_takes(size_t m, size_t rows, size_t cols) {
-    if (m >= 2 && rows >= 65536) return true;
-    const int forced = env_int("KVAD_MMA_MIN", 0);  // tuning knob: from this many rows
-    if (forced > 0) return m >= (size_t)forced;
-    // The VALU kernel's time grows with its token slots (2, 4, 8), the
-    // matrix-core kernel's hardly at all.  Measured with the rows'
-    // quantisation (us, VALU / matrix cores): at two rows the VALU everywhere
-    // but a vocabulary head (Q4_K 4096x4096 7.2 / 7.8; q8 151936x896 42.0 /
-    // 32.6); at three and four, large matrices change over (Q4_K 14336x4096
-    // 14.9 / 13.4, 4096x14336 17.5 / 14.8, 4096x4096 8.6 / 7.7, q4 11008x4096
-    // 13.2 / 10.9, q8 8960x1536 9.2 / 8.4) and small or flat ones do not (q8
-    // 4864x896 5.5 / 5.7, 896x4864 8.3 / 9.5, 1536x8960 10.6 / 12.5).
-    return m >= 5 || (m >= 3 && rows >= 4096 && rows * cols >= (size_t)12 << 20);
+bool mma_takes(size_t m, size_t rows) {
+    // From five rows on, and from two over a vocabulary head's codes (q8
+    // 151936x896 at 2 rows 42.0 us on the VALU, 32.6).  At three and four rows
+    // the matrix cores are a little ahead over large matrices too (Q4_K
+    // 14336x4096 14.9 / 13.4, 4096x14336 17.5 / 14.8, q8 8960x1536 9.2 / 8.4), but
+    // there a row on the VALU is its matvec to the bit, and Q4_K's sums are
+    // nearer 64 bits (0.8e-7, and 1.4e-7 on the matrix cores).
+    return m >= mma_min_tokens() || (m >= 2 && rows >= 65536);
 }
 
 bool matmul_takes_multi(int precision, size_t m, size_t rows, size_t cols) {

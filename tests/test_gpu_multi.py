@@ -3,8 +3,7 @@ quant.rs:751-907, as forward_each calls it, llama.rs:418-434), which the
 library runs as a multi-token GEMV that streams the weights once for every
 token: on the VALU (dot4 per row and token; two token rows, or any with
 KVAD_MMA_MIN above m) or on the matrix cores (one v_mfma_i32_16x16x32_i8
-per block of 16 rows x 16 tokens; from five token rows, from three over
-large matrices).
+per block of 16 rows x 16 tokens; from five token rows).
 
 Bar: f32 outputs within 1e-5 x max|ref| of the oracle's matmul.  On the VALU
 path each token's row equals, to the bit, a single-token matvec of that
@@ -60,6 +59,19 @@ def test_few_tokens_match_the_oracle_and_single_matvecs(ctx, monkeypatch, path, 
                     np.testing.assert_array_equal(got[t], one)
                 else:
                     close(got[t], one)
+
+
+@pytest.mark.parametrize("prec,rows,cols", [("q8", 8960, 1536), ("q8", 65552, 256), ("q4", 11008, 2048),
+                                            ("q4k", 14336, 2048), ("q4k", 4096, 4096)])
+def test_up_to_four_rows_are_their_matvecs(ctx, prec, rows, cols):
+    # over large matrices too, where the matrix cores would be a little ahead
+    say("four rows", prec, rows, cols)
+    w, _ = make(ctx, prec, rows, cols, seed=rows)
+    for m in (2, 3, 4):
+        xs = O.normal(cols + m, m * cols)
+        got = w.matmul_bt(xs, m).reshape(m, rows)
+        for t in range(m):
+            np.testing.assert_array_equal(got[t], w.matvec_bt(xs[t * cols:(t + 1) * cols]))
 
 
 # the matrix cores: ragged 16-row groups, k tails of 1..3 blocks past whole
