@@ -35,15 +35,15 @@ from test_gpu_llm import build  # noqa: E402
 from test_gpu_moe_stages import close, mv  # noqa: E402
 
 
-def close_residual(x_new, x_old, y, what):
-    """x_new = x_old + y in f32: y held to 1e-5 x max|y|, plus the rounding of
-    the f32 add (half an ulp of x_new)."""
+def close_residual(x_new, x_old, y, what, slack=0.0):
+    """x_new = x_old + y in f32: y held to 1e-5 x max|y| (and slack), plus the
+    rounding of the f32 add (half an ulp of x_new)."""
     got = np.asarray(x_new, np.float64) - np.asarray(x_old, np.float64)
     y = np.asarray(y, np.float64)
     scale = float(np.max(np.abs(y)))
     err = float(np.max(np.abs(got - y)))
     ulp = float(np.max(np.spacing(np.abs(np.asarray(x_new, np.float32)))))
-    assert err <= 1e-5 * scale + ulp / 2, f"{what}: max err {err:.3e} vs scale {scale:.3e}, ulp {ulp:.1e}"
+    assert err <= 1e-5 * scale + ulp / 2 + slack, f"{what}: max err {err:.3e} vs scale {scale:.3e}, ulp {ulp:.1e}"
     return max(err - ulp / 2, 0.0) / scale
 
 

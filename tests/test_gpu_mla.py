@@ -27,7 +27,7 @@ def _run(ctx, ql, qp, c, pe, H, L):
     return K.mla_attend(ctx, cache, 0, H, ql, qp, L, SCALE).reshape(H, 512)
 
 
-@pytest.mark.parametrize("H, L", [(16, 1), (16, 3), (16, 64), (16, 65), (16, 200), (16, 1000), (16, 5000),
+@pytest.mark.parametrize("H, L", [(16, 1), (16, 3), (16, 16), (16, 17), (16, 31), (20, 32), (16, 33), (16, 64), (16, 65), (16, 200), (16, 1000), (16, 5000),
                                   (8, 130), (20, 333)])
 def test_latent_attention_matches_the_oracle(ctx, H, L):
     ql, qp, c, pe = _case(H * 7919 + L, H, L)
@@ -39,7 +39,9 @@ def test_latent_attention_matches_the_oracle(ctx, H, L):
         assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("L", [40, 300])  # one split (the kernel's own weights), several (the merge's correction)
+# one launch (the kernel's own weights; its second 16 positions too), two splits
+# and several (the merge's correction)
+@pytest.mark.parametrize("L", [15, 30, 32, 40, 300])
 def test_weights_below_1e_8_are_dropped(ctx, L):
     H = 16
     ql, qp, c, pe = _case(L, H, L)
