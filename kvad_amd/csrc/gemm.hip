@@ -699,9 +699,12 @@ size_t split_bytes() { return (size_t)env_int("KVAD_GEMM_SPLIT_MIB", 64) << 20; 
 const int SPLIT_MIN_STAGES = env_int("KVAD_GEMM_SPLIT_MIN", 2);  // tuning knobs
 const int SPLIT_MAX = env_int("KVAD_GEMM_SPLIT_MAX", 32);
 const int SPLIT_PER_CU = env_int("KVAD_GEMM_SPLIT_PER_CU", 2);
-// Under twelve stages of 128 the second launch costs more than the shorter
-// chains save: (512 tokens, 896 rows, 896) 14.1 us in two splits, 11.2
-// unsplit, (80, 4864, 896) 14.0 and 10.9.
+// Under twelve stages of 128 a second launch costs more than two shorter chains
+// save ((512 tokens, 896 rows, 896) 14.1 us in two splits, 11.2 unsplit, (80,
+// 4864, 896) 14.0 and 10.9), and so do a joint launch's two or three; three chains
+// and more of one weight pay for it (Q4_K (90, 1968, 1280) 19.2 us unsplit, 12.7
+// in five, (85, 3146, 1280) 20.1 and 17.0 in three; q8 (72, 96, 1376) 13.6 and
+// 10.3).
 constexpr int SPLIT_LEAST = 12;
 
 // Rows of every weight of a launch, and their tiles.
@@ -711,23 +714,28 @@ long long row_tiles(const GemmArgs &a, int tile_n) {
     return tiles(a.N) + (a.y2 ? tiles(a.N2) : 0) + (a.y3 ? tiles(a.N3) : 0);
 }
 
+bool rows_in_fours(const GemmArgs &a) { return !(a.N % 4 || (a.y2 && a.N2 % 4) || (a.y3 && a.N3 % 4)); }
+
 // How many splits a launch's k-stages are cut into (under 2: none): `stages` of
-// them, at least `min_st` a split, none under `least`, so that the grid comes to
+// them, at least `min_st` a split, under `least` three splits or none, so that the grid comes to
 // about SPLIT_PER_CU workgroups per CU (a CU holds several: one's loads wait while
 // another's MFMAs run), at most SPLIT_MAX splits, and partials (4 M N bytes a
 // split, written and read again) of at most the weights' wbytes or 4 MiB,
 // whichever is more (a small weight such as a router's 64 rows would otherwise
-// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); twice
-// that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
+// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); from
+// `least` stages on twice that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
 // 4096) 36.3 -> 27.5 us in four splits instead of two, (512, 896, 4864) 27.5 ->
-// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two).
+// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two) and the
+// rows are in fours: others' partials go value by value (q8 (313, 477, 4544) 26.9
+// us with twice the partials, 21.5 without, (117, 434, 7648) 33.9 and 27.0).
 long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st, int least, size_t wbytes, int cu) {
     const size_t plane = (size_t)a.M * all_rows(a) * 4;
-    const size_t most = std::max(wbytes, (size_t)4 << 20) * (2 * tiles <= cu ? 2 : 1);
-    long long ks = stages < least ? 1 : ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
+    const size_t most = std::max(wbytes, (size_t)4 << 20) * (stages >= least && 2 * tiles <= cu && rows_in_fours(a) ? 2 : 1);
+    long long ks = ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
     ks = std::min<long long>(ks, stages / min_st);
     ks = std::min<long long>(ks, SPLIT_MAX);
     ks = std::min<long long>(ks, (long long)(most / plane));
+    if (stages < least && (ks < 3 || a.y2)) ks = 1;
     const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
     if (forced > 0) ks = std::min(forced, stages);
     return std::min<long long>(ks, (long long)(split_bytes() / plane));
@@ -766,8 +774,7 @@ bool fills_rounds(kh_ctx *ctx, int precision, const GemmArgs &a, long long cu) {
     if (t > cu) return stages >= 16 && (t >= 3 * cu || (4 * t >= 7 * cu && t <= 2 * cu));
     if (stages < 64) return false;
     const long long ks = split_count_i8(a, 128, 128, (int)cu);
-    const bool fours = !(a.N % 4 || (a.y2 && a.N2 % 4) || (a.y3 && a.N3 % 4));
-    if (ks > 5 && !fours && precision != KH_Q4K) return false;
+    if (ks > 5 && !rows_in_fours(a) && precision != KH_Q4K) return false;
     return ks >= 2 && stages >= 13 * ks && 4 * t * ks >= 7 * cu && t * ks <= 2 * cu && split_partials(ctx, 0);
 }
 Shape pick_shape(kh_ctx *ctx, int precision, const GemmArgs &a) {

@@ -353,3 +353,23 @@ def test_matmuls_run_unsplit_without_a_split_workspace(ctx, monkeypatch, mib):
             del w
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("prec,m,rows,cols,ks", [("q4k", 90, 1968, 1280, 5), ("q8", 72, 96, 1376, 5), ("q8", 512, 896, 896, 1),
+                                                 ("q8", 80, 4864, 896, 1), ("q8", 313, 477, 4544, 7),
+                                                 ("q8", 313, 480, 4544, 13)])
+def test_split_rule(ctx, monkeypatch, prec, m, rows, cols, ks):
+    # under twelve k-stages three splits or none; partials up to twice the
+    # weights only for rows in fours, whose partials go by vectors.  A number of
+    # splits has sums of its own, so the bits show it.
+    say("split rule", prec, m, rows, cols)
+    w, parts = make(ctx, prec, rows, cols, seed=rows)
+    xs = O.normal(m + 9, m * cols)
+    got = w.matmul_bt(xs, m)
+    monkeypatch.setenv("KVAD_GEMM_KSPLIT", str(ks))
+    np.testing.assert_array_equal(w.matmul_bt(xs, m), got)
+    monkeypatch.setenv("KVAD_GEMM_KSPLIT", "1" if ks > 1 else "3")
+    assert not np.array_equal(w.matmul_bt(xs, m), got)
+    r = np.r_[0:3, rows - 3:rows]
+    sub = tuple(np.ascontiguousarray(np.asarray(p).reshape(rows, -1)[r]).ravel() for p in parts)
+    close(got.reshape(m, rows)[:, r], oracle_matmul(prec, sub, len(r), cols, xs, m).reshape(m, len(r)))
