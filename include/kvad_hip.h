@@ -137,7 +137,10 @@ int kh_matvec_many_dev(kh_ctx *ctx, size_t n, const kh_weight *const *w, const f
                        float *const *y);
 
 /* Weight::matmul_bt (quant.rs:751-858): y[m, rows] = xs[m, cols] W^T (+ bias);
- * m == 1 is kh_matvec. */
+ * m == 1 is kh_matvec.  A quantised weight's rows of y are kh_matvec's of
+ * their own row of xs to the bit for m <= 4 (for a weight of 65536 rows or
+ * more while 4 * cols, or 2 * cols at m == 2, is at most 12288); from five rows
+ * on they agree to rounding (1e-5 of the largest), in one fixed order. */
 int kh_matmul(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y);
 int kh_matmul_dev(kh_ctx *ctx, const kh_weight *w, const float *xs, size_t m, const float *bias, float *y);
 

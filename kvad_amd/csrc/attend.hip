@@ -600,8 +600,8 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(const int32_t *len_
     }
 }
 
-// Fixed-order butterfly within each wave, then the four wave results in wave
-// order; every thread gets the result.  s_w holds four floats.
+// Fixed-order butterfly within each of NW waves, then the wave results in wave
+// order; every thread gets the result.  s_w holds NW floats.
 template <int NW, typename F>
 __device__ __forceinline__ float block_reduce(float v, float *s_w, F op) {
 #pragma unroll
@@ -745,7 +745,7 @@ __device__ __forceinline__ void merge_head(const float *pm, const float *pl, con
     constexpr int NT = 64 * NW;
     constexpr int NQ = D / 4, NSG = NT / NQ;  // float4 slices of the dims; split groups
     constexpr int PER = MAX_SPLITS / NT;       // splits per thread at most
-    constexpr int NB = NW >= 16 ? 4 : 8;       // partial values in flight per thread
+    constexpr int NB = 8;                      // partial values in flight per thread
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ float s_w[2][NW];
@@ -1969,9 +1969,10 @@ __global__ __launch_bounds__(64 * NW) void mla_one_kernel(MlaArgs a) {
 // passes through memory.  Values: wave w forms O[heads][dims 64 w .. + 63].
 // Between tiles the sums are rescaled to the running maximum.
 //
-// Bound by the f32 matrix cores (68 products of 32 cycles a wave and tile, two
-// waves a SIMD) and by the chain load - scores - exchange - values of the first
-// tile.  One wave per 16 positions over all 576 dims, which read the rows from
+// Bound by the chain load - scores - exchange - values of its tiles: 16 heads
+// over 6001 positions, one tile a workgroup, take 12.5 us of which the matrix
+// cores' 68 products of 32 cycles a wave and tile are 1.3 (waves waiting 54% of
+// their cycles); over 32768 7.2 of 27, 128 heads over 20000 35 of 119.  One wave per 16 positions over all 576 dims, which read the rows from
 // memory twice, had both chains four times as long: 16 heads over 1000 / 3000 / 6001 / 20000 /
 // 32768 positions (scores spread by 2, split and merge) 16.2 / 20.5 / 24.0 /
 // 36.3 / 50 -> 12.0 / 15.5 / 18.4 / 32.3 / 37.5 us, 128 heads over 20000 150 ->

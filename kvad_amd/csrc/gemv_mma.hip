@@ -38,7 +38,7 @@
 // about 3 us included; against a kernel that loaded in the operand layout up
 // to 8 tokens and the int8 GEMM above): Q4_K 14336x4096 at 5 / 12 / 32 / 64
 // tokens 19.7 / 24.2 / 26.9 / 43.5 -> 13.8 / 14.0 / 19.5 / 30.8, 4096x14336
-// 18.6 / 24.5 / 25.9 / 38.0 -> 15.2 / 15.2 / 22.4 / 37.3, 4096x4096 9.2 / 13.7
+// 18.6 / 24.5 / 25.9 / 38.0 -> 15.7 / 16.2 / 22.4 / 37.3, 4096x4096 9.2 / 13.7
 // / 16.2 / 19.5 -> 7.7 / 7.9 / 10.4 / 17.3; q8 4864x896 at 5 / 16 / 64 6.4 /
 // 8.7 / 13.5 -> 5.8 / 5.9 / 8.7; q4 4096x4096 at 8 / 16 9.4 / 13.6 -> 7.7 /
 // 7.8.  Eight waves of up to 256 registers a workgroup and one workgroup a CU
