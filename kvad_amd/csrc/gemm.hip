@@ -722,19 +722,25 @@ bool rows_in_fours(const GemmArgs &a) { return !(a.N % 4 || (a.y2 && a.N2 % 4) |
 // another's MFMAs run), at most SPLIT_MAX splits, and partials (4 M N bytes a
 // split, written and read again) of at most the weights' wbytes or 4 MiB,
 // whichever is more (a small weight such as a router's 64 rows would otherwise
-// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit); from
-// `least` stages on twice that where the tiles fill half the CUs or fewer ((512 tokens, 1024 rows,
-// 4096) 36.3 -> 27.5 us in four splits instead of two, (512, 896, 4864) 27.5 ->
-// 25.6; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two) and the
-// rows are in fours: others' partials go value by value (q8 (313, 477, 4544) 26.9
-// us with twice the partials, 21.5 without, (117, 434, 7648) 33.9 and 27.0).
-long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st, int least, size_t wbytes, int cu) {
+// never split: 512 tokens x 64 x 2048, 16 workgroups, 22.6 us unsplit).  Up to
+// `twice` splits (128 x 128 tiles, which fill a round by them, and f32: any; else
+// four) may take twice that from `least` + 4 stages on, where the tiles fill half
+// the CUs or fewer and the rows are in fours ((512 tokens, 1024 rows, 4096) 25.2 ->
+// 22.7 us in four splits instead of two, Q4_K 36.7 -> 28.2, (512, 896, 4864) 27.2 ->
+// 24.9; (512, 2048, 2048), a tile for every CU, 19.0 unsplit, 24.9 in two); more
+// than four do not pay for it ((128, 896, 4864) in nine 14.6, in eighteen 15.6),
+// nor do rows whose partials go value by value (q8 (313, 477, 4544) 21.5 and 26.9).
+long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st, int least, int twice, size_t wbytes,
+                      int cu) {
     const size_t plane = (size_t)a.M * all_rows(a) * 4;
-    const size_t most = std::max(wbytes, (size_t)4 << 20) * (stages >= least && 2 * tiles <= cu && rows_in_fours(a) ? 2 : 1);
+    const size_t most = std::max(wbytes, (size_t)4 << 20);
+    long long most_ks = (long long)(most / plane);
+    if (most_ks < twice && stages >= least + 4 && 2 * tiles <= cu && rows_in_fours(a))
+        most_ks = std::min<long long>(twice, (long long)(2 * most / plane));
     long long ks = ((long long)SPLIT_PER_CU * cu + tiles / 2) / tiles;
     ks = std::min<long long>(ks, stages / min_st);
     ks = std::min<long long>(ks, SPLIT_MAX);
-    ks = std::min<long long>(ks, (long long)(most / plane));
+    ks = std::min<long long>(ks, most_ks);
     if (stages < least && (ks < 3 || a.y2)) ks = 1;
     const int forced = env_int("KVAD_GEMM_KSPLIT", 0);  // tuning knob: k splits (1: none)
     if (forced > 0) ks = std::min(forced, stages);
@@ -743,7 +749,7 @@ long long split_count(const GemmArgs &a, long long tiles, int stages, int min_st
 // The int8 GEMM's, in tiles of tile_m tokens by tile_n rows.
 long long split_count_i8(const GemmArgs &a, int tile_m, int tile_n, int cu) {
     return split_count(a, row_tiles(a, tile_n) * ((a.M + tile_m - 1) / tile_m), (a.K + BK - 1) / BK, SPLIT_MIN_STAGES,
-                       SPLIT_LEAST, (size_t)all_rows(a) * a.K, cu);
+                       SPLIT_LEAST, tile_m == 128 ? SPLIT_MAX : 4, (size_t)all_rows(a) * a.K, cu);
 }
 
 // Whether 128 x 128 tiles, of which a CU holds two, use the chip well enough
@@ -795,6 +801,11 @@ Shape pick_shape(kh_ctx *ctx, int precision, const GemmArgs &a) {
     if (M > 64 && nt * ((M + 127) / 128) >= 4LL * cu) return T128x128;
     if (fills_rounds(ctx, precision, a, cu)) return T128x128;
     if (M > 64 && M < 128 && nt >= cu) return T128x128;
+    // three token tiles of 32 rather than two of 64, half of the second empty:
+    // Q4_K, whose tiles cost the most (67 tokens, 5728 rows, 12544 columns 77 -> 66
+    // us, (80, 3028, 6144) 27.0 -> 24.6); q8 and q4 are behind over small weights
+    // (q8 (68, 2196, 3456) 14.8 -> 16.6)
+    if (M > 64 && M <= 96 && precision == KH_Q4K) return T128x32;
     if (M > 64) return T64x64;
     if (M > 32 && nt >= cu) return T128x64;
     return T128x32;
@@ -952,7 +963,7 @@ void set_split(kh_ctx *ctx, GemmArgs &a, long long ks) {
 void plan_split_f32(kh_ctx *ctx, GemmArgs &a, int tile_m) {
     const long long tiles = (long long)((a.N + 127) / 128) * ((a.M + tile_m - 1) / tile_m);
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    set_split(ctx, a, split_count(a, tiles, (a.K + FK - 1) / FK, 2, 0, (size_t)a.N * a.K * 4, cu));
+    set_split(ctx, a, split_count(a, tiles, (a.K + FK - 1) / FK, 2, 0, SPLIT_MAX, (size_t)a.N * a.K * 4, cu));
 }
 
 }  // namespace

@@ -357,11 +357,12 @@ def test_matmuls_run_unsplit_without_a_split_workspace(ctx, monkeypatch, mib):
 
 @pytest.mark.parametrize("prec,m,rows,cols,ks", [("q4k", 90, 1968, 1280, 5), ("q8", 72, 96, 1376, 5), ("q8", 512, 896, 896, 1),
                                                  ("q8", 80, 4864, 896, 1), ("q8", 313, 477, 4544, 7),
-                                                 ("q8", 313, 480, 4544, 13)])
+                                                 ("q8", 128, 896, 4864, 9), ("q8", 512, 1024, 4096, 4),
+                                                 ("q8", 512, 1022, 4096, 2)])
 def test_split_rule(ctx, monkeypatch, prec, m, rows, cols, ks):
     # under twelve k-stages three splits or none; partials up to twice the
-    # weights only for rows in fours, whose partials go by vectors.  A number of
-    # splits has sums of its own, so the bits show it.
+    # weights only to make four splits, and only for rows in fours, whose partials
+    # go by vectors.  A number of splits has sums of its own, so the bits show it.
     say("split rule", prec, m, rows, cols)
     w, parts = make(ctx, prec, rows, cols, seed=rows)
     xs = O.normal(m + 9, m * cols)
